@@ -149,7 +149,8 @@ def time_apply(R, op, X, stream, reps=20):
 
 # ------------------------------------------------------------------ other configurations
 KERNEL_NAMES = {-1: "-", 0: "regs x2", 1: "regs", 2: "lds", 3: "regs x2 (fp64)", 4: "regs (fp64)",
-                5: "null-space cholesky", 6: "null-space cholesky 8x3", 7: "lds packed"}
+                5: "null-space cholesky", 6: "null-space cholesky 8x3", 7: "lds packed",
+                8: "null-space elimination"}
 # solve kernels of the 4M 2-D Laplacian (k = 20, m = 6) by kernel id:
 # (description, name in a rocprofv3 trace, what bounds it)
 SOLVE_KERNELS = {
@@ -160,6 +161,8 @@ SOLVE_KERNELS = {
         "k_nsc<32, 1, 20, 6, 2, 1, 1, 3>", "valu-fp64"),
     6: ("k_nsc<8,3,20,6,2,1,1,2> (null-space Cholesky + FP64 refinement, 8 lanes x 3 rows per stencil)",
         "k_nsc<8, 3, 20, 6, 2, 1, 1, 2>", "valu-fp64"),
+    8: ("k_nse<3,2,6,15,1,4> (null-space elimination in registers, 16 lanes per stencil)",
+        "k_nse<3, 2, 6, 15, 1, 4>", "valu-fp64"),
 }
 
 

@@ -345,7 +345,7 @@ int rbfx_last_build_timing(double ms[4]);
  * with n = k + m <= 32, 33..64 and 65..RBFX_MAX_N, and the kernel each ran on
  * (0: registers, two stencils per wavefront; 1: registers, one; 2: system in LDS,
  * FP64; 3, 4: kernels 0, 1 in FP64 within an FP32 + refinement build; 5, 6: null-space
- * Cholesky; 7: packed lower triangle in LDS, FP64; -1: none). Uneven builds (ragged k or a degree map) classify stencils into these
+ * Cholesky; 7: packed lower triangle in LDS, FP64; 8: null-space elimination; -1: none). Uneven builds (ragged k or a degree map) classify stencils into these
  * buckets; the kernel of a bucket is timed on a sample the first time a
  * configuration is seen, and the fastest is kept (counts of -1: not read back).  */
 int rbfx_last_build_buckets(int64_t n[3], int32_t kernel[3]);
@@ -361,8 +361,11 @@ int rbfx_last_build_buckets(int64_t n[3], int32_t kernel[3]);
  * refinement fail are re-solved by kernel 0 or 7); 6 the same with 8 lanes of three
  * rows per stencil (k <= 20, at most 6 monomials); 7 rook LDL^T with the packed lower
  * triangle of the system in LDS (symmetric pivot moves; half the LDS of kernel 2, so
- * more wavefronts per CU). A pinned kernel that cannot serve a build is ignored by that
- * build.                                                                        */
+ * more wavefronts per CU); 8 null-space elimination in registers, 16 lanes per stencil
+ * (interior stencils of uniform builds: PHS3, PHS5 and PHS7 definite as for 5, in 2-D up
+ * to degree 4 and 3 operator columns, in 3-D up to degree 3 and 6 columns, at most 26
+ * points beyond the monomials, no multipliers; the stencils whose pivots fail are re-solved
+ * by kernel 0 or 7). A pinned kernel that cannot serve a build is ignored by that build. */
 int rbfx_tune_bucket(int32_t bucket, int32_t kernel);
 
 /* Counters of the last rbfx_build_weights on this thread (no reference counterpart):

@@ -18,6 +18,7 @@
 
 #include "build.h"
 #include "build_nsc.h"
+#include "build_nse.h"
 #include "knn.h"
 #include "learned.h"
 #include "mlp.h"
@@ -266,6 +267,10 @@ static int spmv_impl(const rbfx_spmv_args* a, bool async)
 //             wavefront, k <= 20, m <= 6).
 //   K_SYM     rook LDL^T with the packed lower triangle in LDS (n <= RBFX_MAX_N; half the
 //             LDS of K_WIDE, so more wavefronts per CU)
+//   K_NSE     null-space build by elimination (LU of the polynomial block, then a definite
+//             system without pivot search), 16 lanes per stencil with the system in
+//             registers, for PHS bases, up to 26 points beyond the monomials and 3 (2-D)
+//             or 6 (3-D) operator columns; hands back like K_NSC
 enum {
     K_REG32 = 0,
     K_REG64 = 1,
@@ -275,7 +280,8 @@ enum {
     K_NSC = 5,
     K_NSC2 = 6,
     K_SYM = 7,
-    kNumKernels = 8
+    K_NSE = 8,
+    kNumKernels = 9
 };
 int g_force_kernel[3] = {-1, -1, -1};  // rbfx_tune_bucket overrides
 // Launch plans of an uneven build: one launch per size bucket, each on its own kernel,
@@ -303,9 +309,10 @@ struct Shape {
     int dim, kmax, m, n_cols, basis_kind, poly_deg;
     bool hermite;
     bool uniform;  // every stencil has k points and m monomials (no ragged k, no degree map)
+    bool lambda;   // the caller wants the multipliers too
 };
 
-static bool is_nsc(int kid) { return kid == K_NSC || kid == K_NSC2; }
+static bool is_nsc(int kid) { return kid == K_NSC || kid == K_NSC2 || kid == K_NSE; }
 
 // In FP32 + refinement mode the FP64 kernels are candidates too (their stencils get
 // status FP64): with packed FP32 arithmetic unused, FP32 issues at the FP64 rate on
@@ -328,6 +335,10 @@ static bool kernel_serves(int kid, int bucket, bool fp32, const Shape& sh, bool 
         const int kb = std::min(sh.kmax, cap);
         return rbfx::nsc_fits(sh.dim, kb, sh.m, sh.n_cols, kid == K_NSC2 ? 1 : 0);
     }
+    case K_NSE:
+        return sh.uniform && !sh.lambda && rbfx::nsc_sign(sh.basis_kind, sh.poly_deg) != 0 &&
+               sh.kmax + sh.m <= (bucket == 0 ? 32 : (bucket == 1 ? 64 : RBFX_MAX_N)) &&
+               rbfx::nse_fits(sh.basis_kind, sh.dim, sh.kmax, sh.m, sh.n_cols);
     default: return false;
     }
 }
@@ -358,7 +369,9 @@ static hipError_t launch_kernel_id(int kid, const rbfx::BuildDev& P, const Shape
         Q.fail_list = hb.list;
         Q.fail_count = hb.count;
         hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, hb.count);
-        hipError_t e = rbfx::launch_build_nsc(Q, sh.dim, std::min(sh.kmax, cap), sh.m, kid == K_NSC2 ? 1 : 0, n_work, st);
+        hipError_t e = kid == K_NSE ? rbfx::launch_build_nse(Q, sh.dim, n_work, st)
+                                    : rbfx::launch_build_nsc(Q, sh.dim, std::min(sh.kmax, cap), sh.m,
+                                                             kid == K_NSC2 ? 1 : 0, n_work, st);
         if (e != hipSuccess) return e;
         int32_t nf = (int32_t)n_work;
         if (!async) {
@@ -397,6 +410,11 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
     if (bucket == 1 && !rbfx::sym_fits(64, sh.n_cols)) dflt = K_REG64;
     if (kernel_serves(K_NSC, bucket, fp32, sh, false)) dflt = K_NSC;
     if (kernel_serves(K_NSC2, bucket, fp32, sh, false)) dflt = K_NSC2;  // (the faster mapping where it fits)
+    // The elimination is faster than the other kernels on every shape it serves. Builds of
+    // several columns too small to be timed keep the weights, bit for bit, of the rook
+    // kernel that solves the same columns one build at a time.
+    if (kernel_serves(K_NSE, bucket, fp32, sh, false) && (sh.n_cols == 1 || bucket > 0 || count >= kTuneMin))
+        dflt = K_NSE;
     *kid = dflt;
     const int forced = g_force_kernel[bucket];
     if (forced >= 0 && kernel_serves(forced, bucket, fp32, sh, true)) {
@@ -854,6 +872,7 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
     sh.poly_deg = deg;
     sh.hermite = a->is_boundary != nullptr;
     sh.uniform = !a->adj_ptr && !a->poly_deg_map;
+    sh.lambda = a->out_lambda != nullptr;
     // stage boundaries: ev0 | main kernel | ev1 | FP32 list solve | ev2 | FP64 fallback | ev3
     // (blocking builds only; an asynchronous build records nothing but kernels)
     auto mark = [&](int i) -> hipError_t {
@@ -1047,7 +1066,7 @@ int rbfx_tune_bucket(int32_t bucket, int32_t kernel)
     if (kernel >= 0) {
         // a kernel that can serve the bucket for some configuration (a pinned kernel that
         // cannot serve a particular build is ignored by that build)
-        Shape any{2, 20, 6, 1, RBFX_PHS3, 2, false, true};
+        Shape any{2, 20, 6, 1, RBFX_PHS3, 2, false, true, false};
         bool ok = false;
         for (int kmax : {20, 30, 40, 60})
             for (int fp32 = 0; fp32 < 2; ++fp32) {

@@ -1,0 +1,56 @@
+// Dispatch of the null-space build by elimination over basis, dimension and stencil
+// shape (kernel template in build_nse_kernel.h, instantiations in build_nse_*.hip).
+#include "build_nse.h"
+
+namespace rbfx {
+
+hipError_t launch_nse_2d_phs3(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_2d_phs5(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_2d_phs7(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_3d_low(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_3d_phs3(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_3d_phs5(const BuildDev& P, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_3d_phs7(const BuildDev& P, int64_t n_work, hipStream_t s);
+
+// The null points (k - m) and the operator columns share the lanes of one or two slots
+// of 16, so at most 26 null points; the monomial tables of degree 1 to 4 (2-D) and 1 to 3
+// (3-D) that the basis is definite with. Other shapes (1-D, other bases, wider
+// stencils, more columns) stay with the other kernels.
+bool nse_fits(int kind, int dim, int k, int m, int n_cols)
+{
+    const int nn = k - m;
+    if (nn < 1 || n_cols < 1) return false;
+    if (kind != RBFX_PHS3 && kind != RBFX_PHS5 && kind != RBFX_PHS7) return false;
+    if (dim == 2) {
+        if (n_cols > 3) return false;
+        if (m == 3) return kind == RBFX_PHS3 && nn <= 13 - n_cols;
+        if (m == 6) return kind != RBFX_PHS7 && nn <= 26;
+        return (m == 10 || m == 15) && nn <= 26;
+    }
+    if (dim == 3) {
+        if (n_cols > 6) return false;
+        const int rc = n_cols == 2 ? 3 : (n_cols == 5 ? 6 : n_cols);
+        if (m == 4) return kind == RBFX_PHS3 && nn <= 16 - rc;
+        if (m == 10) return kind != RBFX_PHS7 && nn <= 26;
+        return m == 20 && nn <= 26;
+    }
+    return false;
+}
+
+hipError_t launch_build_nse(const BuildDev& P, int dim, int64_t n_work, hipStream_t s)
+{
+    if (!nse_fits(P.basis_kind, dim, P.k, P.n_mono, P.n_cols)) return hipErrorInvalidValue;
+    // uniform builds only: the kernel takes every stencil's k and m from P.k and P.n_mono
+    if (P.adj_ptr || P.deg_map || P.out_lambda) return hipErrorInvalidValue;
+    if (dim == 2) {
+        if (P.basis_kind == RBFX_PHS3) return launch_nse_2d_phs3(P, n_work, s);
+        if (P.basis_kind == RBFX_PHS5) return launch_nse_2d_phs5(P, n_work, s);
+        return launch_nse_2d_phs7(P, n_work, s);
+    }
+    if (P.n_mono <= 10) return launch_nse_3d_low(P, n_work, s);
+    if (P.basis_kind == RBFX_PHS3) return launch_nse_3d_phs3(P, n_work, s);
+    if (P.basis_kind == RBFX_PHS5) return launch_nse_3d_phs5(P, n_work, s);
+    return launch_nse_3d_phs7(P, n_work, s);
+}
+
+}  // namespace rbfx
