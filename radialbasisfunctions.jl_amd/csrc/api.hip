@@ -1205,39 +1205,35 @@ int64_t rbfx_mlp_bf16_count(void) { return rbfx::mlp_n_wbf16(); }
 
 namespace {
 
-// run workspace: Z_l (FP32), H_l (BF16), dY and two dZ buffers (BF16), 256-B aligned
-struct MlpWs {
-    float* Z[rbfx::kMlpLayers];
-    __bf16* H[rbfx::kMlpLayers - 1];
-    __bf16* dY;
-    __bf16* dZ[2];
-    int64_t bytes;
-};
-
-MlpWs mlp_ws(void* base, int64_t M)
+// run workspace: H_l and dZ_l, dY, the transposed weights, and aligned copies of the weights
+// and the inputs (all BF16), 256-B aligned from the first 256-B boundary of the buffer
+int64_t mlp_ws(void* base, int64_t M, rbfx::MlpPass& p)
 {
-    MlpWs w;
-    char* p = static_cast<char*>(base);
-    int64_t off = 0;
-    auto take = [&](int64_t bytes) {
-        char* q = p ? p + off : nullptr;
-        off += (bytes + 255) / 256 * 256;
+    const uintptr_t b0 = reinterpret_cast<uintptr_t>(base);
+    uintptr_t at = (b0 + 255) / 256 * 256;
+    auto take = [&](int64_t elems) {
+        __bf16* q = reinterpret_cast<__bf16*>(at);
+        at += (uintptr_t)((elems * 2 + 255) / 256 * 256);
         return q;
     };
-    for (int l = 0; l < rbfx::kMlpLayers; ++l) w.Z[l] = reinterpret_cast<float*>(take(M * rbfx::mlp_n(l) * 4));
-    for (int l = 0; l < rbfx::kMlpLayers - 1; ++l) w.H[l] = reinterpret_cast<__bf16*>(take(M * rbfx::kHid * 2));
-    w.dY = reinterpret_cast<__bf16*>(take(M * rbfx::kOutPad * 2));
-    w.dZ[0] = reinterpret_cast<__bf16*>(take(M * rbfx::kHid * 2));
-    w.dZ[1] = reinterpret_cast<__bf16*>(take(M * rbfx::kHid * 2));
-    w.bytes = off;
-    return w;
+    for (auto& h : p.H) h = take(M * rbfx::kHid);
+    for (auto& z : p.dZ) z = take(M * rbfx::kHid);
+    p.dY = take(M * rbfx::kOutPad);
+    p.wt = take(rbfx::mlp_n_wbf16());
+    p.wcopy = take(rbfx::mlp_n_wbf16());
+    p.xcopy = take(M * rbfx::kInPad);
+    return (int64_t)(at - b0) + 256;
 }
 
 }  // namespace
 
 extern "C" {
 
-int64_t rbfx_mlp_workspace_bytes(int32_t batch) { return batch > 0 ? mlp_ws(nullptr, batch).bytes : 0; }
+int64_t rbfx_mlp_workspace_bytes(int32_t batch)
+{
+    rbfx::MlpPass p;
+    return batch > 0 ? mlp_ws(nullptr, batch, p) : 0;
+}
 
 int rbfx_mlp_run(const rbfx_mlp_run_args* a)
 {
@@ -1249,86 +1245,22 @@ int rbfx_mlp_run(const rbfx_mlp_run_args* a)
     if (a->target && (!a->grads || !a->loss || a->n_out < 1 || a->n_out > kOutPad))
         return set_err(RBFX_EINVAL, "rbfx_mlp_run: training needs grads, loss and 1 <= n_out <= %d", kOutPad);
     hipStream_t st = (hipStream_t)a->stream;
-    const int M = a->batch;
-    MlpWs w = mlp_ws(a->workspace, M);
-    const __bf16* X = reinterpret_cast<const __bf16*>(a->x);
-    const __bf16* WB = reinterpret_cast<const __bf16*>(a->wbf16);
-    float* Zout = a->y_out ? a->y_out : w.Z[kMlpLayers - 1];
-    for (int l = 0; l < kMlpLayers; ++l) {
-        GemmArgs g;
-        std::memset(&g, 0, sizeof(g));
-        g.M = M;
-        g.N = mlp_n(l);
-        g.K = mlp_k(l);
-        g.A = l == 0 ? X : w.H[l - 1];
-        g.sAm = mlp_k(l);
-        g.sAk = 1;
-        g.B = WB + mlp_wb_off(l);
-        g.sBn = mlp_k(l);
-        g.sBk = 1;
-        g.C = l == kMlpLayers - 1 ? Zout : w.Z[l];
-        g.ldc = mlp_n(l);
-        g.bias = a->params + mlp_b_off(l);
-        if (l < kMlpLayers - 1) {
-            g.epi = EPI_BIAS_GELU;
-            g.H = w.H[l];
-            g.ldh = kHid;
-        } else {
-            g.epi = EPI_BIAS;
-        }
-        HIPCHK(launch_gemm(g, st));
-    }
-    if (a->target) {
-        HIPCHK(launch_fill_f32(a->loss, 1, 0.0f, st));
-        HIPCHK(launch_fill_f32(a->grads, mlp_n_params(), 0.0f, st));
-        HIPCHK(launch_mse_grad(M, a->n_out, Zout, kOutPad, a->target, a->n_out, a->row_weight, w.dY, kOutPad,
-                               a->loss, st));
-        const __bf16* dZ = w.dY;
-        int64_t ld_dz = kOutPad;
-        for (int l = kMlpLayers - 1; l >= 0; --l) {
-            const __bf16* Hin = l == 0 ? X : w.H[l - 1];
-            GemmArgs gw;
-            std::memset(&gw, 0, sizeof(gw));
-            gw.M = mlp_n(l);
-            gw.N = mlp_k(l);
-            gw.K = M;
-            gw.A = dZ;
-            gw.sAm = 1;
-            gw.sAk = ld_dz;
-            gw.B = Hin;
-            gw.sBn = 1;
-            gw.sBk = mlp_k(l);
-            gw.C = a->grads + mlp_w_off(l);
-            gw.ldc = mlp_k(l);
-            gw.epi = EPI_F32;
-            gw.accumulate = 1;
-            gw.k_split = 512;
-            HIPCHK(launch_gemm(gw, st));
-            HIPCHK(launch_colsum_bf16(M, mlp_n(l), dZ, ld_dz, a->grads + mlp_b_off(l), st));
-            if (l > 0) {
-                __bf16* dZn = w.dZ[l & 1];
-                GemmArgs gd;
-                std::memset(&gd, 0, sizeof(gd));
-                gd.M = M;
-                gd.N = mlp_k(l);
-                gd.K = mlp_n(l);
-                gd.A = dZ;
-                gd.sAm = ld_dz;
-                gd.sAk = 1;
-                gd.B = WB + mlp_wb_off(l);
-                gd.sBn = 1;
-                gd.sBk = mlp_k(l);
-                gd.epi = EPI_GELU_BWD;
-                gd.Z = w.Z[l - 1];
-                gd.ldz = kHid;
-                gd.H = dZn;
-                gd.ldh = kHid;
-                HIPCHK(launch_gemm(gd, st));
-                dZ = dZn;
-                ld_dz = kHid;
-            }
-        }
-    }
+    MlpPass p;
+    mlp_ws(a->workspace, a->batch, p);
+    p.M = a->batch;
+    p.n_out = a->n_out;
+    p.x = reinterpret_cast<const __bf16*>(a->x);
+    p.params = a->params;
+    p.w = reinterpret_cast<const __bf16*>(a->wbf16);
+    p.target = a->target;
+    p.row_weight = a->row_weight;
+    p.y = a->y_out;
+    p.grads = a->grads;
+    p.loss = a->loss;
+    // (the kernels read 16 bytes at a time: operands that are not aligned go through a copy)
+    if (reinterpret_cast<uintptr_t>(a->wbf16) % 16 == 0) p.wcopy = nullptr;
+    if (reinterpret_cast<uintptr_t>(a->x) % 16 == 0) p.xcopy = nullptr;
+    HIPCHK(launch_mlp(p, st));
     HIPCHK(hipStreamSynchronize(st));
     return RBFX_OK;
 }

@@ -40,42 +40,32 @@ __host__ __device__ constexpr int64_t mlp_wb_off(int l)
 }
 __host__ __device__ constexpr int64_t mlp_n_wbf16() { return mlp_wb_off(kMlpLayers); }
 
-// C[m][n] = sum_k A(m,k) B(n,k) with element strides, BF16 operands, FP32 accumulation
-enum GemmEpi {
-    EPI_F32 = 0,        // C (FP32) = acc            (accumulate: C += acc, atomically)
-    EPI_BIAS = 1,       // C (FP32) = acc + bias[n]
-    EPI_BIAS_GELU = 2,  // C (FP32) = acc + bias[n]; H (BF16) = gelu(C)
-    EPI_GELU_BWD = 3,   // H (BF16) = acc * gelu'(Z[m][n])
+// One pass over a batch of M rows: forward, and with a target also the loss and the
+// gradients. Workspace pointers are 16-byte aligned.
+struct MlpPass {
+    int M, n_out;
+    const __bf16* x;        // M x kInPad
+    const float* params;
+    const __bf16* w;        // BF16 weights
+    const float* target;    // M x n_out, or null
+    const float* row_weight;
+    float* y;               // M x kOutPad, or null
+    float* grads;
+    float* loss;
+    // workspace
+    __bf16* H[kMlpLayers - 1];   // M x kHid
+    __bf16* dZ[kMlpLayers - 1];  // M x kHid
+    __bf16* dY;                  // M x kOutPad
+    __bf16* wt;                  // weights of layers 1..3, transposed
+    __bf16* wcopy;               // aligned copy of w, or null where w is aligned itself
+    __bf16* xcopy;               // aligned copy of x, or null where x is aligned itself
 };
 
-struct GemmArgs {
-    int M, N, K;
-    const __bf16* A;
-    int64_t sAm, sAk;
-    const __bf16* B;
-    int64_t sBn, sBk;
-    float* C;
-    int64_t ldc;
-    const float* bias;
-    __bf16* H;
-    int64_t ldh;
-    const float* Z;
-    int64_t ldz;
-    int epi;
-    int accumulate;
-    int k_split;  // reduction length per grid.z slice (multiple of 32)
-};
+hipError_t launch_mlp(const MlpPass& a, hipStream_t s);
 
-hipError_t launch_gemm(const GemmArgs& g, hipStream_t s);
-
-// training step pieces
-hipError_t launch_mse_grad(int M, int n_out, const float* Y, int64_t ldy, const float* T, int64_t ldt,
-                           const float* row_weight, __bf16* dY, int64_t ld_dy, float* loss, hipStream_t s);
-hipError_t launch_colsum_bf16(int M, int N, const __bf16* X, int64_t ldx, float* out, hipStream_t s);
 hipError_t launch_adam(int64_t n, float* p, const float* g, float* m, float* v, float lr, float b1, float b2,
                        float eps, int t, hipStream_t s);
 hipError_t launch_params_to_bf16(const float* p, __bf16* wb, hipStream_t s);
-hipError_t launch_fill_f32(float* p, int64_t n, float v, hipStream_t s);
 
 // tanh(u) = 1 - 2 / (exp(2u) + 1): one hardware exp and one reciprocal. exp(2u)
 // overflows to +inf for large u (giving 1) and underflows to 0 for very negative u

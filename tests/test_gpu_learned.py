@@ -239,3 +239,42 @@ def test_trained_network_gains_over_untrained(RBF, gpu, trained):
         op = RBF.laplacian(pts, basis=RBF.PHS(3, poly_deg=2), k=20, device=gpu, precision="learned", model=m)
         counts[name] = op.status_counts[RBF._abi.ST_LEARNED]
     assert counts["trained"] > counts["untrained"], counts
+
+
+@pytest.mark.parametrize("M,shift", [(1, 0), (15, 0), (17, 0), (255, 1), (257, 0), (8193, 0)])
+def test_mlp_pass_at_tile_edges(RBF, gpu, M, shift):
+    """One pass at batch sizes around the 16 (or, beyond 8192, 32) rows of a workgroup and
+    the 128- and 256-row slices of the weight gradient; with shift, inputs and weights that
+    start off a 16-byte boundary. Bounds as in the tests above."""
+    import torch
+
+    n_out = 26
+    p = _params(3)
+    X = _inputs(M, M)
+    rng = np.random.default_rng(M)
+    T = np.zeros((M, 32))
+    T[:, :n_out] = rng.standard_normal((M, n_out))
+    params, wb = _dev_model(RBF, gpu, p)
+    x = torch.as_tensor(X, dtype=torch.float32, device=gpu).to(torch.bfloat16)
+    if shift:
+        xs = torch.empty(x.numel() + shift, dtype=torch.bfloat16, device=gpu)
+        xs[shift:] = x.reshape(-1)
+        x = xs[shift:].view(M, -1)
+        ws = torch.empty(wb.numel() + shift, dtype=torch.bfloat16, device=gpu)
+        ws[shift:] = wb
+        wb = ws[shift:]
+    y = torch.empty((M, 32), dtype=torch.float32, device=gpu)
+    tgt = torch.as_tensor(T[:, :n_out].astype(np.float32), device=gpu).contiguous()
+    grads = torch.empty(RBF._abi.MLP_N_PARAMS, dtype=torch.float32, device=gpu)
+    loss = torch.zeros(1, dtype=torch.float32, device=gpu)
+    ws = torch.empty(RBF._lib.mlp_workspace_bytes(M), dtype=torch.uint8, device=gpu)
+    RBF._lib.mlp_run(x, params, wb, ws, M, target=tgt, grads=grads, loss=loss, y_out=y, n_out=n_out)
+    Y_ref, _ = MO.forward(p, X)
+    assert _rel(y.cpu().numpy(), Y_ref) < 2e-2
+    l_ref, g_ref = MO.loss_and_grad(p, X, T, n_out)
+    assert abs(loss.item() - l_ref) <= 1e-3 * l_ref
+    g = grads.cpu().numpy().astype(np.float64)
+    for l in range(MO.LAYERS):
+        n, k = MO.n_of(l), MO.k_of(l)
+        for o, c in ((MO.w_off(l), n * k), (MO.b_off(l), n)):
+            assert _rel(g[o:o + c], g_ref[o:o + c]) < 2e-2, (l, c)
