@@ -277,6 +277,13 @@ int rbfx_knn(const double* data, int64_t n_data, const double* query, int64_t n_
              int32_t dim, int32_t k, const int64_t* q_ptr, int32_t* out_idx,
              void* stream);
 
+/* rbfx_knn, and with out_order != NULL also a processing order of the queries for
+ * rbfx_build_args.order and rbfx_spmv_args.row_order (a permutation of 0..n_query-1 in
+ * which queries close in the list are close in space: a Z-curve over the search's own
+ * grid, so it costs no sort of its own; which of a cell's queries comes first is not fixed). */
+int rbfx_knn_ordered(const double* data, int64_t n_data, const double* query, int64_t n_query, int32_t dim,
+                     int32_t k, const int64_t* q_ptr, int32_t* out_idx, int32_t* out_order, void* stream);
+
 /* build_weights_kernel (execution.jl:128-174) and the per-stencil solve it drives
  * (_build_stencil!, assembly.jl:201-222; Hermite dispatch assembly.jl:240-467).  */
 int rbfx_build_weights(const rbfx_build_args* args);

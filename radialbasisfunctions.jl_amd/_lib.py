@@ -46,6 +46,9 @@ def lib():
                 L.rbfx_knn.restype = C.c_int
                 L.rbfx_knn.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int32, C.c_int32,
                                        C.c_void_p, C.c_void_p, C.c_void_p]
+                L.rbfx_knn_ordered.restype = C.c_int
+                L.rbfx_knn_ordered.argtypes = [C.c_void_p, C.c_int64, C.c_void_p, C.c_int64, C.c_int32, C.c_int32,
+                                               C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]
                 L.rbfx_build_weights.restype = C.c_int
                 L.rbfx_build_weights.argtypes = [C.POINTER(abi.BuildArgs)]
                 L.rbfx_spmv.restype = C.c_int
@@ -102,7 +105,7 @@ def exported_symbols():
             "rbfx_mlp_workspace_bytes", "rbfx_mlp_run", "rbfx_mlp_adam", "rbfx_mlp_sync_bf16",
             "rbfx_stencil_features", "rbfx_spatial_order", "rbfx_build_weights_async", "rbfx_spmv_async",
             "rbfx_build_weights_noalloc", "rbfx_source_tiles",
-            "rbfx_permute_rows", "rbfx_last_build_buckets", "rbfx_tune_bucket", "rbfx_last_build_stats",
+            "rbfx_permute_rows", "rbfx_knn_ordered", "rbfx_last_build_buckets", "rbfx_tune_bucket", "rbfx_last_build_stats",
             "rbfx_tune_save", "rbfx_tune_load", "rbfx_tune_reset", "rbfx_tune_plan"]
 
 
@@ -143,8 +146,9 @@ def ptr(x):
     return None if x is None else C.c_void_p(x.data_ptr())
 
 
-def knn(data, query, k, q_ptr=None):
-    """data (N,d) f64 cuda, query (Q,d) f64 cuda -> (Q,k) int32 cuda (or flat with q_ptr)."""
+def knn(data, query, k, q_ptr=None, order=False):
+    """data (N,d) f64 cuda, query (Q,d) f64 cuda -> (Q,k) int32 cuda (or flat with q_ptr);
+    with order=True also a spatial processing order of the queries (Q,) int32."""
     t = torch()
     dev = data.device
     n_q = query.shape[0]
@@ -152,10 +156,11 @@ def knn(data, query, k, q_ptr=None):
         out = t.empty((n_q, k), dtype=t.int32, device=dev)
     else:
         out = t.empty(int(q_ptr[-1].item()), dtype=t.int32, device=dev)
+    perm = t.empty(n_q, dtype=t.int32, device=dev) if order else None
     with t.cuda.device(dev):
-        _check(lib().rbfx_knn(ptr(data), data.shape[0], ptr(query), n_q, data.shape[1], int(k), ptr(q_ptr),
-                              ptr(out), stream_ptr(dev)))
-    return out
+        _check(lib().rbfx_knn_ordered(ptr(data), data.shape[0], ptr(query), n_q, data.shape[1], int(k), ptr(q_ptr),
+                                      ptr(out), ptr(perm), stream_ptr(dev)))
+    return (out, perm) if order else out
 
 
 def build_weights(args, dev):

@@ -1175,8 +1175,8 @@ int rbfx_last_build_timing(double ms[4])
     return RBFX_OK;
 }
 
-int rbfx_knn(const double* data, int64_t n_data, const double* query, int64_t n_query, int32_t dim, int32_t k,
-             const int64_t* q_ptr, int32_t* out_idx, void* stream)
+int rbfx_knn_ordered(const double* data, int64_t n_data, const double* query, int64_t n_query, int32_t dim, int32_t k,
+                     const int64_t* q_ptr, int32_t* out_idx, int32_t* out_order, void* stream)
 {
     if (!data || !query || !out_idx) return set_err(RBFX_EINVAL, "rbfx_knn: null pointer argument");
     if (dim < 1 || dim > 3) return set_err(RBFX_EINVAL, "rbfx_knn: dim must be 1, 2 or 3 (got %d)", dim);
@@ -1186,9 +1186,15 @@ int rbfx_knn(const double* data, int64_t n_data, const double* query, int64_t n_
     hipStream_t st = (hipStream_t)stream;
     std::lock_guard<std::mutex> lk(g_mu);
     DeviceState& ds = dev_state();
-    HIPCHK(rbfx::run_knn(ds.knn, data, n_data, query, n_query, dim, k, q_ptr, out_idx, st));
+    HIPCHK(rbfx::run_knn(ds.knn, data, n_data, query, n_query, dim, k, q_ptr, out_idx, out_order, st));
     HIPCHK(hipStreamSynchronize(st));
     return RBFX_OK;
+}
+
+int rbfx_knn(const double* data, int64_t n_data, const double* query, int64_t n_query, int32_t dim, int32_t k,
+             const int64_t* q_ptr, int32_t* out_idx, void* stream)
+{
+    return rbfx_knn_ordered(data, n_data, query, n_query, dim, k, q_ptr, out_idx, nullptr, stream);
 }
 
 int rbfx_build_weights(const rbfx_build_args* a) { return build_impl(a, Mode::kBlocking); }

@@ -6,14 +6,27 @@
 // fused multiply-adds (the same rounding a KD-tree query sees); equal distances
 // are ordered by lower index.
 //
-// Data points are binned into a uniform grid (counting sort: count, scan,
-// scatter), queries are binned into the same grid so that a wavefront works on
-// spatially adjacent queries, and every query scans rings of cells outward until
-// no unvisited cell can hold a point closer than its current k-th neighbour.
-// The top-k list lives in registers (static-index insertion network).
+// Data points are binned into a uniform grid (counting sort: count, scan, scatter),
+// queries are binned into the same grid so that a wavefront works on spatially adjacent
+// queries (queries that are the data points share their binning), and every query scans
+// cells outward until no unvisited cell can hold a point closer than its current k-th
+// neighbour: first the block of two rings around its cell, row by row from the nearest,
+// then ring by ring. Clouds of up to 4,000 points are binned by one workgroup, grid sizing
+// included, with no host round trip.
+//
+// The top-k list lives in registers. A lane's candidates wait in LDS and are merged 16 at
+// a time (sorting networks on all lanes at once): inserting each as it came cost the whole
+// wavefront one insertion per candidate, since some lane accepts nearly every one.
+// Bound: latency of the dependent cell-range and point loads at small sizes, VALU issue of
+// the merges beyond. Measured, whole search, before (three points per cell
+// whatever k, rings from the first, each candidate inserted as it came) and now: 900 points,
+// 2-D, k = 12: 172 -> 70 us; 100,000, 3-D, k = 20: 444 -> 216 us; 4M, 2-D, k = 20: 3.49 ->
+// 2.16 ms; 2M, 3-D, k = 40: 9.0 -> 5.2 ms.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
+
+#include <utility>
 
 #include "knn.h"
 #include "knn_grid.h"
@@ -44,31 +57,85 @@ __device__ __forceinline__ int64_t cell_of(const double* p, const Grid& G)
 }
 
 // ---------------------------------------------------------------- bbox
-__global__ void k_bbox_partial(const double* __restrict__ x, int64_t n, int dim, double* out)
+// min / max of three coordinates over a workgroup of T threads (result in every thread 0..63)
+template <int T>
+__device__ __forceinline__ void block_box(double (&v)[6], double* lds)
 {
-    __shared__ double smin[3][256], smax[3][256];
-    double mn[3] = {1e300, 1e300, 1e300}, mx[3] = {-1e300, -1e300, -1e300};
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        for (int d = 0; d < dim; ++d) {
-            const double v = x[i * dim + d];
-            mn[d] = fmin(mn[d], v);
-            mx[d] = fmax(mx[d], v);
-        }
-    for (int d = 0; d < 3; ++d) { smin[d][threadIdx.x] = mn[d]; smax[d][threadIdx.x] = mx[d]; }
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w)
-            for (int d = 0; d < 3; ++d) {
-                smin[d][threadIdx.x] = fmin(smin[d][threadIdx.x], smin[d][threadIdx.x + w]);
-                smax[d][threadIdx.x] = fmax(smax[d][threadIdx.x], smax[d][threadIdx.x + w]);
-            }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0)
+#pragma unroll
+    for (int s = 1; s < 64; s <<= 1)
+#pragma unroll
         for (int d = 0; d < 3; ++d) {
-            out[blockIdx.x * 6 + d] = smin[d][0];
-            out[blockIdx.x * 6 + 3 + d] = smax[d][0];
+            v[d] = fmin(v[d], __shfl_xor(v[d], s, 64));
+            v[3 + d] = fmax(v[3 + d], __shfl_xor(v[3 + d], s, 64));
         }
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int d = 0; d < 6; ++d) lds[(threadIdx.x >> 6) * 6 + d] = v[d];
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < T / 64; ++w)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            v[d] = fmin(v[d], lds[w * 6 + d]);
+            v[3 + d] = fmax(v[3 + d], lds[w * 6 + 3 + d]);
+        }
+    __syncthreads();
+}
+
+__device__ __forceinline__ void box_of(const double* __restrict__ x, int64_t n, int dim, int64_t i, int64_t step,
+                                       double (&v)[6])
+{
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        v[d] = 1e300;
+        v[3 + d] = -1e300;
+    }
+    for (; i < n; i += step)
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            if (d < dim) {
+                const double c = x[i * dim + d];
+                v[d] = fmin(v[d], c);
+                v[3 + d] = fmax(v[3 + d], c);
+            }
+}
+
+// Partial boxes, and the last workgroup to finish reduces them into `out` (pinned host
+// memory) and clears the counter for the next call.
+constexpr int kBoxBlocks = 256;
+__global__ __launch_bounds__(256) void k_bbox(const double* __restrict__ x, int64_t n, int dim, double* part,
+                                              unsigned int* done, double* out)
+{
+    __shared__ double lds[4 * 6];
+    __shared__ unsigned int s_rank;
+    double v[6];
+    box_of(x, n, dim, blockIdx.x * (int64_t)256 + threadIdx.x, (int64_t)gridDim.x * 256, v);
+    block_box<256>(v, lds);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int d = 0; d < 6; ++d)
+            __hip_atomic_store(&part[blockIdx.x * 6 + d], v[d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __threadfence();
+        s_rank = atomicAdd(done, 1u);
+    }
+    __syncthreads();
+    if (s_rank != gridDim.x - 1) return;
+    __threadfence();
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+        v[d] = 1e300;
+        v[3 + d] = -1e300;
+    }
+    if (threadIdx.x < gridDim.x)
+#pragma unroll
+        for (int d = 0; d < 6; ++d)
+            v[d] = __hip_atomic_load(&part[threadIdx.x * 6 + d], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    block_box<256>(v, lds);
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int d = 0; d < 6; ++d) out[d] = v[d];
+        *done = 0u;
+    }
 }
 
 // ---------------------------------------------------------------- binning
@@ -81,8 +148,9 @@ __global__ void k_fill_i32(int32_t* __restrict__ p, int64_t n, int32_t v)
 
 template <int DIM>
 __global__ void k_cell_count(const double* __restrict__ x, int64_t n, Grid G, int32_t* __restrict__ cell,
-                             int32_t* __restrict__ count)
+                             int32_t* __restrict__ count, Grid* out)
 {
+    if (out && blockIdx.x == 0 && threadIdx.x == 0) *out = G;  // (for the search, which reads it from memory)
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
         const int32_t c = (int32_t)cell_of<DIM>(x + i * DIM, G);
         cell[i] = c;
@@ -92,11 +160,12 @@ __global__ void k_cell_count(const double* __restrict__ x, int64_t n, Grid G, in
 
 template <int DIM>
 __global__ void k_scatter(const double* __restrict__ x, int64_t n, const int32_t* __restrict__ cell,
-                          int32_t* __restrict__ cursor, int32_t* __restrict__ sorted_idx,
-                          double* __restrict__ sorted_x)
+                          const int32_t* __restrict__ start, int32_t* __restrict__ count,
+                          int32_t* __restrict__ sorted_idx, double* __restrict__ sorted_x)
 {
+    // (the counts run back down to zero as the slots are dealt out, last first)
     for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x) {
-        const int32_t slot = atomicAdd(&cursor[cell[i]], 1);
+        const int32_t slot = start[cell[i]] + atomicSub(&count[cell[i]], 1) - 1;
         sorted_idx[slot] = (int32_t)i;
         if (sorted_x)
 #pragma unroll
@@ -125,90 +194,356 @@ __device__ __forceinline__ double sqdist(const double* a, const double (&q)[DIM]
     return s;
 }
 
-template <int DIM, int KCAP>
-__global__ __launch_bounds__(128) void k_query(const double* __restrict__ sx, const int32_t* __restrict__ sidx,
-                                               const int32_t* __restrict__ cell_start,
-                                               const double* __restrict__ query,
-                                               const int32_t* __restrict__ qorder, int64_t n_query, Grid G,
-                                               int kmax, const int64_t* __restrict__ q_ptr,
-                                               int32_t* __restrict__ out)
+// ---------------------------------------------------------------- small clouds
+constexpr int kSmallPoints = 4000;
+constexpr int kSmallCells = 4 * kSmallPoints + 16;  // (knn_grid_size's bound; 64,064 bytes of LDS)
+
+// Bounding box, grid, counting sort: one workgroup.
+template <int DIM>
+__global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x, int n, double target, Grid* grid,
+                                                    int32_t* __restrict__ start, int32_t* __restrict__ sorted_idx,
+                                                    double* __restrict__ sorted_x)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (t >= n_query) return;
-    const int64_t qi = qorder ? qorder[t] : t;
+    __shared__ int32_t cnt[kSmallCells];
+    __shared__ double lds[16 * 6];
+    __shared__ int wsum[16];
+    __shared__ Grid G;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    double v[6];
+    box_of(x, n, DIM, t, 1024, v);
+    block_box<1024>(v, lds);
+    if (t == 0) {
+        double ext[3];
+        for (int d = 0; d < 3; ++d) ext[d] = v[3 + d] - v[d];
+        G.dim = DIM;
+        knn_grid_size(DIM, ext, n, &G.s, G.n, target);
+        G.inv_s = 1.0 / G.s;
+        for (int d = 0; d < 3; ++d) G.lo[d] = d < DIM ? v[d] : 0.0;
+        *grid = G;
+    }
+    __syncthreads();
+    const int ncell = G.n[0] * G.n[1] * G.n[2];
+    for (int c = t; c < ncell; c += 1024) cnt[c] = 0;
+    __syncthreads();
+    for (int i = t; i < n; i += 1024) atomicAdd(&cnt[cell_of<DIM>(x + (int64_t)i * DIM, G)], 1);
+    __syncthreads();
+    // exclusive scan: each thread a run of cells, then over the threads
+    const int run = (ncell + 1023) / 1024, c0 = t * run;
+    int sum = 0;
+    for (int c = c0; c < c0 + run && c < ncell; ++c) sum += cnt[c];
+    int inc = sum;
+    for (int s = 1; s < 64; s <<= 1) {
+        const int o = __shfl_up(inc, s, 64);
+        if (lane >= s) inc += o;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    int at = inc - sum;
+    for (int q = 0; q < w; ++q) at += wsum[q];
+    for (int c = c0; c < c0 + run && c < ncell; ++c) {
+        const int k = cnt[c];
+        cnt[c] = at;
+        start[c] = at;
+        at += k;
+    }
+    if (t == 0) start[ncell] = n;
+    __syncthreads();
+    for (int i = t; i < n; i += 1024) {
+        const int slot = atomicAdd(&cnt[cell_of<DIM>(x + (int64_t)i * DIM, G)], 1);
+        sorted_idx[slot] = i;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) sorted_x[(int64_t)slot * DIM + d] = x[(int64_t)i * DIM + d];
+    }
+}
+
+// ---------------------------------------------------------------- merging networks
+struct NetPair {
+    int a, b;
+};
+template <int CAP>
+struct Net {
+    int n = 0;
+    NetPair c[CAP] = {};
+};
+// Batcher's odd-even mergesort of N = 2^m entries
+template <int N>
+constexpr Net<N * 8> sort_net()
+{
+    Net<N * 8> r;
+    for (int p = 1; p < N; p *= 2)
+        for (int k = p; k >= 1; k /= 2)
+            for (int j = k % p; j + k < N; j += 2 * k)
+                for (int i = 0; i < k; ++i)
+                    if ((i + j) / (2 * p) == (i + j + k) / (2 * p) && i + j + k < N) r.c[r.n++] = {i + j, i + j + k};
+    return r;
+}
+// merge of a bitonic sequence of P entries, the comparators that the first KEEP outputs need
+template <int P, int KEEP>
+constexpr Net<P * 4> merge_net()
+{
+    Net<P * 4> all, r;
+    for (int k = P / 2; k >= 1; k /= 2)
+        for (int i = 0; i < P; ++i)
+            if ((i & k) == 0) all.c[all.n++] = {i, i + k};
+    bool need[P] = {};
+    bool use[P * 4] = {};
+    for (int i = 0; i < KEEP; ++i) need[i] = true;
+    for (int q = all.n - 1; q >= 0; --q)
+        if (need[all.c[q].a] || need[all.c[q].b]) {
+            use[q] = true;
+            need[all.c[q].a] = need[all.c[q].b] = true;
+        }
+    for (int q = 0; q < all.n; ++q)
+        if (use[q]) r.c[r.n++] = all.c[q];
+    return r;
+}
+
+// (a, b) -> (smaller, larger) in (distance, index) order
+__device__ __forceinline__ void comp(double& da, int& ia, double& db, int& ib)
+{
+    // (the instructions themselves: fmin would first quiet each operand; no NaN gets here)
+    const bool sw = lt(db, ib, da, ia);
+    double lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(da), "v"(db));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(da), "v"(db));
+    const int il = sw ? ib : ia, ih = sw ? ia : ib;
+    da = lo;
+    db = hi;
+    ia = il;
+    ib = ih;
+}
+
+template <int N, int... Q>
+__device__ __forceinline__ void run_sort(double* d, int* i, std::integer_sequence<int, Q...>)
+{
+    constexpr auto net = sort_net<N>();
+    (comp(d[net.c[Q].a], i[net.c[Q].a], d[net.c[Q].b], i[net.c[Q].b]), ...);
+}
+template <int P, int KEEP, int... Q>
+__device__ __forceinline__ void run_merge(double* d, int* i, std::integer_sequence<int, Q...>)
+{
+    constexpr auto net = merge_net<P, KEEP>();
+    (comp(d[net.c[Q].a], i[net.c[Q].a], d[net.c[Q].b], i[net.c[Q].b]), ...);
+}
+
+// candidates waiting per lane (the longest lists leave registers for 8 only)
+constexpr int pend_of(int kcap) { return kcap <= 40 ? 16 : 8; }
+
+// KCAP sorted entries (bd, bi) and the lane's n pending candidates -> the KCAP smallest
+template <int KCAP>
+__device__ __forceinline__ void merge_pending(double (&bd)[KCAP], int (&bi)[KCAP], const double (*pd)[64],
+                                              const int (*pi)[64], int n)
+{
+    constexpr int P = KCAP <= 16 ? 16 : (KCAP <= 32 ? 32 : 64), kPend = pend_of(KCAP);
+    const int lane = threadIdx.x & 63;
+    double d[P];
+    int i[P];
+    double sd[kPend];
+    int si[kPend];
+#pragma unroll
+    for (int u = 0; u < kPend; ++u) {
+        const double dv = pd[u][lane];
+        const int iv = pi[u][lane];
+        sd[u] = u < n ? dv : __builtin_huge_val();
+        si[u] = u < n ? iv : 0x7fffffff;
+    }
+    run_sort<kPend>(sd, si, std::make_integer_sequence<int, sort_net<kPend>().n>{});
+    // the sorted candidates reversed behind the list: smaller of each overlapping pair
+#pragma unroll
+    for (int u = 0; u < P; ++u) {
+        d[u] = u < KCAP ? bd[u < KCAP ? u : 0] : __builtin_huge_val();
+        i[u] = u < KCAP ? bi[u < KCAP ? u : 0] : 0x7fffffff;
+        if (P - 1 - u < kPend) {
+            const double cd = sd[P - 1 - u < kPend ? P - 1 - u : 0];
+            const int ci = si[P - 1 - u < kPend ? P - 1 - u : 0];
+            const bool sw = lt(cd, ci, d[u], i[u]);
+            d[u] = sw ? cd : d[u];
+            i[u] = sw ? ci : i[u];
+        }
+    }
+    run_merge<P, KCAP>(d, i, std::make_integer_sequence<int, merge_net<P, KCAP>().n>{});
+#pragma unroll
+    for (int u = 0; u < KCAP; ++u) {
+        bd[u] = d[u];
+        bi[u] = i[u];
+    }
+}
+
+// rows (dy, dz) of the block of two rings, nearest first
+__device__ constexpr int8_t kRowY[25] = {0, -1, 1, 0, 0, -1, 1, -1, 1, -2, 2, 0, 0, -2, -2, 2, 2, -1, 1, -1, 1, -2, 2, -2, 2};
+__device__ constexpr int8_t kRowZ[25] = {0, 0, 0, -1, 1, -1, -1, 1, 1, 0, 0, -2, 2, -1, 1, -1, 1, -2, -2, 2, 2, -2, -2, 2, 2};
+__device__ constexpr int8_t kRowY2[5] = {0, -1, 1, -2, 2};
+
+template <int DIM, int KCAP>
+__global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, const int32_t* __restrict__ sidx,
+                                              const int32_t* __restrict__ cell_start,
+                                              const double* __restrict__ query,
+                                              const int32_t* __restrict__ qorder, int64_t n_query,
+                                              const Grid* __restrict__ Gd, int kmax,
+                                              const int64_t* __restrict__ q_ptr, int32_t* __restrict__ out)
+{
+    constexpr int kPend = pend_of(KCAP);
+    __shared__ double s_pd[kPend][64];
+    __shared__ int s_pi[kPend][64];
+    const int lane = threadIdx.x;
+    const int64_t t = blockIdx.x * (int64_t)64 + lane;
+    const Grid G = *Gd;
+    const bool live = t < n_query;
+    const int64_t qi = !live ? 0 : (qorder ? qorder[t] : t);
     double q[DIM];
 #pragma unroll
     for (int d = 0; d < DIM; ++d) q[d] = query[qi * DIM + d];
-    int c[3] = {0, 0, 0};
-#pragma unroll
-    for (int d = 0; d < DIM; ++d) c[d] = cell_coord(q[d], G.lo[d], G.inv_s, G.n[d]);
+    const int c0 = cell_coord(q[0], G.lo[0], G.inv_s, G.n[0]);
+    const int c1 = DIM >= 2 ? cell_coord(q[DIM >= 2 ? 1 : 0], G.lo[1], G.inv_s, G.n[1]) : 0;
+    const int c2 = DIM == 3 ? cell_coord(q[DIM - 1], G.lo[2], G.inv_s, G.n[2]) : 0;
 
     double bd[KCAP];
     int bi[KCAP];
-    // slots [0, KCAP-kmax) hold sentinels below every real distance, so the
-    // insertion threshold is always the last slot
+    // slots [0, KCAP-kmax) hold sentinels below every real distance, so the threshold is
+    // always the last slot
 #pragma unroll
     for (int s = 0; s < KCAP; ++s) {
         bd[s] = (s < KCAP - kmax) ? -1.0 : __builtin_huge_val();
         bi[s] = (s < KCAP - kmax) ? -1 : 0x7fffffff;
     }
-    int filled = 0;
+    auto row_id = [&](int cy, int cz) { return ((int64_t)cz * G.n[1] + cy) * G.n[0]; };
+    // squared distance from the query to the box of cells [xl, xh] x cy x cz: no closer point
+    // (relative to the grid's corner, so nothing is rounded at the size of the coordinates)
+    auto side = [&](int d, int lo_cell, int hi_cell) __attribute__((always_inline)) {
+        const double at = q[d] - G.lo[d];
+        const double g = fmax(lo_cell * G.s - at, at - (hi_cell + 1) * G.s);
+        return g > 0.0 ? g * g : 0.0;
+    };
+    auto run_gap = [&](int xl, int xh, int cy, int cz) __attribute__((always_inline)) {
+        double g2 = side(0, xl, xh);
+        if constexpr (DIM >= 2) g2 += side(1, cy, cy);
+        if constexpr (DIM == 3) g2 += side(2, cz, cz);
+        return g2 * (1.0 - 1e-9);
+    };
+    // whether the k-th neighbour is closer than everything outside the visited rings
     int maxn = G.n[0];
-    for (int d = 1; d < DIM; ++d) maxn = max(maxn, G.n[d]);
-
-    for (int rho = 0;; ++rho) {
-        int lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) { lo[d] = c[d] - rho; hi[d] = c[d] + rho; }
-        // iterate the shell of cells at Chebyshev distance rho
-        const int z0 = (DIM == 3) ? max(lo[2], 0) : 0, z1 = (DIM == 3) ? min(hi[2], G.n[2] - 1) : 0;
-        for (int cz = z0; cz <= z1; ++cz) {
-            const bool zedge = (DIM == 3) && (cz == lo[2] || cz == hi[2]);
-            const int y0 = (DIM >= 2) ? max(lo[1], 0) : 0, y1 = (DIM >= 2) ? min(hi[1], G.n[1] - 1) : 0;
-            for (int cy = y0; cy <= y1; ++cy) {
-                const bool yedge = (DIM >= 2) && (cy == lo[1] || cy == hi[1]);
-                const bool full_row = zedge || yedge || (DIM == 1 && rho == 0);
-                const int x0 = max(lo[0], 0), x1 = min(hi[0], G.n[0] - 1);
-                const int step = full_row ? 1 : (hi[0] - lo[0] > 0 ? hi[0] - lo[0] : 1);
-                for (int cx = full_row ? x0 : lo[0]; cx <= (full_row ? x1 : hi[0]); cx += step) {
-                    if (cx < 0 || cx >= G.n[0]) continue;
-                    const int64_t cid = ((int64_t)cz * G.n[1] + cy) * G.n[0] + cx;
-                    const int32_t b = cell_start[cid], e = cell_start[cid + 1];
-                    for (int32_t s = b; s < e; ++s) {
-                        const double d2 = sqdist<DIM>(sx + (int64_t)s * DIM, q);
-                        const int id = sidx[s];
-                        if (!lt(d2, id, bd[KCAP - 1], bi[KCAP - 1])) continue;
-                        // insertion position p = number of entries preceding the candidate
-                        // (the list is sorted, so they are slots [0, p)); then shift right
-                        int p = 0;
-#pragma unroll
-                        for (int u = 0; u < KCAP - 1; ++u) p += lt(bd[u], bi[u], d2, id) ? 1 : 0;
-#pragma unroll
-                        for (int u = KCAP - 1; u >= 1; --u) {
-                            bd[u] = u > p ? bd[u - 1] : (u == p ? d2 : bd[u]);
-                            bi[u] = u > p ? bi[u - 1] : (u == p ? id : bi[u]);
-                        }
-                        if (p == 0) { bd[0] = d2; bi[0] = id; }
-                        ++filled;
-                    }
-                }
-            }
-        }
-        // lower bound on the distance of any point outside the visited box
+    if (DIM >= 2) maxn = max(maxn, G.n[1]);
+    if (DIM == 3) maxn = max(maxn, G.n[2]);
+    auto settled = [&](int rho) {
         double bound = 1e300;
         bool covers_all = true;
-#pragma unroll
-        for (int d = 0; d < DIM; ++d) {
-            const double blo = G.lo[d] + (double)(c[d] - rho) * G.s;
-            const double bhi = G.lo[d] + (double)(c[d] + rho + 1) * G.s;
-            if (c[d] - rho > 0) bound = fmin(bound, q[d] - blo);
-            if (c[d] + rho + 1 < G.n[d]) bound = fmin(bound, bhi - q[d]);
-            if (c[d] - rho > 0 || c[d] + rho + 1 < G.n[d]) covers_all = false;
-        }
-        if (covers_all || rho > maxn) break;
-        if (filled >= kmax && bound > 0.0 && bd[KCAP - 1] < bound * bound * (1.0 - 1e-9)) break;
-    }
+        auto side_bound = [&](int d, int cd) __attribute__((always_inline)) {
+            const double at = q[d] - G.lo[d];
+            if (cd - rho > 0) bound = fmin(bound, at - (cd - rho) * G.s);
+            if (cd + rho + 1 < G.n[d]) bound = fmin(bound, (cd + rho + 1) * G.s - at);
+            if (cd - rho > 0 || cd + rho + 1 < G.n[d]) covers_all = false;
+        };
+        side_bound(0, c0);
+        if constexpr (DIM >= 2) side_bound(1, c1);
+        if constexpr (DIM == 3) side_bound(2, c2);
+        if (covers_all || rho > maxn) return true;
+        return bi[KCAP - 1] != 0x7fffffff && bound > 0.0 && bd[KCAP - 1] < bound * bound * (1.0 - 1e-9);
+    };
 
+    // One loop over runs of cells: first the rows of the block of two rings, nearest first,
+    // then, for the lanes that are not settled, ring by ring (whole rows on a ring's faces,
+    // the two end cells elsewhere). The next run's range is loaded while a run is scanned.
+    // Within a run, four candidates per step as long as any lane has some; a merge when any
+    // lane might run out of room, and at the end of the block and of each ring. (The loop
+    // holds the only copy of the merge.)
+    constexpr int R0 = 2, NROW = DIM == 1 ? 1 : (DIM == 2 ? 5 : 25), STEP = 4;
+    int np = 0;  // pending candidates
+    int rho = R0, j = 0, dy = 0, dz = 0, part = 0;
+    bool open = live;
+    struct Run {
+        int32_t s0, s1;
+        double gap;
+        bool in, last;
+    };
+    auto next = [&]() __attribute__((always_inline)) {
+        Run r;
+        int cy, cz, xl = c0 - rho, xh = c0 + rho;
+        bool in = open;
+        if (rho == R0) {
+            cy = c1 + (DIM == 3 ? kRowY[j] : (DIM == 2 ? kRowY2[j] : 0));
+            cz = c2 + (DIM == 3 ? kRowZ[j] : 0);
+            r.last = ++j == NROW;
+        } else {
+            cy = c1 + dy;
+            cz = c2 + dz;
+            const bool face = (DIM == 3 && (dz == -rho || dz == rho)) || (DIM >= 2 && (dy == -rho || dy == rho));
+            if (!face) {
+                if (part == 0) {
+                    in = in && xl >= 0;
+                    xh = xl;
+                } else {
+                    in = in && xh < G.n[0];
+                    xl = xh;
+                }
+            }
+            part = face ? 0 : part ^ 1;
+            const bool step = part == 0, wrap = !(DIM >= 2 && dy < rho);
+            dz += step && wrap ? 1 : 0;
+            dy = !step ? dy : (wrap ? (DIM >= 2 ? -rho : 0) : dy + 1);
+            r.last = part == 0 && (DIM == 3 ? dz > rho : dz > 0);
+        }
+        r.in = in && cy >= 0 && cy < G.n[1] && cz >= 0 && cz < G.n[2];
+        r.gap = run_gap(xl, xh, cy, cz);
+        r.in = r.in && (r.gap < bd[KCAP - 1] || bi[KCAP - 1] == 0x7fffffff);
+        r.s0 = r.s1 = 0;
+        if (r.in) {
+            const int64_t id = row_id(cy, cz);
+            r.s0 = cell_start[id + max(xl, 0)];
+            r.s1 = cell_start[id + min(xh, G.n[0] - 1) + 1];
+        }
+        return r;
+    };
+    Run cur = next();
+    for (;;) {
+        Run nxt;
+        if (!cur.last) nxt = next();
+        // (a run wholly farther than the k-th neighbour so far holds nothing)
+        int32_t s0 = cur.s0;
+        const int32_t s1 = cur.gap < bd[KCAP - 1] || bi[KCAP - 1] == 0x7fffffff ? cur.s1 : s0;
+        bool more = __ballot(s0 < s1) != 0ull;
+        while (more || cur.last) {
+            if (more) {
+                double x[STEP][DIM];
+                int id[STEP];
+#pragma unroll
+                for (int u = 0; u < STEP; ++u) {
+                    const int32_t s = s0 + u < s1 ? s0 + u : (s0 < s1 ? s0 : 0);
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) x[u][d] = sx[(int64_t)s * DIM + d];
+                    id[u] = sidx[s];
+                }
+#pragma unroll
+                for (int u = 0; u < STEP; ++u) {
+                    const double d2 = sqdist<DIM>(x[u], q);
+                    if (s0 + u < s1 && lt(d2, id[u], bd[KCAP - 1], bi[KCAP - 1])) {
+                        s_pd[np][lane] = d2;
+                        s_pi[np][lane] = id[u];
+                        ++np;
+                    }
+                }
+                s0 += STEP;
+                more = __ballot(s0 < s1) != 0ull;
+            }
+            const bool full = __ballot(np > kPend - STEP) != 0ull;
+            if (full || (cur.last && !more)) {
+                merge_pending<KCAP>(bd, bi, s_pd, s_pi, np);
+                np = 0;
+            }
+            if (!more) break;
+        }
+        if (cur.last) {
+            open = open && !settled(rho);
+            if (!__ballot(open)) break;
+            ++rho;
+            dy = DIM >= 2 ? -rho : 0;
+            dz = DIM == 3 ? -rho : 0;
+            part = 0;
+            cur = next();
+        } else {
+            cur = nxt;
+        }
+    }
+    if (!live) return;
     const int64_t base = q_ptr ? q_ptr[qi] : qi * (int64_t)kmax;
     const int kq = q_ptr ? (int)(q_ptr[qi + 1] - q_ptr[qi]) : kmax;
 #pragma unroll
@@ -218,131 +553,215 @@ __global__ __launch_bounds__(128) void k_query(const double* __restrict__ sx, co
     }
 }
 
-// ---------------------------------------------------------------- driver
-template <int DIM>
-static hipError_t knn_dim(KnnWorkspace& ws, const double* data, int64_t n_data, const double* query,
-                          int64_t n_query, int k, const int64_t* q_ptr, int32_t* out, hipStream_t st,
-                          const double* bb /* host bbox: lo[3], hi[3] */)
+// ---------------------------------------------------------------- processing order
+__device__ __forceinline__ uint32_t compact_bits(uint32_t m, int dim, int d)
 {
+    uint32_t r = 0;
+    for (int b = 0; b * dim + d < 31; ++b) r |= ((m >> (b * dim + d)) & 1u) << b;
+    return r;
+}
+// number of points of each cell along the Z-curve (0 beyond the grid)
+__global__ __launch_bounds__(256) void k_curve_count(Grid G, int64_t n_curve, const int32_t* __restrict__ start,
+                                                     int32_t* __restrict__ cnt)
+{
+    const int64_t m = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (m > n_curve) return;
+    int v = 0;
+    if (m < n_curve) {
+        int x[3];
+        bool in = true;
+        for (int d = 0; d < 3; ++d) {
+            x[d] = d < G.dim ? (int)compact_bits((uint32_t)m, G.dim, d) : 0;
+            in = in && x[d] < G.n[d];
+        }
+        if (in) {
+            const int64_t c = ((int64_t)x[2] * G.n[1] + x[1]) * G.n[0] + x[0];
+            v = start[c + 1] - start[c];
+        }
+    }
+    cnt[m] = v;
+}
+__global__ __launch_bounds__(256) void k_curve_place(Grid G, int64_t n_curve, const int32_t* __restrict__ start,
+                                                     const int32_t* __restrict__ at, const int32_t* __restrict__ sorted,
+                                                     int32_t* __restrict__ order)
+{
+    const int64_t m = blockIdx.x * (int64_t)256 + threadIdx.x;
+    if (m >= n_curve) return;
+    int x[3];
+    for (int d = 0; d < 3; ++d) {
+        x[d] = d < G.dim ? (int)compact_bits((uint32_t)m, G.dim, d) : 0;
+        if (x[d] >= G.n[d]) return;
+    }
+    const int64_t c = ((int64_t)x[2] * G.n[1] + x[1]) * G.n[0] + x[0];
+    const int32_t b = start[c], e = start[c + 1];
+    int32_t o = at[m];
+    for (int32_t s = b; s < e; ++s) order[o++] = sorted[s];
+}
+
+// ---------------------------------------------------------------- driver
+static hipError_t grow(void** p, size_t& cap, size_t need)
+{
+    if (need <= cap) return hipSuccess;
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+    cap = 0;
+    hipError_t e = hipMalloc(p, need);
+    if (e == hipSuccess) cap = need;
+    return e;
+}
+
+static hipError_t scan(KnnWorkspace& ws, const int32_t* in, int32_t* out, int64_t n, hipStream_t st)
+{
+    size_t need = 0;
+    hipError_t e = hipcub::DeviceScan::ExclusiveSum(nullptr, need, in, out, (int)n, st);
+    if (e == hipSuccess) e = grow(&ws.scan_tmp, ws.scan_tmp_bytes, need + 256);
+    if (e != hipSuccess) return e;
+    size_t have = ws.scan_tmp_bytes;
+    return hipcub::DeviceScan::ExclusiveSum(ws.scan_tmp, have, in, out, (int)n, st);
+}
+
+// the register list costs merges and VGPRs with KCAP, so KCAP follows k closely in the
+// common range
+template <int DIM>
+static hipError_t launch_query(const KnnWorkspace& ws, const double* query, const int32_t* qorder, int64_t n_query,
+                               int k, const int64_t* q_ptr, int32_t* out, hipStream_t st)
+{
+    const dim3 gq((unsigned)((n_query + 63) / 64));
+#define RBFX_KNN_LAUNCH(KC)                                                                                  \
+    if (k <= KC) {                                                                                           \
+        hipLaunchKernelGGL((k_query<DIM, KC>), gq, dim3(64), 0, st, ws.sx, ws.sidx, ws.start, query, qorder, \
+                           n_query, (const Grid*)ws.grid, k, q_ptr, out);                                                   \
+        return hipGetLastError();                                                                            \
+    }
+    RBFX_KNN_LAUNCH(16)
+    RBFX_KNN_LAUNCH(20)
+    RBFX_KNN_LAUNCH(24)
+    RBFX_KNN_LAUNCH(32)
+    RBFX_KNN_LAUNCH(40)
+    RBFX_KNN_LAUNCH(48)
+    RBFX_KNN_LAUNCH(64)
+#undef RBFX_KNN_LAUNCH
+    return hipErrorInvalidValue;
+}
+
+// Z-curve order of the binned queries, by a counting sort over the curve. A grid whose
+// curve is mostly outside it (very unequal sides) keeps the row-by-row cell order.
+static hipError_t curve_order(KnnWorkspace& ws, const Grid& G, int64_t ncell, const int32_t* start,
+                              const int32_t* sorted, int64_t n_query, int32_t* order, hipStream_t st)
+{
+    int bits = 0;
+    for (int d = 0; d < G.dim; ++d)
+        while ((1ll << bits) < G.n[d]) ++bits;
+    const int64_t n_curve = bits * G.dim < 31 ? 1ll << (bits * G.dim) : INT64_MAX;
+    if (n_curve > 8 * ncell + 1024)
+        return hipMemcpyAsync(order, sorted, sizeof(int32_t) * n_query, hipMemcpyDeviceToDevice, st);
+    hipError_t e;
+    // (qcell is free by now when the queries are the data points, and large enough or grown)
+    if ((e = grow((void**)&ws.qcount, ws.cap_qcount, (size_t)(n_curve + 1) * 4)) != hipSuccess) return e;
+    if ((e = grow((void**)&ws.qcell, ws.cap_qcell, (size_t)(n_curve + 1) * 4)) != hipSuccess) return e;
+    const dim3 grid((unsigned)((n_curve + 1 + 255) / 256));
+    hipLaunchKernelGGL(k_curve_count, grid, dim3(256), 0, st, G, n_curve, start, ws.qcount);
+    if ((e = scan(ws, ws.qcount, ws.qcell, n_curve + 1, st)) != hipSuccess) return e;
+    hipLaunchKernelGGL(k_curve_place, grid, dim3(256), 0, st, G, n_curve, start, ws.qcell, sorted, order);
+    return hipGetLastError();
+}
+
+template <int DIM>
+static hipError_t knn_dim(KnnWorkspace& ws, const double* data, int64_t n_data, const double* query, int64_t n_query,
+                          int k, const int64_t* q_ptr, int32_t* out, int32_t* out_order, hipStream_t st)
+{
+    const bool self = query == data && n_query == n_data;
+    const double target = knn_cell_target(DIM, k);
+    hipError_t err;
+    if ((err = ws.reserve_points(n_data, n_query, DIM, self, st)) != hipSuccess) return err;
     Grid G;
+    if (n_data <= kSmallPoints && !out_order) {
+        if ((err = ws.reserve_cells(kSmallCells, true)) != hipSuccess) return err;
+        hipLaunchKernelGGL(k_bin_small<DIM>, dim3(1), dim3(1024), 0, st, data, (int)n_data, target, (Grid*)ws.grid,
+                           ws.start, ws.sidx, ws.sx);
+        return launch_query<DIM>(ws, query, self ? ws.sidx : nullptr, n_query, k, q_ptr, out, st);
+    }
+    // bounding box of the data (queries outside it bin into boundary cells)
+    const int nb = (int)std::min<int64_t>((n_data + 2047) / 2048, kBoxBlocks);
+    hipLaunchKernelGGL(k_bbox, dim3(nb), dim3(256), 0, st, data, n_data, DIM, ws.bbox,
+                       (unsigned int*)(ws.bbox + 6 * kBoxBlocks), ws.hbox);
+    if ((err = hipStreamSynchronize(st)) != hipSuccess) return err;
+    const double* bb = ws.hbox;
     G.dim = DIM;
     double ext[3] = {0, 0, 0};
     for (int d = 0; d < DIM; ++d) ext[d] = bb[3 + d] - bb[d];
     double s = 1.0;
-    const int64_t ncell = knn_grid_size(DIM, ext, n_data, &s, G.n);
+    const int64_t ncell = knn_grid_size(DIM, ext, n_data, &s, G.n, target);
     G.s = s;
     G.inv_s = 1.0 / s;
     for (int d = 0; d < 3; ++d) G.lo[d] = (d < DIM) ? bb[d] : 0.0;
 
-    hipError_t err;
-    if ((err = ws.reserve(ncell, n_data, n_query, DIM)) != hipSuccess) return err;
+    if ((err = ws.reserve_cells(ncell, self)) != hipSuccess) return err;
     const int TB = 256;
-    const int gridN = (int)std::min<int64_t>((n_data + TB - 1) / TB, 65535);
-    const int gridQ = (int)std::min<int64_t>((n_query + TB - 1) / TB, 65535);
-
-    // data binning
     const int gridC = (int)std::min<int64_t>((ncell + 1 + TB - 1) / TB, 65535);
-    hipLaunchKernelGGL(k_fill_i32, dim3(gridC), dim3(TB), 0, st, ws.count, ncell + 1, 0);
-    hipLaunchKernelGGL(k_cell_count<DIM>, dim3(gridN), dim3(TB), 0, st, data, n_data, G, ws.cell, ws.count);
-    size_t tmp_bytes = ws.scan_tmp_bytes;
-    if ((err = hipcub::DeviceScan::ExclusiveSum(ws.scan_tmp, tmp_bytes, ws.count, ws.start, (int)(ncell + 1), st)) !=
-        hipSuccess)
-        return err;
-    if ((err = hipMemcpyAsync(ws.cursor, ws.start, sizeof(int32_t) * (ncell + 1), hipMemcpyDeviceToDevice, st)) !=
-        hipSuccess)
-        return err;
-    hipLaunchKernelGGL(k_scatter<DIM>, dim3(gridN), dim3(TB), 0, st, data, n_data, ws.cell, ws.cursor,
-                       ws.sidx, ws.sx);
-    // query binning (spatially coherent wavefronts)
-    hipLaunchKernelGGL(k_fill_i32, dim3(gridC), dim3(TB), 0, st, ws.qcount, ncell + 1, 0);
-    hipLaunchKernelGGL(k_cell_count<DIM>, dim3(gridQ), dim3(TB), 0, st, query, n_query, G, ws.qcell, ws.qcount);
-    tmp_bytes = ws.scan_tmp_bytes;
-    if ((err = hipcub::DeviceScan::ExclusiveSum(ws.scan_tmp, tmp_bytes, ws.qcount, ws.qstart, (int)(ncell + 1),
-                                                st)) != hipSuccess)
-        return err;
-    hipLaunchKernelGGL(k_scatter<DIM>, dim3(gridQ), dim3(TB), 0, st, query, n_query, ws.qcell, ws.qstart,
-                       ws.qorder, (double*)nullptr);
-
-    const int QB = 128;
-    const dim3 gq((unsigned)((n_query + QB - 1) / QB));
-    // the insertion network costs KCAP - 1 steps per accepted candidate, so KCAP
-    // follows k closely in the common range
-    if (k <= 16)
-        hipLaunchKernelGGL((k_query<DIM, 16>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else if (k <= 20)
-        hipLaunchKernelGGL((k_query<DIM, 20>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else if (k <= 24)
-        hipLaunchKernelGGL((k_query<DIM, 24>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else if (k <= 32)
-        hipLaunchKernelGGL((k_query<DIM, 32>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else if (k <= 40)
-        hipLaunchKernelGGL((k_query<DIM, 40>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else if (k <= 48)
-        hipLaunchKernelGGL((k_query<DIM, 48>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    else
-        hipLaunchKernelGGL((k_query<DIM, 64>), gq, dim3(QB), 0, st, ws.sx, ws.sidx, ws.start, query, ws.qorder,
-                           n_query, G, k, q_ptr, out);
-    return hipGetLastError();
+    // counting sort of a point set into cells
+    auto bin = [&](const double* x, int64_t n, int32_t* cell, int32_t* count, int32_t* start, int32_t* idx,
+                   double* sorted_x) -> hipError_t {
+        const int gridN = (int)std::min<int64_t>((n + TB - 1) / TB, 65535);
+        hipLaunchKernelGGL(k_fill_i32, dim3(gridC), dim3(TB), 0, st, count, ncell + 1, 0);
+        hipLaunchKernelGGL(k_cell_count<DIM>, dim3(gridN), dim3(TB), 0, st, x, n, G, cell, count,
+                           sorted_x ? (Grid*)ws.grid : nullptr);
+        const hipError_t e = scan(ws, count, start, ncell + 1, st);
+        if (e != hipSuccess) return e;
+        hipLaunchKernelGGL(k_scatter<DIM>, dim3(gridN), dim3(TB), 0, st, x, n, cell, start, count, idx, sorted_x);
+        return hipGetLastError();
+    };
+    if ((err = bin(data, n_data, ws.cell, ws.count, ws.start, ws.sidx, ws.sx)) != hipSuccess) return err;
+    const int32_t *qstart = ws.start, *qorder = ws.sidx;
+    if (!self) {  // (spatially coherent wavefronts)
+        if ((err = bin(query, n_query, ws.qcell, ws.qcount, ws.qstart, ws.qorder, nullptr)) != hipSuccess) return err;
+        qstart = ws.qstart;
+        qorder = ws.qorder;
+    }
+    if ((err = launch_query<DIM>(ws, query, qorder, n_query, k, q_ptr, out, st)) != hipSuccess) return err;
+    if (out_order) return curve_order(ws, G, ncell, qstart, qorder, n_query, out_order, st);
+    return hipSuccess;
 }
 
-hipError_t KnnWorkspace::reserve(int64_t ncell, int64_t n_data, int64_t n_query, int dim)
+hipError_t KnnWorkspace::reserve_points(int64_t n_data, int64_t n_query, int dim, bool self, hipStream_t st)
 {
-    auto grow = [](void** p, size_t& cap, size_t need) -> hipError_t {
-        if (need <= cap) return hipSuccess;
-        if (*p) (void)hipFree(*p);
-        *p = nullptr;
-        cap = 0;
-        hipError_t e = hipMalloc(p, need);
-        if (e == hipSuccess) cap = need;
-        return e;
-    };
     hipError_t e;
-    const size_t nc = (size_t)(ncell + 1);
-    if ((e = grow((void**)&count, cap_count, nc * 4)) != hipSuccess) return e;
-    if ((e = grow((void**)&start, cap_start, nc * 4)) != hipSuccess) return e;
-    if ((e = grow((void**)&cursor, cap_cursor, nc * 4)) != hipSuccess) return e;
-    if ((e = grow((void**)&qcount, cap_qcount, nc * 4)) != hipSuccess) return e;
-    if ((e = grow((void**)&qstart, cap_qstart, nc * 4)) != hipSuccess) return e;
+    if (!bbox) {
+        if ((e = hipMalloc((void**)&bbox, sizeof(double) * (6 * kBoxBlocks + 1))) != hipSuccess) return e;
+        hipLaunchKernelGGL(k_fill_i32, dim3(1), dim3(64), 0, st, (int32_t*)(bbox + 6 * kBoxBlocks), (int64_t)2, 0);
+    }
+    if (!hbox && (e = hipHostMalloc((void**)&hbox, sizeof(double) * 6, hipHostMallocDefault)) != hipSuccess) return e;
+    if (!grid && (e = hipMalloc(&grid, sizeof(Grid))) != hipSuccess) return e;
     if ((e = grow((void**)&cell, cap_cell, (size_t)n_data * 4)) != hipSuccess) return e;
     if ((e = grow((void**)&sidx, cap_sidx, (size_t)n_data * 4)) != hipSuccess) return e;
     if ((e = grow((void**)&sx, cap_sx, (size_t)n_data * dim * 8)) != hipSuccess) return e;
-    if ((e = grow((void**)&qcell, cap_qcell, (size_t)n_query * 4)) != hipSuccess) return e;
-    if ((e = grow((void**)&qorder, cap_qorder, (size_t)n_query * 4)) != hipSuccess) return e;
-    size_t need = 0;
-    if ((e = hipcub::DeviceScan::ExclusiveSum(nullptr, need, count, start, (int)nc)) != hipSuccess) return e;
-    if ((e = grow(&scan_tmp, scan_tmp_bytes, need + 256)) != hipSuccess) return e;
-    if ((e = grow((void**)&bbox, cap_bbox, 6 * 8 * 1024)) != hipSuccess) return e;
+    if (!self) {
+        if ((e = grow((void**)&qcell, cap_qcell, (size_t)n_query * 4)) != hipSuccess) return e;
+        if ((e = grow((void**)&qorder, cap_qorder, (size_t)n_query * 4)) != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t KnnWorkspace::reserve_cells(int64_t ncell, bool self)
+{
+    const size_t nc = (size_t)(ncell + 1) * 4;
+    hipError_t e;
+    if ((e = grow((void**)&count, cap_count, nc)) != hipSuccess) return e;
+    if ((e = grow((void**)&start, cap_start, nc)) != hipSuccess) return e;
+    if (!self) {
+        if ((e = grow((void**)&qcount, cap_qcount, nc)) != hipSuccess) return e;
+        if ((e = grow((void**)&qstart, cap_qstart, nc)) != hipSuccess) return e;
+    }
     return hipSuccess;
 }
 
 hipError_t run_knn(KnnWorkspace& ws, const double* data, int64_t n_data, const double* query, int64_t n_query,
-                   int dim, int k, const int64_t* q_ptr, int32_t* out, hipStream_t st)
+                   int dim, int k, const int64_t* q_ptr, int32_t* out, int32_t* out_order, hipStream_t st)
 {
-    hipError_t e;
-    if ((e = ws.reserve(1, n_data, n_query, dim)) != hipSuccess) return e;
-    // bounding box of data and queries together (queries outside the data box
-    // still bin into boundary cells, so only the data box matters for grid size)
-    const int nb = 1024;
-    hipLaunchKernelGGL(k_bbox_partial, dim3(nb), dim3(256), 0, st, data, n_data, dim, ws.bbox);
-    static thread_local double hb[6 * 1024];
-    if ((e = hipMemcpyAsync(hb, ws.bbox, sizeof(double) * 6 * nb, hipMemcpyDeviceToHost, st)) != hipSuccess) return e;
-    if ((e = hipStreamSynchronize(st)) != hipSuccess) return e;
-    double bb[6] = {1e300, 1e300, 1e300, -1e300, -1e300, -1e300};
-    for (int b = 0; b < nb; ++b)
-        for (int d = 0; d < 3; ++d) {
-            bb[d] = fmin(bb[d], hb[b * 6 + d]);
-            bb[3 + d] = fmax(bb[3 + d], hb[b * 6 + 3 + d]);
-        }
     switch (dim) {
-    case 1: return knn_dim<1>(ws, data, n_data, query, n_query, k, q_ptr, out, st, bb);
-    case 2: return knn_dim<2>(ws, data, n_data, query, n_query, k, q_ptr, out, st, bb);
-    case 3: return knn_dim<3>(ws, data, n_data, query, n_query, k, q_ptr, out, st, bb);
+    case 1: return knn_dim<1>(ws, data, n_data, query, n_query, k, q_ptr, out, out_order, st);
+    case 2: return knn_dim<2>(ws, data, n_data, query, n_query, k, q_ptr, out, out_order, st);
+    case 3: return knn_dim<3>(ws, data, n_data, query, n_query, k, q_ptr, out, out_order, st);
     default: return hipErrorInvalidValue;
     }
 }

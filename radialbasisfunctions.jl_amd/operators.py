@@ -494,9 +494,13 @@ class RadialBasisOperator:
             if dm.size and (dm.min() < -1 or dm.max() > self.basis.poly_deg):
                 raise ArgumentError(f"poly_deg_map entries must lie in -1..{self.basis.poly_deg}")
             self._d_deg = t.as_tensor(dm.astype(np.int8), device=self.dev)
+        order = None
         if adjl is None:
             self.adj_ptr = None
-            self.adj_idx = _lib.knn(self._d_data, self._d_eval, self.k)
+            if self.n_eval >= self.SPATIAL_ORDER_MIN:
+                self.adj_idx, order = _lib.knn(self._d_data, self._d_eval, self.k, order=True)
+            else:
+                self.adj_idx = _lib.knn(self._d_data, self._d_eval, self.k)
         else:
             ptr, idx, kmax = _adjacency(adjl, self.n_eval)
             self.k = kmax
@@ -504,7 +508,7 @@ class RadialBasisOperator:
             self.adj_idx = _to_device(idx, self.dev, t.int32)
         self.status_counts = None
         self._host_weights = None
-        self._row_order = None
+        self._row_order = order  # (otherwise made at the first build)
         self._max_row = None
         self._plan = None
         self._tiles = None
@@ -604,7 +608,7 @@ class RadialBasisOperator:
         if self._row_order is None and self.n_eval >= self.SPATIAL_ORDER_MIN:
             # stencils solved (and rows applied) along a Z-curve of the eval points, so
             # neighbouring wavefronts gather neighbouring coordinates; results do not
-            # depend on the order
+            # depend on the order (the neighbour search gives one along with its result)
             self._row_order = _lib.spatial_order(self._d_eval)
         a.order = _lib.ptr(self._row_order)
         a.poly_deg_map = _lib.ptr(self._d_deg)
