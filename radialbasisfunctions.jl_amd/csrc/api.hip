@@ -55,6 +55,13 @@ int set_err(int code, const char* fmt, ...)
 // map: the null-space kernels serve only such builds).
 typedef std::tuple<int, int, int, int, int, int, int, int, int> TuneKey;
 
+// What a blocking build reports to the host, written by the device into pinned memory:
+// stencils per status, and how many the null-space kernel handed back.
+struct BuildReport {
+    unsigned long long hist[16];
+    int32_t handed;
+};
+
 // per-device library scratch (grow-only)
 struct DeviceState {
     rbfx::KnnWorkspace knn;
@@ -63,6 +70,8 @@ struct DeviceState {
     int32_t* fail_count = nullptr;
     int32_t* status = nullptr;
     size_t cap_status = 0;
+    // [0..15] status counts, [16] workgroups done, [17] hand-backs of a blocking build of one
+    // size (its own count: a captured build replays without the library's knowledge)
     unsigned long long* hist = nullptr;
     int32_t* reject_list = nullptr;
     size_t cap_reject = 0;
@@ -77,6 +86,8 @@ struct DeviceState {
     int32_t* nsc_list = nullptr;   // stencils the null-space kernels hand back
     size_t cap_nsc = 0;
     int32_t* nsc_count = nullptr;
+    BuildReport* report = nullptr;  // pinned host memory
+    bool report_clean = false;      // the accumulators behind the report are zero
     double* packed = nullptr;  // per-position stencil offsets of a register-kernel launch
     size_t cap_packed = 0;
 };
@@ -110,15 +121,41 @@ hipError_t grow(void** p, size_t& cap, size_t need)
     return e;
 }
 
-__global__ void k_hist16(const int32_t* __restrict__ st, int64_t n, unsigned long long* __restrict__ h)
+// Status counts of n stencils. A wavefront adds each status it sees once (nearly always
+// one status for all 64 lanes, where one LDS atomic per lane serialised on one word: 1.3M
+// stencils 53 -> 8 us); the last workgroup writes the report and clears the accumulators and
+// the hand-back count for the next build, so a build needs no clearing launches.
+__global__ __launch_bounds__(256) void k_report(const int32_t* __restrict__ st, int64_t n, unsigned long long* h,
+                                                unsigned int* done, int32_t* handed, BuildReport* out)
 {
     __shared__ unsigned int loc[16];
+    __shared__ unsigned int s_rank;
     if (threadIdx.x < 16) loc[threadIdx.x] = 0;
     __syncthreads();
-    for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.x * blockDim.x)
-        atomicAdd(&loc[st[i] & 15], 1u);
+    const int lane = threadIdx.x & 63;
+    const int64_t step = (int64_t)gridDim.x * 256;
+    for (int64_t i0 = blockIdx.x * (int64_t)256 + (threadIdx.x & ~63); i0 < n; i0 += step) {
+        const int64_t i = i0 + lane;
+        const int s = i < n ? st[i] & 15 : -1;
+        unsigned long long todo = __ballot(s >= 0);
+        while (todo) {
+            const int v = __builtin_amdgcn_readlane(s, __builtin_ctzll(todo));
+            const unsigned long long same = __ballot(s == v) & todo;
+            if (lane == 0) atomicAdd(&loc[v], (unsigned)__popcll(same));
+            todo &= ~same;
+        }
+    }
     __syncthreads();
     if (threadIdx.x < 16 && loc[threadIdx.x]) atomicAdd(&h[threadIdx.x], (unsigned long long)loc[threadIdx.x]);
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) s_rank = atomicAdd(done, 1u);
+    __syncthreads();
+    if (s_rank != gridDim.x - 1) return;
+    __threadfence();
+    if (threadIdx.x < 16) out->hist[threadIdx.x] = atomicExch(&h[threadIdx.x], 0ull);
+    if (threadIdx.x == 16) out->handed = handed ? atomicExch(handed, 0) : 0;
+    if (threadIdx.x == 17) *done = 0u;
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n)
@@ -357,8 +394,18 @@ struct HandBack {
     int32_t* count;
 };
 
+// The re-solve of a null-space launch's hand-backs, left to the caller: one launch of a
+// whole build needs no read-back of its own before the build's report.
+struct Deferred {
+    bool pending = false;
+    rbfx::BuildDev F;
+    int bucket = 0, rows_cap = 0;
+};
+
+// df (optional): leave the hand-backs to the caller, who clears hb.count
 static hipError_t launch_kernel_id(int kid, const rbfx::BuildDev& P, const Shape& sh, const HandBack& hb, int bucket,
-                                   bool fp32, int rows_cap, int64_t n_work, bool async, hipStream_t st)
+                                   bool fp32, int rows_cap, int64_t n_work, bool async, hipStream_t st,
+                                   Deferred* df = nullptr)
 {
     rbfx::BuildDev Q = P;
     if (fp32 && (kid == K_WIDE || kid == K_SYM || kid == K_REG32_F64 || kid == K_REG64_F64 || is_nsc(kid)))
@@ -368,13 +415,13 @@ static hipError_t launch_kernel_id(int kid, const rbfx::BuildDev& P, const Shape
         const int cap = bucket == 0 ? 32 : (bucket == 1 ? 64 : RBFX_MAX_N);
         Q.fail_list = hb.list;
         Q.fail_count = hb.count;
-        hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, hb.count);
+        if (!df) hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, hb.count);
         hipError_t e = kid == K_NSE ? rbfx::launch_build_nse(Q, sh.dim, n_work, st)
                                     : rbfx::launch_build_nsc(Q, sh.dim, std::min(sh.kmax, cap), sh.m,
                                                              kid == K_NSC2 ? 1 : 0, n_work, st);
         if (e != hipSuccess) return e;
         int32_t nf = (int32_t)n_work;
-        if (!async) {
+        if (!async && !df) {
             e = read_count(hb.count, &nf, st);
             if (e != hipSuccess) return e;
             g_stats[0] += nf;
@@ -386,6 +433,13 @@ static hipError_t launch_kernel_id(int kid, const rbfx::BuildDev& P, const Shape
         F.list = hb.list;
         F.list_len = hb.count;
         F.packed = nullptr;         // packed offsets follow the launch's own work order
+        if (df) {
+            df->pending = true;
+            df->F = F;
+            df->bucket = bucket;
+            df->rows_cap = rows_cap;
+            return hipSuccess;
+        }
         return launch_kernel_id(rook_for(bucket, Q.n_cols), F, sh, hb, bucket, false, rows_cap, nf, async, st);
     }
     if (kid == K_WIDE) return rbfx::launch_build_wide(Q, sh.dim, rows_cap, n_work, st);
@@ -547,8 +601,9 @@ static int reserve_nsc_list(DeviceState& ds, int64_t n, bool async)
 // run in one launch. Uneven stencils (ragged k, per-stencil degree) are classified into
 // size buckets in processing order, and each bucket runs on the kernel chosen for it.
 // (A tuning sample's queued FP32 failures are discarded with the old count.)
+// A blocking FP64 build of one size leaves its hand-backs in df.
 static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Shape& sh, DeviceState& ds, int nmax,
-                     bool fp32, Mode mode, const HandBack* static_hb, hipStream_t st)
+                     bool fp32, Mode mode, const HandBack* static_hb, hipStream_t st, Deferred* df = nullptr)
 {
     const int dim = a->dim;
     const bool async = mode != Mode::kBlocking;
@@ -584,7 +639,9 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
         g_bucket_n[b] = a->n_eval;
         g_bucket_kernel[b] = kid;
         if (fp32) hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, ds.fail_count);
-        HIPCHK(launch_kernel_id(kid, Q, sh, hb, b, fp32, nmax, a->n_eval, async, st));
+        if (!is_nsc(kid)) df = nullptr;
+        if (df) hb.count = (int32_t*)(ds.hist + 17);
+        HIPCHK(launch_kernel_id(kid, Q, sh, hb, b, fp32, nmax, a->n_eval, async, st, df));
         return RBFX_OK;
     }
     if (mode == Mode::kNoAlloc)  // (the entry point refuses these builds before any work)
@@ -821,7 +878,12 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         if (!async) HIPCHK(grow((void**)&ds.status, ds.cap_status, need));
         status = ds.status;
     }
-    if (!ds.hist && !async) HIPCHK(hipMalloc((void**)&ds.hist, 16 * sizeof(unsigned long long)));
+    if (!async) {
+        if (!ds.hist) HIPCHK(hipMalloc((void**)&ds.hist, 18 * sizeof(unsigned long long)));
+        if (!ds.report) HIPCHK(hipHostMalloc((void**)&ds.report, sizeof(BuildReport), hipHostMallocDefault));
+        if (!ds.report_clean) hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, ds.hist, 18);
+        ds.report_clean = false;  // (until this build's report has cleared them again)
+    }
 
     rbfx::BuildDev P;
     std::memset(&P, 0, sizeof(P));
@@ -884,11 +946,13 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         return hipEventRecord(ds.ev[i], st);
     };
     HIPCHK(mark(0));
-    if (a->precision == RBFX_PREC_FP64) {
-        const int rc = solve_all(a, P, sh, ds, nmax, false, mode, mode == Mode::kNoAlloc ? &static_hb : nullptr, st);
+    Deferred df;
+    const bool plain = a->precision == RBFX_PREC_FP64;  // (one stage: marks 0 and 1 only)
+    if (plain) {
+        const int rc = solve_all(a, P, sh, ds, nmax, false, mode, mode == Mode::kNoAlloc ? &static_hb : nullptr, st,
+                                 async ? nullptr : &df);
         if (rc != RBFX_OK) return rc;
         HIPCHK(mark(1));
-        HIPCHK(mark(2));
     } else {
         if (!async) {
             HIPCHK(grow((void**)&ds.fail_list, ds.cap_fail, need));
@@ -991,25 +1055,43 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
                 HIPCHK(rbfx::launch_build(F, a->dim, std::min(nmax, 64), false, nfail, st));
         }
     }
-    HIPCHK(mark(3));
+    if (!plain) HIPCHK(mark(3));
     if (async) {
         HIPCHK(hipGetLastError());
         g_err.clear();
         return RBFX_OK;
     }
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, st, ds.hist, 16);
-    const int64_t hb = std::min<int64_t>((a->n_eval + 255) / 256, 4096);
-    hipLaunchKernelGGL(k_hist16, dim3((unsigned)hb), dim3(256), 0, st, status, a->n_eval, ds.hist);
-    unsigned long long h[16];
-    HIPCHK(hipMemcpyAsync(h, ds.hist, sizeof(h), hipMemcpyDeviceToHost, st));
-    HIPCHK(hipStreamSynchronize(st));
-    for (int i = 0; i < 3; ++i) {
-        float ms = 0.f;
-        HIPCHK(hipEventElapsedTime(&ms, ds.ev[i], ds.ev[i + 1]));
-        g_stage_ms[i] = ms;
+    const int64_t rb = std::min<int64_t>((a->n_eval + 255) / 256, 1024);
+    auto report = [&](int32_t* handed) -> hipError_t {
+        hipLaunchKernelGGL(k_report, dim3((unsigned)rb), dim3(256), 0, st, status, a->n_eval, ds.hist,
+                           (unsigned int*)(ds.hist + 16), handed, ds.report);
+        return hipStreamSynchronize(st);
+    };
+    int32_t* handed = (int32_t*)(ds.hist + 17);
+    HIPCHK(report(df.pending ? handed : nullptr));
+    const int32_t nf = df.pending ? ds.report->handed : 0;
+    g_stats[0] += nf;
+    if (nf > 0) {
+        // (the list's length is the count, which the report cleared)
+        hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(1), 0, st, handed, nf);
+        HIPCHK(launch_kernel_id(rook_for(df.bucket, df.F.n_cols), df.F, sh, HandBack{ds.nsc_list, handed}, df.bucket,
+                                false, df.rows_cap, nf, false, st));
+        HIPCHK(mark(1));
+        HIPCHK(report(handed));
     }
-    {
+    ds.report_clean = true;
+    unsigned long long h[16];
+    for (int i = 0; i < 16; ++i) h[i] = ds.report->hist[i];
+    if (plain) {
         float ms = 0.f;
+        HIPCHK(hipEventElapsedTime(&ms, ds.ev[0], ds.ev[1]));
+        g_stage_ms[0] = g_stage_ms[3] = ms;
+    } else {
+        float ms = 0.f;
+        for (int i = 0; i < 3; ++i) {
+            HIPCHK(hipEventElapsedTime(&ms, ds.ev[i], ds.ev[i + 1]));
+            g_stage_ms[i] = ms;
+        }
         HIPCHK(hipEventElapsedTime(&ms, ds.ev[0], ds.ev[3]));
         g_stage_ms[3] = ms;
     }
