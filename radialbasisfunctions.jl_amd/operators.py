@@ -451,6 +451,10 @@ class RadialBasisOperator:
     scipy.sparse matrices (a tuple for rank >= 1)."""
 
     SPATIAL_ORDER_MIN = 65536  # below this the X vector sits in L2 anyway
+    # up to here the processing order is the neighbour search's curve over its cells, which
+    # costs 20 us and serves builds and applies as well as a Morton sort (150 us) while X fits
+    # one XCD's L2 (4 MB); beyond, the sort's finer order (1M points, 2-D: apply 62 against 68 us)
+    CELL_ORDER_MAX = 524288
     SPMV_MAPPING = 0  # rbfx_spmv_args.mapping: 0 automatic, 1 lanes per row, 2 staged through LDS, 3 vector loads,
     # 4 source tiles
     SOURCE_TILE_FIELDS = 8  # mapping 4 (source tiles) serves applies of this many fields or more
@@ -497,7 +501,7 @@ class RadialBasisOperator:
         order = None
         if adjl is None:
             self.adj_ptr = None
-            if self.n_eval >= self.SPATIAL_ORDER_MIN:
+            if self.SPATIAL_ORDER_MIN <= self.n_eval <= self.CELL_ORDER_MAX:
                 self.adj_idx, order = _lib.knn(self._d_data, self._d_eval, self.k, order=True)
             else:
                 self.adj_idx = _lib.knn(self._d_data, self._d_eval, self.k)
@@ -608,7 +612,7 @@ class RadialBasisOperator:
         if self._row_order is None and self.n_eval >= self.SPATIAL_ORDER_MIN:
             # stencils solved (and rows applied) along a Z-curve of the eval points, so
             # neighbouring wavefronts gather neighbouring coordinates; results do not
-            # depend on the order (the neighbour search gives one along with its result)
+            # depend on the order
             self._row_order = _lib.spatial_order(self._d_eval)
         a.order = _lib.ptr(self._row_order)
         a.poly_deg_map = _lib.ptr(self._d_deg)
