@@ -198,20 +198,22 @@ __device__ __forceinline__ double sqdist(const double* a, const double (&q)[DIM]
 constexpr int kSmallPoints = 4000;
 constexpr int kSmallCells = 4 * kSmallPoints + 16;  // (knn_grid_size's bound; 64,064 bytes of LDS)
 
-// Bounding box, grid, counting sort: one workgroup.
+// Bounding box, grid, counting sort: one workgroup (512 threads: the grid sizing needs the
+// registers that 1,024 would not leave).
+constexpr int kSmallThreads = 512;
 template <int DIM>
-__global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x, int n, double target, Grid* grid,
+__global__ __launch_bounds__(kSmallThreads) void k_bin_small(const double* __restrict__ x, int n, double target, Grid* grid,
                                                     int32_t* __restrict__ start, int32_t* __restrict__ sorted_idx,
                                                     double* __restrict__ sorted_x)
 {
     __shared__ int32_t cnt[kSmallCells];
-    __shared__ double lds[16 * 6];
-    __shared__ int wsum[16];
+    __shared__ double lds[kSmallThreads / 64 * 6];
+    __shared__ int wsum[kSmallThreads / 64];
     __shared__ Grid G;
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
     double v[6];
-    box_of(x, n, DIM, t, 1024, v);
-    block_box<1024>(v, lds);
+    box_of(x, n, DIM, t, kSmallThreads, v);
+    block_box<kSmallThreads>(v, lds);
     if (t == 0) {
         double ext[3];
         for (int d = 0; d < 3; ++d) ext[d] = v[3 + d] - v[d];
@@ -223,12 +225,12 @@ __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x
     }
     __syncthreads();
     const int ncell = G.n[0] * G.n[1] * G.n[2];
-    for (int c = t; c < ncell; c += 1024) cnt[c] = 0;
+    for (int c = t; c < ncell; c += kSmallThreads) cnt[c] = 0;
     __syncthreads();
-    for (int i = t; i < n; i += 1024) atomicAdd(&cnt[cell_of<DIM>(x + (int64_t)i * DIM, G)], 1);
+    for (int i = t; i < n; i += kSmallThreads) atomicAdd(&cnt[cell_of<DIM>(x + (int64_t)i * DIM, G)], 1);
     __syncthreads();
     // exclusive scan: each thread a run of cells, then over the threads
-    const int run = (ncell + 1023) / 1024, c0 = t * run;
+    const int run = (ncell + kSmallThreads - 1) / kSmallThreads, c0 = t * run;
     int sum = 0;
     for (int c = c0; c < c0 + run && c < ncell; ++c) sum += cnt[c];
     int inc = sum;
@@ -248,7 +250,7 @@ __global__ __launch_bounds__(1024) void k_bin_small(const double* __restrict__ x
     }
     if (t == 0) start[ncell] = n;
     __syncthreads();
-    for (int i = t; i < n; i += 1024) {
+    for (int i = t; i < n; i += kSmallThreads) {
         const int slot = atomicAdd(&cnt[cell_of<DIM>(x + (int64_t)i * DIM, G)], 1);
         sorted_idx[slot] = i;
 #pragma unroll
@@ -677,7 +679,7 @@ static hipError_t knn_dim(KnnWorkspace& ws, const double* data, int64_t n_data, 
     Grid G;
     if (n_data <= kSmallPoints && !out_order) {
         if ((err = ws.reserve_cells(kSmallCells, true)) != hipSuccess) return err;
-        hipLaunchKernelGGL(k_bin_small<DIM>, dim3(1), dim3(1024), 0, st, data, (int)n_data, target, (Grid*)ws.grid,
+        hipLaunchKernelGGL(k_bin_small<DIM>, dim3(1), dim3(kSmallThreads), 0, st, data, (int)n_data, target, (Grid*)ws.grid,
                            ws.start, ws.sidx, ws.sx);
         return launch_query<DIM>(ws, query, self ? ws.sidx : nullptr, n_query, k, q_ptr, out, st);
     }
