@@ -161,8 +161,8 @@ SOLVE_KERNELS = {
         "k_nsc<32, 1, 20, 6, 2, 1, 1, 3>", "valu-fp64"),
     6: ("k_nsc<8,3,20,6,2,1,1,2> (null-space Cholesky + FP64 refinement, 8 lanes x 3 rows per stencil)",
         "k_nsc<8, 3, 20, 6, 2, 1, 1, 2>", "valu-fp64"),
-    8: ("k_nse<3,2,6,15,1,4> (null-space elimination in registers, 16 lanes per stencil)",
-        "k_nse<3, 2, 6, 15, 1, 4>", "valu-fp64"),
+    8: ("k_nse<3,2,6,15,1,4,false> (null-space elimination in registers, 16 lanes per stencil)",
+        "k_nse<3, 2, 6, 15, 1, 4, false>", "valu-fp64"),
 }
 
 

@@ -60,6 +60,7 @@ typedef std::tuple<int, int, int, int, int, int, int, int, int> TuneKey;
 struct BuildReport {
     unsigned long long hist[16];
     int32_t handed;
+    int32_t counts[32];  // (an uneven build's list lengths)
 };
 
 // per-device library scratch (grow-only)
@@ -77,10 +78,10 @@ struct DeviceState {
     size_t cap_reject = 0;
     int32_t* reject_count = nullptr;
     hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};  // stage boundaries of a build
-    // size buckets of an uneven build: three lists of stencil ids (n_eval each) + counts
+    // lists of an uneven build: stencil ids per size bucket and null-space class (n_eval each)
     int32_t* bucket_list = nullptr;
     size_t cap_bucket = 0;
-    int32_t* bucket_count = nullptr;  // [3] list lengths, [3..5] tuning sample sizes
+    int32_t* bucket_count = nullptr;  // [kCounts] list lengths (k_classify), [kSamples..] tuning sample sizes
     hipEvent_t tev[2] = {nullptr, nullptr};
     std::map<TuneKey, int> tuned;  // configuration -> kernel the autotuner picked
     int32_t* nsc_list = nullptr;   // stencils the null-space kernels hand back
@@ -174,9 +175,9 @@ __global__ __launch_bounds__(kReportThreads) void k_report(const int32_t* __rest
     __syncthreads();
     if (s_rank != gridDim.x - 1) return;
     __threadfence();
-    if (threadIdx.x < 16) out->hist[threadIdx.x] = atomicExch(&h[threadIdx.x], 0ull);
-    if (threadIdx.x == 16) out->handed = handed ? atomicExch(handed, 0) : 0;
-    if (threadIdx.x == 17) *done = 0u;
+    if (t < 16) out->hist[t] = atomicExch(&h[t], 0ull);
+    if (t == 16) out->handed = handed ? atomicExch(handed, 0) : 0;
+    if (t == 17) *done = 0u;
 }
 
 __global__ void k_zero_u64(unsigned long long* p, int n)
@@ -185,15 +186,27 @@ __global__ void k_zero_u64(unsigned long long* p, int n)
 }
 
 __global__ void k_zero_i32(int32_t* p) { *p = 0; }
+__global__ void k_zero_counts(int32_t* p) { p[threadIdx.x] = 0; }
 __global__ void k_set_i32(int32_t* p, int32_t v) { *p = v; }
 
-// Size buckets of an uneven build, in processing order: n = k + m <= 32, <= 64, above.
-// Lanes of a wavefront append with one atomic per bucket, so each list keeps the
-// (spatial) order of the stencils at wavefront granularity.
-__global__ __launch_bounds__(256) void k_classify(const rbfx::BuildDev P, int dim, int32_t* lists, int32_t* counts)
+// Lists of an uneven build, in processing order: the size buckets n = k + m <= 32, <= 64,
+// above, and the null-space classes (a stencil of a class is in its class's list only).
+// counts: [0..2] bucket lists, [kTotals..] stencils of each size whatever their list,
+// [kClasses..] class lists. One atomic per list and workgroup (one per
+// wavefront serialises on the list's count: 254 us for 1.3M stencils, now 39), and the lists keep the order of 1,024 stencils.
+constexpr int kSamples = 3, kTotals = 8, kClasses = 16, kCounts = 32;
+struct ClassTab {
+    int n;
+    rbfx::NseClass c[rbfx::kNseClasses];
+};
+__global__ __launch_bounds__(1024) void k_classify(const rbfx::BuildDev P, int dim, ClassTab tab, int32_t* lists,
+                                                   int32_t* counts)
 {
-    const int64_t wi = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    int b = -1;
+    constexpr int NL = 3 + rbfx::kNseClasses;
+    __shared__ int wcnt[16][NL], wtot[16][3], base[NL];
+    const int64_t wi = (int64_t)blockIdx.x * 1024 + threadIdx.x;
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    int l = -1, b = -1;
     int32_t e = 0;
     if (wi < P.n_eval) {
         e = P.order ? P.order[wi] : (int32_t)wi;
@@ -201,21 +214,37 @@ __global__ __launch_bounds__(256) void k_classify(const rbfx::BuildDev P, int di
             const int kk = P.adj_ptr ? (int)(P.adj_ptr[e + 1] - P.adj_ptr[e]) : P.k;
             const int m = rbfx::stencil_n_mono(P, e, dim);
             const int nn = kk + (m < 0 ? 0 : m);
-            b = nn <= 32 ? 0 : (nn <= 64 ? 1 : 2);
+            l = b = nn <= 32 ? 0 : (nn <= 64 ? 1 : 2);
+            for (int c = 0; c < tab.n; ++c)
+                if (m == tab.c[c].m && kk - m > tab.c[c].lo && kk - m <= tab.c[c].hi) l = 3 + c;
         }
     }
-    const int lane = threadIdx.x & 63;
-    for (int bb = 0; bb < 3; ++bb) {
-        const unsigned long long mask = __ballot(b == bb);
-        if (!mask) continue;
-        const int leader = __builtin_ctzll(mask);
-        int base = 0;
-        if (lane == leader) base = atomicAdd(&counts[bb], __popcll(mask));
-        base = __shfl(base, leader, 64);
-        if (b == bb) {
-            const int rank = __popcll(mask & ((1ull << lane) - 1ull));
-            lists[(int64_t)bb * P.n_eval + base + rank] = e;
-        }
+    int rank = 0;
+    for (int q = 0; q < 3 + tab.n; ++q) {
+        const unsigned long long mask = __ballot(l == q);
+        if (l == q) rank = __popcll(mask & ((1ull << lane) - 1ull));
+        if (lane == 0) wcnt[w][q] = __popcll(mask);
+    }
+    for (int q = 0; q < 3; ++q) {
+        const unsigned long long mask = __ballot(b == q);
+        if (lane == 0) wtot[w][q] = __popcll(mask);
+    }
+    __syncthreads();
+    const int t = threadIdx.x;
+    if (t < 3 + tab.n) {
+        int sum = 0;
+        for (int q = 0; q < 16; ++q) sum += wcnt[q][t];
+        base[t] = sum ? atomicAdd(&counts[t < 3 ? t : kClasses + t - 3], sum) : 0;
+    } else if (t >= 64 && t < 67) {
+        int sum = 0;
+        for (int q = 0; q < 16; ++q) sum += wtot[q][t - 64];
+        if (sum) atomicAdd(&counts[kTotals + t - 64], sum);
+    }
+    __syncthreads();
+    if (l >= 0) {
+        int at = base[l] + rank;
+        for (int q = 0; q < w; ++q) at += wcnt[q][l];
+        lists[(int64_t)l * P.n_eval + at] = e;
     }
 }
 
@@ -563,6 +592,20 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
     return RBFX_OK;
 }
 
+// Whether pick_kernel would time its candidates for this bucket of `count` stencils.
+static bool would_time(const rbfx_build_args* a, const Shape& sh, const DeviceState& ds, int bucket, bool fp32,
+                       int64_t count)
+{
+    if (count < kTuneMin || (g_force_kernel[bucket] >= 0 && kernel_serves(g_force_kernel[bucket], bucket, fp32, sh, true)))
+        return false;
+    const TuneKey key{a->dim,         sh.n_cols, a->precision, bucket, sh.kmax, sh.m, sh.basis_kind, sh.hermite ? 1 : 0,
+                      sh.uniform ? 1 : 0};
+    auto it = ds.tuned.find(key);
+    if (it != ds.tuned.end() && kernel_serves(it->second, bucket, fp32, sh, false)) return false;
+    auto jt = g_tune_saved.find(key);
+    return !(jt != g_tune_saved.end() && kernel_serves(jt->second, bucket, fp32, sh, false));
+}
+
 // Device time of one launch of kernel kid on a sample (a warm-up run, then a timed one).
 static int time_sample(int kid, const rbfx::BuildDev& S, const Shape& sh, DeviceState& ds, const HandBack& hb,
                        int bucket, bool fp32, int rows_cap, int32_t sample, hipStream_t st, float* ms)
@@ -640,7 +683,17 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
         if (rc != RBFX_OK) return rc;
         hb = HandBack{ds.nsc_list, ds.nsc_count};
     }
+    // Uneven builds: more than one size bucket, and null-space classes beside them (pinned
+    // kernels and plans serve every stencil of their bucket or build: no classes). Ragged
+    // stencils of up to 32 rows stay one launch, which the build without allocation shares.
     const bool uneven = (a->adj_ptr || a->poly_deg_map) && nmax > 32;
+    ClassTab tab;
+    tab.n = 0;
+    const bool pinned = g_force_plan != 0 || g_force_kernel[0] >= 0 || g_force_kernel[1] >= 0 || g_force_kernel[2] >= 0;
+    if (uneven && !pinned && !sh.lambda && mode != Mode::kNoAlloc)
+        tab.n = rbfx::nse_classes(sh.basis_kind, dim, sh.poly_deg, sh.n_cols, tab.c);
+    // (an asynchronous build uses what an earlier blocking one made room for)
+    if (async && (!ds.bucket_count || ds.cap_bucket < sizeof(int32_t) * (3 + tab.n) * (size_t)a->n_eval)) tab.n = 0;
     if (!uneven) {
         const int b = nmax <= 32 ? 0 : (nmax <= 64 ? 1 : 2);
         int kid = K_REG32;
@@ -693,55 +746,103 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
         return RBFX_OK;
     };
     if (plan == kPlanSingle) return launch_single();
-    const size_t need = sizeof(int32_t) * 3 * (size_t)a->n_eval;
+    const size_t need = sizeof(int32_t) * (3 + tab.n) * (size_t)a->n_eval;
     if (!async) {
         HIPCHK(grow((void**)&ds.bucket_list, ds.cap_bucket, need));
-        if (!ds.bucket_count) HIPCHK(hipMalloc((void**)&ds.bucket_count, 6 * sizeof(int32_t)));
+        if (!ds.bucket_count) HIPCHK(hipMalloc((void**)&ds.bucket_count, kCounts * sizeof(int32_t)));
     } else if (ds.cap_bucket < need || !ds.bucket_count) {
         return set_err(RBFX_EINVAL, "asynchronous build: run one blocking build with these sizes first");
     }
-    for (int b = 0; b < 3; ++b) hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, ds.bucket_count + b);
-    hipLaunchKernelGGL(k_classify, dim3((unsigned)((a->n_eval + 255) / 256)), dim3(256), 0, st, P, dim,
-                       ds.bucket_list, ds.bucket_count);
-    HIPCHK(hipGetLastError());
-    int32_t cnt[3] = {(int32_t)a->n_eval, (int32_t)a->n_eval, (int32_t)a->n_eval};
-    if (!async) {
-        HIPCHK(hipMemcpyAsync(cnt, ds.bucket_count, sizeof(cnt), hipMemcpyDeviceToHost, st));
+    const int32_t all = (int32_t)a->n_eval;
+    int32_t cnt[kCounts];
+    auto classify = [&](const ClassTab& t) -> int {
+        hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(kCounts), 0, st, ds.bucket_count);
+        hipLaunchKernelGGL(k_classify, dim3((unsigned)((a->n_eval + 1023) / 1024)), dim3(1024), 0, st, P, dim, t,
+                           ds.bucket_list, ds.bucket_count);
+        HIPCHK(hipGetLastError());
+        return RBFX_OK;
+    };
+    auto read_counts = [&]() -> int {
+        if (async) {  // (grids cover every stencil, the kernels read the list lengths)
+            for (int i = 0; i < kCounts; ++i) cnt[i] = all;
+            if (nmax <= 64) cnt[2] = 0;
+            return RBFX_OK;
+        }
+        HIPCHK(hipMemcpyAsync(ds.report->counts, ds.bucket_count, sizeof(cnt), hipMemcpyDeviceToHost, st));
         HIPCHK(hipStreamSynchronize(st));
-    }
+        std::memcpy(cnt, ds.report->counts, sizeof(cnt));
+        return RBFX_OK;
+    };
+    auto run_classes = [&]() -> int {
+        for (int c = 0; c < tab.n; ++c) {
+            const int32_t n = cnt[kClasses + c];
+            if (n <= 0) continue;
+            rbfx::BuildDev Q = P;
+            Q.list = ds.bucket_list + (int64_t)(3 + c) * a->n_eval;
+            Q.list_len = ds.bucket_count + kClasses + c;
+            Q.fail_list = ds.bucket_list;
+            Q.fail_count = ds.bucket_count;
+            Q.fail_stride = a->n_eval;
+            if (fp32) Q.ok_status = RBFX_ST_FP64;
+            HIPCHK(rbfx::launch_build_nse_class(Q, dim, tab.c[c], n, st));
+        }
+        return RBFX_OK;
+    };
+    auto bucket_of = [&](int b) {
+        rbfx::BuildDev Q = P;
+        Q.list = ds.bucket_list + (int64_t)b * a->n_eval;
+        Q.list_len = ds.bucket_count + kSamples + b;
+        return Q;
+    };
     // (the LDS kernels size their tables by rows_cap: the bucket's bound or the largest
     // stencil of the build, whichever is smaller)
     const int rows_cap[3] = {std::min(32, nmax), std::min(64, nmax), std::min(nmax, RBFX_MAX_N)};
+    int rc = classify(tab);
+    if (rc == RBFX_OK) rc = read_counts();
+    if (rc != RBFX_OK) return rc;
+    // The first time a configuration is seen, its buckets' kernels are timed on samples of
+    // all their stencils (also those of a class), and the plan is decided when every
+    // nonempty bucket was just timed: the single launch's kernel on each bucket's sample
+    // against the bucket's own pick, weighted by the stencils that kernel would get, and the
+    // classes' launches.
+    bool timing = false;
+    if (!async)
+        for (int b = 0; b < 3; ++b) timing = timing || would_time(a, sh, ds, b, fp32, cnt[kTotals + b]);
     int kid[3];
-    float per_stencil[3];
-    for (int b = 0; b < 3; ++b) {
-        rbfx::BuildDev Q = P;
-        Q.list = ds.bucket_list + (int64_t)b * a->n_eval;
-        Q.list_len = ds.bucket_count + 3 + b;
-        const int rc = pick_kernel(a, Q, sh, ds, hb, b, fp32, rows_cap[b], cnt[b], ds.bucket_count + 3 + b, mode, st,
-                                   &kid[b], &per_stencil[b]);
-        if (rc != RBFX_OK) return rc;
-    }
-    // Plan choice, once per configuration, when every nonempty bucket was just timed:
-    // the single launch's kernel on each bucket's sample against the bucket's own pick,
-    // weighted by the bucket counts.
-    if (plan == 0 && !async && single_ok) {
+    if (timing) {
+        int32_t rest[3] = {cnt[0], cnt[1], cnt[2]};
+        float class_ms = 0.f;
+        ClassTab none;
+        none.n = 0;
+        if (tab.n > 0) {
+            for (int i = 0; i < 2; ++i)
+                if (!ds.tev[i]) HIPCHK(hipEventCreate(&ds.tev[i]));
+            HIPCHK(hipEventRecord(ds.tev[0], st));
+            if ((rc = run_classes()) != RBFX_OK) return rc;
+            HIPCHK(hipEventRecord(ds.tev[1], st));
+            HIPCHK(hipEventSynchronize(ds.tev[1]));
+            HIPCHK(hipEventElapsedTime(&class_ms, ds.tev[0], ds.tev[1]));
+            if ((rc = classify(none)) != RBFX_OK) return rc;
+            if ((rc = read_counts()) != RBFX_OK) return rc;
+        }
+        float per_stencil[3];
         bool all_timed = true;
-        for (int b = 0; b < 3; ++b)
+        for (int b = 0; b < 3; ++b) {
+            rc = pick_kernel(a, bucket_of(b), sh, ds, hb, b, fp32, rows_cap[b], cnt[b],
+                             ds.bucket_count + kSamples + b, mode, st, &kid[b], &per_stencil[b]);
+            if (rc != RBFX_OK) return rc;
             if (cnt[b] > 0 && per_stencil[b] < 0.f) all_timed = false;
-        if (all_timed) {
-            double est_bucketed = 0.0, est_single = 0.0;
+        }
+        if (plan == 0 && single_ok && all_timed) {
+            double est_bucketed = class_ms, est_single = 0.0;
             for (int b = 0; b < 3; ++b) {
                 if (cnt[b] <= 0) continue;
                 const int32_t sample = (int32_t)std::min<int64_t>(cnt[b], kTuneSample);
-                rbfx::BuildDev S = P;
-                S.list = ds.bucket_list + (int64_t)b * a->n_eval;
-                S.list_len = ds.bucket_count + 3 + b;
-                hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(1), 0, st, ds.bucket_count + 3 + b, sample);
+                hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(1), 0, st, ds.bucket_count + kSamples + b, sample);
                 float ms = 0.f;
-                const int rc = time_sample(K_SYM, S, sh, ds, hb, 2, fp32, cap_single, sample, st, &ms);
+                rc = time_sample(K_SYM, bucket_of(b), sh, ds, hb, 2, fp32, cap_single, sample, st, &ms);
                 if (rc != RBFX_OK) return rc;
-                est_bucketed += (double)cnt[b] * per_stencil[b];
+                est_bucketed += (double)rest[b] * per_stencil[b];
                 est_single += (double)cnt[b] * ms / sample;
             }
             g_stats[0] = 0;  // (sample runs)
@@ -749,14 +850,34 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
             ds.tuned[pkey] = plan;
             if (plan == kPlanSingle) return launch_single();
         }
+        if (tab.n > 0) {  // (the lists without the classes' stencils again)
+            if ((rc = classify(tab)) != RBFX_OK) return rc;
+            if ((rc = read_counts()) != RBFX_OK) return rc;
+        }
     }
+    int64_t total[3], listed[3];
+    for (int b = 0; b < 3; ++b) {
+        total[b] = cnt[kTotals + b];
+        listed[b] = cnt[b];
+    }
+    if (tab.n > 0) {
+        if ((rc = run_classes()) != RBFX_OK) return rc;
+        if ((rc = read_counts()) != RBFX_OK) return rc;  // (with what they handed back)
+        if (!async)
+            for (int b = 0; b < 3; ++b) g_stats[0] += cnt[b] - listed[b];
+    }
+    if (!timing)
+        for (int b = 0; b < 3; ++b) {
+            rc = pick_kernel(a, bucket_of(b), sh, ds, hb, b, fp32, rows_cap[b], std::min<int64_t>(cnt[b], kTuneMin - 1),
+                             nullptr, mode, st, &kid[b]);
+            if (rc != RBFX_OK) return rc;
+        }
     if (fp32) hipLaunchKernelGGL(k_zero_i32, dim3(1), dim3(1), 0, st, ds.fail_count);
     for (int b = 0; b < 3; ++b) {
-        g_bucket_n[b] = async ? -1 : cnt[b];
-        g_bucket_kernel[b] = kid[b];
+        g_bucket_n[b] = async ? -1 : total[b];
+        g_bucket_kernel[b] = !async && cnt[b] <= 0 && total[b] > 0 ? K_NSE : kid[b];
         if (cnt[b] <= 0) continue;
-        rbfx::BuildDev Q = P;
-        Q.list = ds.bucket_list + (int64_t)b * a->n_eval;
+        rbfx::BuildDev Q = bucket_of(b);
         Q.list_len = ds.bucket_count + b;
         HIPCHK(launch_kernel_id(kid[b], Q, sh, hb, b, fp32, rows_cap[b], cnt[b], async, st));
     }
@@ -1028,7 +1149,7 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         }
         if (a->precision == RBFX_PREC_LEARNED) {
             // the rejected stencils (one size class) on the kernel picked for it
-            if (!async && !ds.bucket_count) HIPCHK(hipMalloc((void**)&ds.bucket_count, 6 * sizeof(int32_t)));
+            if (!async && !ds.bucket_count) HIPCHK(hipMalloc((void**)&ds.bucket_count, kCounts * sizeof(int32_t)));
             const int b = nmax <= 32 ? 0 : 1;
             int kid = b == 0 ? K_REG32 : K_REG64;
             rbfx::BuildDev Q = P;  // (P itself stays unpacked for the FP64 re-solve below)

@@ -66,6 +66,7 @@ struct BuildDev {
     // FP32 path: stencils that must be re-solved in FP64 are appended here
     int32_t* fail_list;
     int32_t* fail_count;
+    int64_t fail_stride;  // ragged null-space launches: entries per size bucket's list
     int refine_steps;
     double accept_tol;
     int ok_status;  // status written for a stencil solved by this launch

@@ -15,4 +15,17 @@ bool nse_fits(int basis_kind, int dim, int k, int m, int n_cols);
 // the rook-pivoted kernels; every other stencil gets status P.ok_status.
 hipError_t launch_build_nse(const BuildDev& P, int dim, int64_t n_work, hipStream_t s);
 
+// Shape classes of an uneven build (ragged stencils, per-stencil degrees): stencils of m
+// monomials and lo < k - m <= hi points beyond them run together in one launch. At most
+// kNseClasses of them, for the degrees up to poly_deg that a kernel is built for.
+struct NseClass {
+    int m, lo, hi;
+};
+constexpr int kNseClasses = 8;
+int nse_classes(int basis_kind, int dim, int poly_deg, int n_cols, NseClass* out);
+
+// The stencils of P.list, all of class c. What they hand back goes to the list of its size
+// bucket (k + m <= 32, <= 64, above): P.fail_list + b * P.fail_stride, P.fail_count + b.
+hipError_t launch_build_nse_class(const BuildDev& P, int dim, const NseClass& c, int64_t n_work, hipStream_t s);
+
 }  // namespace rbfx

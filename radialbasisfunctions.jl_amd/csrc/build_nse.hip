@@ -1,6 +1,7 @@
 // Dispatch of the null-space build by elimination over basis, dimension and stencil
 // shape (kernel template in build_nse_kernel.h, instantiations in build_nse_*.hip).
 #include "build_nse.h"
+#include "build_nsc.h"
 
 namespace rbfx {
 
@@ -11,6 +12,9 @@ hipError_t launch_nse_3d_low(const BuildDev& P, int64_t n_work, hipStream_t s);
 hipError_t launch_nse_3d_phs3(const BuildDev& P, int64_t n_work, hipStream_t s);
 hipError_t launch_nse_3d_phs5(const BuildDev& P, int64_t n_work, hipStream_t s);
 hipError_t launch_nse_3d_phs7(const BuildDev& P, int64_t n_work, hipStream_t s);
+
+hipError_t launch_nse_rag_2d(const BuildDev& P, int m, int hi, int64_t n_work, hipStream_t s);
+hipError_t launch_nse_rag_3d(const BuildDev& P, int m, int hi, int64_t n_work, hipStream_t s);
 
 // The null points (k - m) and the operator columns share the lanes of one or two slots
 // of 16, so at most 26 null points; the monomial tables of degree 1 to 4 (2-D) and 1 to 3
@@ -51,6 +55,39 @@ hipError_t launch_build_nse(const BuildDev& P, int dim, int64_t n_work, hipStrea
     if (P.basis_kind == RBFX_PHS3) return launch_nse_3d_phs3(P, n_work, s);
     if (P.basis_kind == RBFX_PHS5) return launch_nse_3d_phs5(P, n_work, s);
     return launch_nse_3d_phs7(P, n_work, s);
+}
+
+// operator columns of the kernel that serves n_cols of them (0: none)
+static int nse_rc(int dim, int n_cols)
+{
+    if (dim == 2) return n_cols <= 3 ? n_cols : 0;
+    if (dim == 3) return n_cols == 2 ? 3 : (n_cols == 5 ? 6 : (n_cols <= 6 ? n_cols : 0));
+    return 0;
+}
+
+// Built: PHS3 with 6 and 10 monomials and PHS5 with 10 in 2-D, PHS3 with 10 and PHS5 with 20
+// in 3-D (the basis must be definite with each stencil's own degree).
+int nse_classes(int kind, int dim, int poly_deg, int n_cols, NseClass* out)
+{
+    const int rc = n_cols >= 1 ? nse_rc(dim, n_cols) : 0;
+    int n = 0;
+    if (rc == 0) return 0;
+    for (int deg = 0; deg <= poly_deg; ++deg) {
+        const int m = n_mono_of(dim, deg);
+        const bool built = dim == 2 ? (kind == RBFX_PHS3 && (m == 6 || m == 10)) || (kind == RBFX_PHS5 && m == 10)
+                                    : (kind == RBFX_PHS3 && m == 10) || (kind == RBFX_PHS5 && m == 20);
+        if (!built || nsc_sign(kind, deg) == 0 || n + 2 > kNseClasses) continue;
+        const int one = m == 20 ? 20 : 16 - rc;
+        out[n++] = NseClass{m, 0, one};
+        out[n++] = NseClass{m, one, 26};
+    }
+    return n;
+}
+
+hipError_t launch_build_nse_class(const BuildDev& P, int dim, const NseClass& c, int64_t n_work, hipStream_t s)
+{
+    if (P.out_lambda) return hipErrorInvalidValue;
+    return dim == 2 ? launch_nse_rag_2d(P, c.m, c.hi, n_work, s) : launch_nse_rag_3d(P, c.m, c.hi, n_work, s);
 }
 
 }  // namespace rbfx

@@ -176,6 +176,17 @@ struct NseLds {
     int32_t src[M + NN];                       // stencil index of each position
 };
 
+// Stencil e (n rows) to the list of what the rook-pivoted kernels solve: the launch's own, or
+// in a ragged launch its size bucket's.
+template <bool RAG>
+__device__ __forceinline__ void nse_hand_back(const BuildDev& P, bool yes, int64_t e, int n)
+{
+    if (!yes || !P.fail_list) return;
+    const int b = !RAG ? 0 : (n <= 32 ? 0 : (n <= 64 ? 1 : 2));
+    const int q = atomicAdd(P.fail_count + b, 1);
+    P.fail_list[b * P.fail_stride + q] = (int32_t)e;
+}
+
 // position of the monomial x_i x_j in the graded order (fill_mono_table)
 template <int DIM>
 __device__ __forceinline__ int nse_pair(int i, int j)
@@ -188,8 +199,10 @@ __device__ __forceinline__ int nse_pair(int i, int j)
 // KIND PHS3, PHS5 or PHS7 (a compile-time constant: with a switch around the loops the
 // compiler hoists the square roots common to its cases and holds all of them); DIM 2 or
 // 3; M monomials; up to NN null points (k - M); up to RC operator columns; W
-// waves per SIMD the register allocation targets
-template <int KIND, int DIM, int M, int NN, int RC, int W>
+// waves per SIMD the register allocation targets; RAG: the stencils of a wavefront differ in
+// k (loops run to the longest of the four; a step past a stencil's own points multiplies
+// its rows by zero)
+template <int KIND, int DIM, int M, int NN, int RC, int W, bool RAG>
 __global__ __attribute__((amdgpu_flat_work_group_size(64, 64), amdgpu_waves_per_eu(W))) void
 k_nse(const BuildDev P)
 {
@@ -215,12 +228,29 @@ k_nse(const BuildDev P)
         alive = 0;
         e = 0;
     }
-    // Uniform builds only (the host checks k - M <= NN and the column count): kk and nn are
-    // scalars. A group without work repeats stencil 0 and writes nothing.
-    const int kk = P.k;
-    const int nn = kk - M;
+    // Uniform builds (the host checks k - M <= NN and the column count): kk and nn are
+    // scalars. A group without work repeats stencil 0 and writes nothing. Ragged ones: kk
+    // and nn are the group's; a stencil outside the class is handed back.
+    int kk = P.k, nn = kk - M, nnw = nn;
+    int64_t s0 = e * (int64_t)kk;
+    int rag_ok = 1;
+    if constexpr (RAG) {
+        if (P.adj_ptr) {
+            s0 = P.adj_ptr[e];
+            kk = (int)(P.adj_ptr[e + 1] - s0);
+        }
+        rag_ok = stencil_n_mono(P, e, DIM) == M && kk > M && kk - M <= NN;
+        nn = rag_ok ? kk - M : 1;
+        nnw = max(max(__builtin_amdgcn_readlane(nn, 0), __builtin_amdgcn_readlane(nn, 16)),
+                  max(__builtin_amdgcn_readlane(nn, 32), __builtin_amdgcn_readlane(nn, 48)));
+    }
+    const int kp = M + nn;  // points of the arithmetic
     const int n_cols = P.n_cols, n_terms = P.n_terms;
     int handoff = 0, fail = 0;
+    if (RAG && alive && !rag_ok) {
+        handoff = 1;
+        alive = 0;
+    }
 
     // ---- points li + 16 s: offsets from the evaluation point
     double x[SLP][DIM], hinv;
@@ -234,8 +264,8 @@ k_nse(const BuildDev P)
 #pragma unroll
         for (int s = 0; s < SLP; ++s) {
             const int q = li + 16 * s;
-            isp[s] = q < kk;
-            const int32_t idx = P.adj_idx[e * (int64_t)kk + (q < kk ? q : 0)];
+            isp[s] = q < kp;
+            const int32_t idx = rag_ok ? P.adj_idx[s0 + (q < kp ? q : 0)] : 0;
             double r2 = 0.0;
 #pragma unroll
             for (int d = 0; d < DIM; ++d) {
@@ -249,9 +279,13 @@ k_nse(const BuildDev P)
         // each group reads its own 16 bits)
         if (P.is_boundary) {
             if (((__ballot(ib) >> (16 * g)) & 0xffffull) != 0ull) {
-                handoff = alive;
+                handoff = handoff | alive;
                 alive = 0;
             }
+        }
+        if (RAG && __ballot(alive) == 0ull) {  // (a wavefront of hand-backs or padding)
+            nse_hand_back<RAG>(P, handoff && li == 0, e, kk + M);
+            return;
         }
         // scaled by a power of two, so the scaling rounds nothing (|x| < 1; a PHS build's
         // weights do not depend on the scale)
@@ -616,7 +650,7 @@ k_nse(const BuildDev P)
 #undef RBFX_NSE_POINT
     nse_for<(NN + 7) / 8>([&](auto ch) RBFX_INL {
         constexpr int j0 = 8 * ch.value, cnt = NN - j0 < 8 ? NN - j0 : 8, jt = j0 / 16, jl = j0 % 16;
-        if (j0 < nn) {
+        if (j0 < nnw) {
             if constexpr (!CREG) asm volatile("" ::: "memory");  // (reread, not kept from the last chunk)
 #pragma unroll
             for (int a = 0; a < M; ++a) {
@@ -655,13 +689,15 @@ k_nse(const BuildDev P)
         double dmax = 0.0;
         nse_for<NN>([&](auto jc) RBFX_INL {
             constexpr int j = jc.value, jt = j / 16, jl = j % 16, rest = NN - 1 - j;
-            if (j < nn) {
+            if (j < nnw) {
                 const double piv = nse_bc<jl>(sn[jt][j]);
                 const double ap = sg * piv;
-                dmax = fmax(dmax, ap);
-                if (!(ap > kNsePivTol * dmax)) fail = 1;
+                const bool has = !RAG || j < nn;
+                dmax = has ? fmax(dmax, ap) : dmax;
+                if (has && !(ap > kNsePivTol * dmax)) fail = 1;
                 asm volatile("" : "+v"(fail));
-                const double rd = nsc_rcp(piv);
+                double rd = nsc_rcp(piv);
+                if constexpr (RAG) rd = has ? rd : 0.0;
                 const bool own = li == jl;
                 dinv[jt] = own ? rd : dinv[jt];
                 double nl[SLN];
@@ -698,17 +734,18 @@ k_nse(const BuildDev P)
             for (int c = 0; c < RC; ++c) wb[s][c] = -S_.buf[(NN + c) * MP + b];
         }
         nse_for<NN>([&](auto i) RBFX_INL {
-            if (i.value < nn) {
+            if (i.value < nnw) {
 #pragma unroll
                 for (int s = 0; s < SLB; ++s) {
                     const int b = li + 16 * s < M ? li + 16 * s : M - 1;
-                    const double cv = S_.buf[i.value * MP + b];
+                    double cv = S_.buf[i.value * MP + b];
+                    if constexpr (RAG) cv = i.value < nn ? cv : 0.0;
                     nse_fmac_row<i.value % 16, RC>(wb[s], u[i.value / 16], cv);
                 }
             }
         });
         if (alive && !fail) {
-            const int64_t o0 = P.out_ptr ? P.out_ptr[e] : e * (int64_t)kk;
+            const int64_t o0 = P.out_ptr ? P.out_ptr[e] : s0;
 #pragma unroll
             for (int t = 0; t < SLN; ++t)
                 if (li + 16 * t < nn) {
@@ -724,23 +761,20 @@ k_nse(const BuildDev P)
                         if (c < n_cols) P.out_val[(int64_t)c * P.out_nnz + o0 + qb[s]] = wb[s][c];
                 }
             if (P.out_col)
-                for (int q = li; q < kk; q += 16) P.out_col[o0 + q] = P.adj_idx[e * (int64_t)kk + q];
+                for (int q = li; q < kp; q += 16) P.out_col[o0 + q] = P.adj_idx[s0 + q];
             if (li == 0 && P.status) P.status[e] = P.ok_status;
         }
     }
-    if ((handoff || (alive && fail)) && li == 0 && P.fail_list) {
-        const int q = atomicAdd(P.fail_count, 1);
-        P.fail_list[q] = (int32_t)e;
-    }
+    nse_hand_back<RAG>(P, (handoff || (alive && fail)) && li == 0, e, kk + M);
 }
 
-template <int KIND, int DIM, int M, int NN, int RC, int W>
+template <int KIND, int DIM, int M, int NN, int RC, int W, bool RAG = false>
 inline hipError_t launch_nse_one(const BuildDev& P, int64_t n_work, hipStream_t s)
 {
     if (n_work <= 0) return hipSuccess;
     BuildDev Q = P;
     Q.n_blocks = (n_work + 3) / 4;
-    hipLaunchKernelGGL((k_nse<KIND, DIM, M, NN, RC, W>), dim3((unsigned)pad_to_xcds(Q.n_blocks)), dim3(64), 0, s, Q);
+    hipLaunchKernelGGL((k_nse<KIND, DIM, M, NN, RC, W, RAG>), dim3((unsigned)pad_to_xcds(Q.n_blocks)), dim3(64), 0, s, Q);
     return hipGetLastError();
 }
 
@@ -780,6 +814,34 @@ inline hipError_t launch_nse_rc(const BuildDev& P, int64_t n_work, hipStream_t s
         if (P.n_cols <= 3) return launch_nse_m<KIND, DIM, M, 3>(P, n_work, s);
         if (P.n_cols == 4) return launch_nse_m<KIND, DIM, M, 4>(P, n_work, s);
         if (P.n_cols <= 6) return launch_nse_m<KIND, DIM, M, 6>(P, n_work, s);
+    }
+    return hipErrorInvalidValue;
+}
+
+// Ragged launches: the two classes of one and two slots (nse_classes).
+template <int KIND, int DIM, int M, int RC>
+inline hipError_t launch_nse_class_m(const BuildDev& P, int hi, int64_t n_work, hipStream_t s)
+{
+    if constexpr (M == 20) {
+        if (hi <= 20) return launch_nse_one<KIND, DIM, M, 20, RC, 2, true>(P, n_work, s);
+        return launch_nse_one<KIND, DIM, M, 26, RC, RC <= 1 ? 2 : 1, true>(P, n_work, s);
+    } else {
+        if (hi <= 16 - RC) return launch_nse_one<KIND, DIM, M, 16 - RC, RC, M <= 6 ? 4 : 3, true>(P, n_work, s);
+        return launch_nse_one<KIND, DIM, M, 26, RC, 2, true>(P, n_work, s);
+    }
+}
+
+template <int KIND, int DIM, int M>
+inline hipError_t launch_nse_class_rc(const BuildDev& P, int hi, int64_t n_work, hipStream_t s)
+{
+    if (P.n_cols == 1) return launch_nse_class_m<KIND, DIM, M, 1>(P, hi, n_work, s);
+    if constexpr (DIM == 2) {
+        if (P.n_cols == 2) return launch_nse_class_m<KIND, DIM, M, 2>(P, hi, n_work, s);
+        if (P.n_cols == 3) return launch_nse_class_m<KIND, DIM, M, 3>(P, hi, n_work, s);
+    } else {
+        if (P.n_cols <= 3) return launch_nse_class_m<KIND, DIM, M, 3>(P, hi, n_work, s);
+        if (P.n_cols == 4) return launch_nse_class_m<KIND, DIM, M, 4>(P, hi, n_work, s);
+        if (P.n_cols <= 6) return launch_nse_class_m<KIND, DIM, M, 6>(P, hi, n_work, s);
     }
     return hipErrorInvalidValue;
 }

@@ -1,0 +1,14 @@
+// Instantiates the null-space build by elimination for uneven builds in 2-D.
+#include "build_nse_kernel.h"
+
+namespace rbfx {
+
+hipError_t launch_nse_rag_2d(const BuildDev& P, int m, int hi, int64_t n_work, hipStream_t s)
+{
+    if (m == 6 && P.basis_kind == RBFX_PHS3) return launch_nse_class_rc<RBFX_PHS3, 2, 6>(P, hi, n_work, s);
+    if (m == 10 && P.basis_kind == RBFX_PHS3) return launch_nse_class_rc<RBFX_PHS3, 2, 10>(P, hi, n_work, s);
+    if (m == 10 && P.basis_kind == RBFX_PHS5) return launch_nse_class_rc<RBFX_PHS5, 2, 10>(P, hi, n_work, s);
+    return hipErrorInvalidValue;
+}
+
+}  // namespace rbfx

@@ -119,3 +119,56 @@ def test_nse_repeated_builds_bit_identical(RBF, gpu):
             torch.cuda.synchronize()
             assert torch.equal(op.vals, first)
         assert torch.equal(y, g.replay())
+
+
+@pytest.mark.parametrize("kind,dim,degs,cols,kmax", [(3, 2, (1, 3), "lap", 40), (3, 2, (2, 2), "hess", 36),
+                                                    (5, 2, (2, 3), "grad", 40), (3, 3, (2, 2), "gradlap", 40),
+                                                    (5, 3, (3, 3), "lap", 50)])
+def test_nse_classes_of_uneven_builds(RBF, O, gpu, kind, dim, degs, cols, kmax):
+    """Ragged stencils of mixed degree: those within a class run on the elimination kernel
+    (null points from 1 to 26, a wavefront's four stencils of different k), the others on the
+    rook kernels; every stencil against the extended-precision oracle at max(1e-10, kappa u),
+    and a captured replay gives the eager build's bits."""
+    import torch
+
+    rng = np.random.default_rng(kind + dim + kmax)
+    n = 1501
+    pts = rng.random((n, dim))
+    L, n_cols, terms = _operator(RBF, O, dim, cols)
+    full = O.knn(pts, pts, kmax)
+    deg = rng.integers(degs[0], degs[1] + 1, n).astype(np.int8)
+    mono = np.array([comb(dim + d, dim) for d in deg])
+    ks = np.maximum(rng.integers(mono + 1, kmax + 1), 2)
+    edges = [1, 12, 13, 14, 15, 16, 20, 21, 26, 27]
+    for i in range(300):  # the edges of the classes, each several times
+        ks[i] = min(kmax, mono[i] + edges[i % len(edges)])
+    adjl = [full[i, :ks[i]] for i in range(n)]
+    op = RBF.RadialBasisOperator(L, pts, basis=RBF.PHS(kind, poly_deg=int(degs[1])), adjl=adjl, poly_deg_map=deg)
+    nb, kern = RBF._lib.last_build_buckets()
+    nn = ks + mono
+    assert nb == [int((nn <= 32).sum()), int(((nn > 32) & (nn <= 64)).sum()), int((nn > 64).sum())]
+    w = op.vals.cpu().numpy()
+    ptr = op.row_ptr.cpu().numpy()
+    u = 2.0 ** -53
+    for d in range(degs[0], degs[1] + 1):
+        sel = np.flatnonzero(deg == d)
+        if not len(sel):
+            continue
+        aptr = np.concatenate([[0], np.cumsum(ks[sel])])
+        adj = (aptr, np.concatenate([adjl[i] for i in sel]))
+        b, o = O.basis_struct(kind, d), _op(O, n_cols, terms)
+        _, _, wr, _, rc = O.build(pts, pts[sel], adj, b, o, scaled=True, long_double=True)
+        assert rc == 0
+        kap = O.condition_numbers(pts, pts[sel], adj, b, o)
+        for j, i in enumerate(sel):
+            g, r = w[:, ptr[i]:ptr[i + 1]], wr[:, aptr[j]:aptr[j + 1]]
+            err = (np.abs(g - r).max(1) / np.abs(r).max(1)).max()
+            assert err <= max(1e-10, kap[j] * u), (d, ks[i], err, kap[j] * u)
+    f = torch.as_tensor(np.sin(3 * pts[:, 0]), device=gpu)
+    eager = op.vals.clone()
+    g = op.capture(f)
+    for _ in range(3):
+        op.vals.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(op.vals, eager)
