@@ -629,6 +629,20 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_wid
 // zero fill, and which the first steps freeze (every step freezes the top active
 // positions): the second update pass is skipped from then on.
 //
+// Bound by VALU issue (88% of the cycles on the 8M-stencil 3-D regrid of 34 rows, 4,937
+// instructions a stencil), so everything is arranged to take fewer of them, each entry's
+// arithmetic unchanged (the weights are the same bits):
+//   - without boundary points each pair of points is evaluated once (8 evaluations a lane
+//     for 30 points, not 30), and the basis kind is a constant around both loops;
+//   - the update reads eight entries of the pivot row at once, one per lane, and the FMAs
+//     broadcast them (DPP), where eight LDS broadcasts had taken a third of the LDS cycles;
+//   - up to 32 active rows both halves of the wavefront share the rows;
+//   - uniform work (the search's masks and maxima, where a row starts, 2x2 flags) is scalar;
+//   - the back substitution takes the reciprocals of all diagonal entries in one division.
+// 147.5 -> 83.5 ms there; 33..64 and 65..70 rows of a disk with boundary points
+// (92,000 stencils) 18.9 -> 14.2 ms. LDS is allocated in steps of 1,280 bytes: 6,344 bytes (34 rows) hold
+// 25 wavefronts on a CU, 6,408 had held 21 (91.6 ms).
+//
 // Row starts: row j holds positions 0..j padded to a multiple of eight (the update's
 // eight-column chunks stay inside the row), plus the fewest entries (0..31) that put the
 // starts of each 16 consecutive rows in 16 different 8-byte bank pairs modulo 16 and of
@@ -680,6 +694,62 @@ constexpr bool sym_rows_spread()
 }
 static_assert(sym_rows_spread(), "row starts spread over the LDS banks");
 
+// v where the lane's bit of a (uniform) mask is set, else 0
+__device__ __forceinline__ uint32_t lanes_in(unsigned long long mask, uint32_t v)
+{
+    uint32_t r;
+    asm("v_cndmask_b32_e64 %0, 0, %1, %2" : "=v"(r) : "v"(v), "s"(mask));
+    return r;
+}
+
+// max on the scalar unit (the compiler takes max3 of the vector one for three operands)
+__device__ __forceinline__ uint32_t smax_u32(uint32_t a, uint32_t b)
+{
+    uint32_t r;
+    asm("s_max_u32 %0, %1, %2" : "=s"(r) : "s"(a), "s"(b) : "scc");
+    return r;
+}
+
+// the largest key of the first `lanes` lanes (uniform; the others hold 0)
+__device__ __forceinline__ uint32_t first_max_u32(uint32_t k, int lanes)
+{
+    k = max(k, (uint32_t)dpp_i<0x121>((int)k));
+    k = max(k, (uint32_t)dpp_i<0x122>((int)k));
+    k = max(k, (uint32_t)dpp_i<0x124>((int)k));
+    k = max(k, (uint32_t)dpp_i<0x128>((int)k));
+    uint32_t m = smax_u32((uint32_t)rdlane((int)k, 0), (uint32_t)rdlane((int)k, 16));
+    if (lanes > 32) m = smax_u32(m, smax_u32((uint32_t)rdlane((int)k, 32), (uint32_t)rdlane((int)k, 48)));
+    return m;
+}
+
+// lane l (uniform) of v set to x (uniform)
+__device__ __forceinline__ int wrlane(int v, int x, int l)
+{
+    asm("s_mov_b32 m0, %2\n\tv_writelane_b32 %0, %1, m0" : "+v"(v) : "s"(x), "s"(l) : "m0");
+    return v;
+}
+__device__ __forceinline__ double wrlane(double v, double x, int l)
+{
+    const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    const unsigned long long w = (unsigned long long)__double_as_longlong(x);
+    const unsigned lo = (unsigned)wrlane((int)(unsigned)u, (int)(unsigned)w, l);
+    const unsigned hi = (unsigned)wrlane((int)(unsigned)(u >> 32), (int)(unsigned)(w >> 32), l);
+    return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+
+// a[q] += m * (w of lane q of the row of 16 lanes), q < 8: the broadcast is the FMA's own
+// DPP operand. All lanes are active wherever this runs; the wait states cover a write of w
+// by the instruction before the block.
+__device__ __forceinline__ void fma8_row(double (&a)[8], double w, double m)
+{
+#define RBFX_F8(D, Q) "v_fmac_f64_dpp %" D ", %8, %9 row_newbcast:" Q " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" RBFX_F8("0", "0") RBFX_F8("1", "1") RBFX_F8("2", "2") RBFX_F8("3", "3") RBFX_F8("4", "4")
+            RBFX_F8("5", "5") RBFX_F8("6", "6") RBFX_F8("7", "7")
+        : "+v"(a[0]), "+v"(a[1]), "+v"(a[2]), "+v"(a[3]), "+v"(a[4]), "+v"(a[5]), "+v"(a[6]), "+v"(a[7])
+        : "v"(w), "v"(m));
+#undef RBFX_F8
+}
+
 // HERM: the build may carry boundary data. Launches without any (P.is_boundary null)
 // whose LDS is small enough use the instantiation without the Hermite paths, whose
 // smaller register allocation leaves room for more wavefronts per SIMD
@@ -693,9 +763,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
     // the stencil points and their boundary data stay in the registers of the lanes that
     // own them and are read by the others with lane reads
     extern __shared__ __attribute__((aligned(16))) double s_T[];
-    // (the static LDS counts toward the wavefronts per CU: the block list is bytes, and
-    // the monomial exponents and operator terms are read from the kernel arguments)
-    __shared__ int8_t s_blk[ROWS];
+    // (no static LDS, which would count toward the wavefronts per CU: the monomial exponents
+    // and operator terms are read from the kernel arguments)
 
     const int L = threadIdx.x;
     const int n_cols = P.n_cols, n_terms = P.n_terms;
@@ -850,9 +919,11 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
 #pragma unroll
     for (int t = 0; t < TWO; ++t) {
         const int j = L + 64 * t;
-        rbj[t] = kSymRb.rb[j];
-        orig[t] = j < kk ? M + j : j - kk;
+        rbj[t] = kSymRb.rb[j] * 8;
+        orig[t] = j < kk ? M + j : (j < n ? j - kk : 255);
     }
+    // an entry by its byte offset (row starts are kept in bytes: no shifts on the way)
+    auto T = [&](int off) -> double& { return *(double*)((char*)s_T + off); };
     // start of row c (c uniform): from the lane that owns position c
     auto rb_of = [&](int c) -> int {
         const int cc = __builtin_amdgcn_readfirstlane(c);
@@ -861,134 +932,165 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
 
     // ---- assembly (FP64) of the lower triangle and the right-hand sides (registers: lane
     // L holds those of its positions)
-    double bcol[TWO][RC];
+    double bcol[RC][TWO];
 #pragma unroll
-    for (int t = 0; t < TWO; ++t) {
+    for (int t = 0; t < TWO; ++t)
 #pragma unroll
-        for (int c = 0; c < RC; ++c) bcol[t][c] = 0.0;
-        const int j = L + 64 * t;
-        if (j >= n) continue;
-        double* Tj = s_T + rbj[t];
-        const bool is_poly = j >= kk;
-        if (is_poly) {
-            // monomial row a = j - kk: its entries at the monomial positions kk..j are zero
-            // (its point entries are written by the point lanes below)
-            for (int c = kk; c <= j; ++c) Tj[c] = 0.0;
+        for (int c = 0; c < RC; ++c) bcol[c][t] = 0.0;
+    // Without boundary points phi is symmetric, so each pair is computed once: the lane of
+    // point j takes the points j + d (mod k) for d = 0..k/2, up to 32 points on both halves of
+    // the wavefront, even and odd d (30 points: 8 evaluations a lane instead of 30)
+    const bool around = !hermite && kk <= 64;
+    auto point_pairs = [&](auto KC) __attribute__((always_inline)) {
+        const int two = kk <= 32 ? 1 : 0, step = 1 + two;
+        const int j = two ? L & 31 : L;
+        double xj[DIM];
+#pragma unroll
+        for (int d = 0; d < DIM; ++d) xj[d] = __shfl(xo[0][d], j, 64);
+        const int rb_own = __shfl(rbj[0], j, 64);
+        int d = two ? L >> 5 : 0, jj = j + d;
+        if (jj >= kk) jj -= kk;
+        for (int d0 = 0; d0 <= kk / 2; d0 += step) {
+            double q2 = 0.0;
+#pragma unroll
+            for (int x = 0; x < DIM; ++x) {
+                const double t_ = xj[x] - __shfl(xo[0][x], jj, 64);
+                q2 += t_ * t_;
+            }
+            const int rb_other = __shfl(rbj[0], jj, 64);
+            const double v = phi_r2_k<decltype(KC)::value>(B.eps, q2);
+            if (j < kk && d <= kk / 2) T(jj > j ? rb_other + 8 * j : rb_own + 8 * jj) = v;
+            d += step;
+            jj += step;
+            if (jj >= kk) jj -= kk;
         }
-        double xi[DIM], bn[DIM];
-        int bt = 0;
-        double ba = 0.0, bb = 0.0;
-        if (!is_poly) {
+    };
+    // With boundary points (or more than 64): row j's entries one after another. The lane
+    // reads stand outside the branches: a lane that a branch leaves out need not hold its
+    // registers inside it.
+    auto point_rows = [&](auto KC) __attribute__((always_inline)) {
 #pragma unroll
-            for (int d = 0; d < DIM; ++d) {
-                xi[d] = xo[t][d];
-                bn[d] = bno[t][d];
-            }
-            if (hermite) {
-                bt = bto[t];
-                ba = bao[t];
-                bb = bbo[t];
-            }
-            // the point's monomial values: column j of monomial row a (position kk + a)
-            for (int a = 0; a < M; ++a) {
-                int ea[3];
-                mono_exps(a, ea);
-                double v = mono_op<DIM>(ea, RBFX_OP_VALUE, 0, 0, xi);
-                if (hermite && bt == 2) v = ba * v + bb * mono_normal<DIM>(ea, bn, xi);
-                s_T[rb_of(kk + a) + j] = v;
-            }
-        }
-        // phi between point j and the points jj <= j (positions jj): instantiated once per
-        // basis kind; without boundary data four independent entries per iteration
-        auto point_cols = [&](auto KC) __attribute__((always_inline)) {
-            if (is_poly) return;
-            if (!hermite) {
-#pragma unroll 4
-                for (int jj = 0; jj < kk; ++jj) {
-                    double q2 = 0.0;
+        for (int t = 0; t < TWO; ++t) {
+            const int j = L + 64 * t;
+            for (int jj = 0; jj < kk; ++jj) {
+                double xj[DIM], nj[DIM];
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) {
-                        const double t_ = xi[d] - px(jj, d);
-                        q2 += t_ * t_;
-                    }
-                    const double v = phi_r2_k<decltype(KC)::value>(B.eps, q2);
-                    if (jj <= j) Tj[jj] = v;
+                for (int d = 0; d < DIM; ++d) {
+                    xj[d] = px(jj, d);
+                    nj[d] = HERM ? pbn(jj, d) : 0.0;
                 }
-                return;
-            }
-            for (int jj = 0; jj <= j; ++jj) {
-                double xj[DIM];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) xj[d] = px(jj, d);
-                const int tj = pbt(jj);
+                const int tj = HERM ? pbt(jj) : 0;
+                const double aj = HERM ? pba(jj) : 0.0, bj = HERM ? pbb(jj) : 0.0;
+                if (j >= kk || jj > j) continue;
                 double Dj[DIM], q2 = 0.0;
 #pragma unroll
                 for (int d = 0; d < DIM; ++d) {
-                    Dj[d] = xi[d] - xj[d];
+                    Dj[d] = xo[t][d] - xj[d];
                     q2 += Dj[d] * Dj[d];
                 }
                 double v = phi_r2_k<decltype(KC)::value>(B.eps, q2);
-                if (bt == 2 || tj == 2) {
-                    double nj[DIM];
-#pragma unroll
-                    for (int d = 0; d < DIM; ++d) nj[d] = pbn(jj, d);
+                if (HERM && (bto[t] == 2 || tj == 2)) {
+                    const double ba = bao[t], bb = bbo[t];
                     double Di, Djn, D2;
-                    phi_grad_hess_dirs<DIM>(B, Dj, q2, bn, nj, Di, Djn, D2);
-                    const double aj = pba(jj), bj = pbb(jj);
-                    if (bt != 2) v = aj * v - bj * Djn;
+                    phi_grad_hess_dirs<DIM>(B, Dj, q2, bno[t], nj, Di, Djn, D2);
+                    if (bto[t] != 2) v = aj * v - bj * Djn;
                     else if (tj != 2) v = ba * v + bb * Di;
                     else v = ba * aj * v - ba * bj * Djn + bb * aj * Di + bb * bj * D2;
                 }
-                Tj[jj] = v;
+                T(rbj[t] + 8 * jj) = v;
             }
-        };
-        switch (B.kind) {
-        case RBFX_PHS1: point_cols(std::integral_constant<int, RBFX_PHS1>{}); break;
-        case RBFX_PHS3: point_cols(std::integral_constant<int, RBFX_PHS3>{}); break;
-        case RBFX_PHS5: point_cols(std::integral_constant<int, RBFX_PHS5>{}); break;
-        case RBFX_PHS7: point_cols(std::integral_constant<int, RBFX_PHS7>{}); break;
-        case RBFX_IMQ: point_cols(std::integral_constant<int, RBFX_IMQ>{}); break;
-        default: point_cols(std::integral_constant<int, RBFX_GAUSSIAN>{}); break;
         }
-        // right-hand sides (kept in registers until the whole assembly is done)
-        if (!is_poly) {
+    };
+    // right-hand sides of the point rows
+    auto point_rhs = [&](auto KC) __attribute__((always_inline)) {
+        BasisDev Bk;
+        Bk.kind = decltype(KC)::value;
+        Bk.eps = B.eps;
+#pragma unroll
+        for (int t = 0; t < TWO; ++t) {
+            if (L + 64 * t >= kk) continue;
             double De[DIM], q2 = 0.0;
 #pragma unroll
             for (int d = 0; d < DIM; ++d) {
-                De[d] = -xi[d];
+                De[d] = -xo[t][d];
                 q2 += De[d] * De[d];
             }
             for (int tt = 0; tt < n_terms; ++tt) {
                 const TermDev tm = P.terms[tt];
-                double v = phi_term<DIM>(B, tm.kind, tm.d1, tm.d2, De, q2);
-                if (hermite && bt == 2) v = ba * v + bb * phi_term_normal<DIM>(B, tm.kind, tm.d1, De, q2, bn);
+                // (or the roots and quotients of every term kind move out of the loop)
+                double q2t = q2;
+                asm volatile("" : "+v"(q2t));
+                double v = phi_term<DIM>(Bk, tm.kind, tm.d1, tm.d2, De, q2t);
+                if (hermite && bto[t] == 2)
+                    v = bao[t] * v + bbo[t] * phi_term_normal<DIM>(Bk, tm.kind, tm.d1, De, q2t, bno[t]);
                 const double sc = term_scale(tm, hinv);
 #pragma unroll
                 for (int c = 0; c < RC; ++c)
-                    if (tm.col == c) bcol[t][c] += sc * v;
+                    bcol[c][t] = tm.col == c ? bcol[c][t] + sc * v : bcol[c][t];
+            }
+        }
+    };
+    auto point_block = [&](auto KC) __attribute__((always_inline)) {
+        if (around) point_pairs(KC);
+        else point_rows(KC);
+        point_rhs(KC);
+    };
+    switch (B.kind) {
+    case RBFX_PHS1: point_block(std::integral_constant<int, RBFX_PHS1>{}); break;
+    case RBFX_PHS3: point_block(std::integral_constant<int, RBFX_PHS3>{}); break;
+    case RBFX_PHS5: point_block(std::integral_constant<int, RBFX_PHS5>{}); break;
+    case RBFX_PHS7: point_block(std::integral_constant<int, RBFX_PHS7>{}); break;
+    case RBFX_IMQ: point_block(std::integral_constant<int, RBFX_IMQ>{}); break;
+    default: point_block(std::integral_constant<int, RBFX_GAUSSIAN>{}); break;
+    }
+    // the eval node's boundary condition (stencils with boundary points)
+    const bool eval_normal = hermite && pbt(eval_local) == 2;
+    const double eav = HERM ? pba(eval_local) : 0.0, ebv = HERM ? pbb(eval_local) : 0.0;
+    double en[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) en[d] = HERM ? pbn(eval_local, d) : 0.0;
+#pragma unroll
+    for (int t = 0; t < TWO; ++t) {
+        const int j = L + 64 * t;
+        if (j >= n) continue;
+        const bool is_poly = j >= kk;
+        if (!is_poly) {
+            // the point's monomial values: column j of monomial row a (position kk + a)
+            for (int a = 0; a < M; ++a) {
+                int ea[3];
+                mono_exps(a, ea);
+                double v = 1.0;
+#pragma unroll
+                for (int d = 0; d < DIM; ++d) {
+                    double w = 1.0;
+#pragma unroll 1
+                    for (int q = 0; q < ea[d]; ++q) w *= xo[t][d];
+                    v *= w;
+                }
+                if (hermite && bto[t] == 2) v = bao[t] * v + bbo[t] * mono_normal<DIM>(ea, bno[t], xo[t]);
+                s_T[kSymRb.rb[kk + a] + j] = v;
             }
         } else {
+            // monomial row a = j - kk: zero at the monomial positions kk..j, and its right-hand
+            // sides
+            for (int c = kk; c <= j; ++c) T(rbj[t] + 8 * c) = 0.0;
             double z[DIM];
 #pragma unroll
             for (int d = 0; d < DIM; ++d) z[d] = 0.0;
             int ea[3];
             mono_exps(j - kk, ea);
-            if (hermite && pbt(eval_local) == 2) {
+            if (eval_normal) {
                 // the eval node's boundary operator applied to P (assembly.jl:452-467)
-                const double eav = pba(eval_local), ebv = pbb(eval_local);
-                double en[DIM];
-#pragma unroll
-                for (int d = 0; d < DIM; ++d) en[d] = pbn(eval_local, d);
                 const double v = eav * mono_op<DIM>(ea, RBFX_OP_VALUE, 0, 0, z) + ebv * mono_normal<DIM>(ea, en, z);
 #pragma unroll
-                for (int c = 0; c < RC; ++c) bcol[t][c] = v;
+                for (int c = 0; c < RC; ++c) bcol[c][t] = v;
             } else {
                 for (int tt = 0; tt < n_terms; ++tt) {
                     const TermDev tm = P.terms[tt];
                     const double v = term_scale(tm, hinv) * mono_op<DIM>(ea, tm.kind, tm.d1, tm.d2, z);
 #pragma unroll
                     for (int c = 0; c < RC; ++c)
-                        if (tm.col == c) bcol[t][c] += v;
+                        bcol[c][t] = tm.col == c ? bcol[c][t] + v : bcol[c][t];
                 }
             }
         }
@@ -998,88 +1100,116 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
     // ---- factorisation with rook pivoting and symmetric moves of the pivots
     const double alpha = 0.6403882032022076;  // (1 + sqrt(17)) / 8
     int n_act = n;
-    int slot = 0;
     bool failed = false;
+    auto bits = [&](int count, int t) -> unsigned long long {
+        const int c = count - 64 * t;
+        return c >= 64 ? ~0ull : (c > 0 ? (1ull << c) - 1ull : 0ull);
+    };
+    // the original indices still active, and the positions where a 2x2 pivot starts
+    unsigned long long om[TWO], twos[TWO];
+#pragma unroll
+    for (int t = 0; t < TWO; ++t) {
+        om[t] = bits(n, t);
+        twos[t] = 0ull;
+    }
     // Column c (uniform) of the active block to this lane's registers (v[t] = A(j, c)
     // for its positions j < n_act: row j's entry if c <= j, else row c's entry j), and
-    // the largest |A(j, c)| over active j != excl as a packed (magnitude, position) key.
+    // the largest |A(j, c)| over active j != c as a packed (magnitude, position) key.
     double v[TWO];
-    auto colkey = [&](int c, int excl) -> uint32_t {
+    auto colkey = [&](int c) -> uint32_t {
         const int cc = __builtin_amdgcn_readfirstlane(c);
         const int rbc = rb_of(cc);
         uint32_t k = 0u;
 #pragma unroll
         for (int t = 0; t < TWO; ++t) {
             const int j = L + 64 * t;
-            const bool a_ = j < n_act;
-            v[t] = a_ ? s_T[j >= cc ? rbj[t] + cc : rbc + j] : 0.0;
-            if (a_ && j != excl) k = max(k, row_key(fabs(v[t]), j));
+            if (t && n_act <= 64) break;
+            unsigned long long m = bits(n_act, t);
+            if (TWO == 1 || cc >> 6 == t) m &= ~(1ull << (cc & 63));
+            // (lanes past the active rows read entry (0, cc) or of row cc, and are masked)
+            v[t] = T(j >= cc ? (j < n_act ? rbj[t] : 0) + 8 * cc : rbc + 8 * j);
+            k = max(k, lanes_in(m, row_key(v[t], j) & 0x7fffffffu));
         }
-        return wave_max_u32(k);
+        return first_max_u32(k, n_act);
     };
     auto colval = [&](int r) -> double {
         const int rr = __builtin_amdgcn_readfirstlane(r);
         return (TWO == 2 && rr >= 64) ? rdlane(v[TWO - 1], rr & 63) : rdlane(v[0], rr & 63);
     };
-    // symmetric swap of positions a and b (both active): the rows and the columns, for
+    // symmetric swap of positions lo <= hi (both active): the rows and the columns, for
     // every row of the system (frozen rows keep their entries at the active positions);
-    // each entry of the lower triangle that moves is moved by exactly one lane
-    auto sym_swap = [&](int a, int b) {
-        const int lo = __builtin_amdgcn_readfirstlane(min(a, b)), hi = __builtin_amdgcn_readfirstlane(max(a, b));
-        if (lo == hi) return;
-        const int rlo = rb_of(lo), rhi = rb_of(hi);
+    // each entry of the lower triangle that moves is moved by exactly one lane: lane k
+    // swaps (k, lo) with (k, hi), lane lo the diagonal entries, lane hi nothing
+    auto swap_entries = [&](int lo, int hi, int rhi) {
+        const int rlo = rb_of(lo);
 #pragma unroll
         for (int t = 0; t < TWO; ++t) {
             const int k = L + 64 * t;
             if (k >= n || k == hi) continue;
-            int x0, x1;
-            if (k < lo) {
-                x0 = rlo + k;  // (lo, k) <-> (hi, k)
-                x1 = rhi + k;
-            } else if (k == lo) {
-                x0 = rlo + lo;  // the diagonal entries
-                x1 = rhi + hi;
-            } else if (k < hi) {
-                x0 = rbj[t] + lo;  // (k, lo) <-> (hi, k)
-                x1 = rhi + k;
-            } else {
-                x0 = rbj[t] + lo;  // (k, lo) <-> (k, hi)
-                x1 = rbj[t] + hi;
-            }
-            const double y0 = s_T[x0], y1 = s_T[x1];
-            s_T[x0] = y1;
-            s_T[x1] = y0;
-        }
-#pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            const double ylo = (TWO == 2 && lo >= 64) ? rdlane(bcol[TWO - 1][c], lo & 63) : rdlane(bcol[0][c], lo & 63);
-            const double yhi = (TWO == 2 && hi >= 64) ? rdlane(bcol[TWO - 1][c], hi & 63) : rdlane(bcol[0][c], hi & 63);
-#pragma unroll
-            for (int t = 0; t < TWO; ++t) {
-                const int k = L + 64 * t;
-                if (k == lo) bcol[t][c] = yhi;
-                else if (k == hi) bcol[t][c] = ylo;
-            }
-        }
-        const int olo = (TWO == 2 && lo >= 64) ? rdlane(orig[TWO - 1], lo & 63) : rdlane(orig[0], lo & 63);
-        const int ohi = (TWO == 2 && hi >= 64) ? rdlane(orig[TWO - 1], hi & 63) : rdlane(orig[0], hi & 63);
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int k = L + 64 * t;
-            if (k == lo) orig[t] = ohi;
-            else if (k == hi) orig[t] = olo;
+            const int k8 = 8 * k;
+            const int x0 = k >= lo ? rbj[t] + 8 * lo : rlo + k8;
+            const int x1 = k > hi ? rbj[t] + 8 * hi : rhi + (k == lo ? 8 * hi : k8);
+            const double y0 = T(x0), y1 = T(x1);
+            T(x0) = y1;
+            T(x1) = y0;
         }
     };
+    auto lane_put = [&](auto& w, auto v_, int p) __attribute__((always_inline)) {
+        if constexpr (TWO == 2) {
+            const auto w0 = w[0], w1 = w[1];  // (by value: a choice of elements would go to memory)
+            w[0] = p < 64 ? wrlane(w0, v_, p & 63) : w0;
+            w[1] = p < 64 ? w1 : wrlane(w1, v_, p & 63);
+        } else {
+            w[0] = wrlane(w[0], v_, p);
+        }
+    };
+    auto lane_get = [&](const auto& w, int p) __attribute__((always_inline)) {
+        const auto w0 = w[0], w1 = w[TWO - 1];
+        const auto a0 = rdlane(w0, p & 63);
+        if constexpr (TWO == 2) return p < 64 ? a0 : rdlane(w1, p & 63);
+        else return a0;
+    };
+    // The pivot of position p goes to the last active position q: its row start rq is
+    // returned, its right-hand sides in vq.
+    auto freeze = [&](int p, int q, double(&vq)[RC]) __attribute__((always_inline)) -> int {
+        const int rq = rb_of(q), o = lane_get(orig, p);
+        if (TWO == 2 && o >= 64) om[TWO - 1] &= ~(1ull << (o & 63));
+        else om[0] &= ~(1ull << (o & 63));
+#pragma unroll
+        for (int c = 0; c < RC; ++c) vq[c] = lane_get(bcol[c], p);
+        if (p != q) {
+            swap_entries(p, q, rq);
+            lane_put(orig, lane_get(orig, q), p);
+            lane_put(orig, o, q);
+#pragma unroll
+            for (int c = 0; c < RC; ++c) {
+                lane_put(bcol[c], lane_get(bcol[c], q), p);
+                lane_put(bcol[c], vq[c], q);
+            }
+        }
+        return rq;
+    };
+    // The trailing update's rows: lane L updates row jr; with up to 32 active rows, both
+    // halves of the wavefront share the rows, the upper half eight columns on.
+    int jr = L, rbu = rbj[0];
+    bool shared = false;
+    const int cadd = (L >> 2) & 8, cadd8 = 8 * cadd, wlane = 8 * (L & 7);
+    auto share_rows = [&]() {
+        jr = L & 31;
+        rbu = __shfl(rbj[0], L & 31, 64);
+        shared = true;
+    };
+    if (n_act <= 32) share_rows();
     while (n_act > 0) {
         // the active row of the lowest original index starts the search
-        uint32_t ko = 0u;
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int j = L + 64 * t;
-            if (j < n_act) ko = max(ko, ((uint32_t)(255 - orig[t]) << 8) | (uint32_t)j);
+        int c0;
+        {
+            const bool first = TWO == 1 || om[0] != 0ull;
+            const int o = first ? __builtin_ctzll(om[0]) : 64 + __builtin_ctzll(om[TWO - 1]);
+            const unsigned long long m0 = __ballot(orig[0] == o), m1 = TWO == 2 ? __ballot(orig[TWO - 1] == o) : 0ull;
+            c0 = (TWO == 1 || m0) ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
         }
-        const int c0 = (int)(wave_max_u32(ko) & 255u);
-        const uint32_t ck = colkey(c0, c0);
+        const uint32_t ck = colkey(c0);
         int imax = ck ? 127 - (int)(ck & 127u) : c0;
         const double akk = colval(c0);
         double colmax = ck ? fabs(colval(imax)) : 0.0;
@@ -1088,12 +1218,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
         // A(p, p), A(kp, kp) and, for a 2x2 pivot, A(p, kp) as the search ends
         double app = akk, akp = akk, apk = akk;
         bool need_rook = absakk < alpha * colmax;
-        if (!(absakk > 0.0 || colmax > 0.0)) {
-            failed = true;  // zero column: singular
+        if (!need_rook && !(absakk > 0.0 || colmax > 0.0)) {
+            failed = true;  // zero column: singular (a search has colmax > 0)
             break;
         }
         for (int it = 0; it < 2 * ROWS && need_rook; ++it) {
-            const uint32_t rk = colkey(imax, imax);
+            const uint32_t rk = colkey(imax);
             const int ri = rk ? 127 - (int)(rk & 127u) : imax;
             const double rowmax = rk ? fabs(colval(ri)) : 0.0;
             const double aim = colval(imax);
@@ -1120,164 +1250,169 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
         const int p1 = __builtin_amdgcn_readfirstlane(kp);  // equals p0 for a 1x1 pivot
         // A(p0, p0), A(p1, p1), A(p0, p1)
         const double d0 = kstep == 1 ? akp : app, d1 = akp, bq = kstep == 1 ? akp : apk;
-        const double det = d0 * d1 - bq * bq;
-        if ((kstep == 1 && d0 == 0.0) || (kstep == 2 && det == 0.0)) {
-            failed = true;
-            break;
+        double idet = 0.0;
+        if (kstep == 1) {
+            failed = d0 == 0.0;
+        } else {
+            const double det = d0 * d1 - bq * bq;
+            failed = det == 0.0;
+            idet = 1.0 / det;
         }
-        const double idet = 1.0 / det;
-        if (L == 0) {
-            s_blk[slot] = (int8_t)kstep;
-            if (kstep == 2) s_blk[slot + 1] = 0;
-        }
+        if (failed) break;
         // p0 to position n_act - 1, p1 (2x2) to n_act - 2
-        sym_swap(p0, n_act - 1);
-        if (kstep == 2) sym_swap(p1 == n_act - 1 ? p0 : p1, n_act - 2);
-        n_act -= kstep;
-        // the pivot rows: p0 at Q0, p1 at Q1 = n_act (2x2)
-        const int Q0 = n_act + kstep - 1;
-        const double* U0 = s_T + rb_of(Q0);
-        const double* U1 = s_T + rb_of(n_act);
-        // the pivot rows' right-hand sides, from their lanes
         double v0[RC], v1[RC];
+        const int q0 = n_act - 1, r0 = freeze(p0, q0, v0);
+        int r1 = r0;
 #pragma unroll
-        for (int c = 0; c < RC; ++c) {
-            v0[c] = (TWO == 2 && Q0 >= 64) ? rdlane(bcol[TWO - 1][c], Q0 & 63) : rdlane(bcol[0][c], Q0 & 63);
-            v1[c] = (TWO == 2 && n_act >= 64) ? rdlane(bcol[TWO - 1][c], n_act & 63) : rdlane(bcol[0][c], n_act & 63);
+        for (int c = 0; c < RC; ++c) v1[c] = 0.0;
+        if (kstep == 2) {
+            r1 = freeze(p1 == q0 ? p0 : p1, q0 - 1, v1);
+            const unsigned long long bit = 1ull << ((q0 - 1) & 63);
+            twos[0] |= TWO == 1 || q0 - 1 < 64 ? bit : 0ull;
+            if (TWO == 2) twos[TWO - 1] |= q0 - 1 < 64 ? 0ull : bit;
         }
-        // The trailing update of the active rows j < n_act over their columns 0..j, eight
-        // at a time (the chunk past the diagonal lands in the row's padding), and of their
-        // right-hand sides; per element the FMAs run in the same order as in k_build_wide.
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int j = L + 64 * t;
-            if (j >= n_act) continue;
-            const double u0 = U0[j];
-            double l0, l1 = 0.0;
-            if (kstep == 1) {
-                l0 = u0 / d0;
-            } else {
-                const double u1 = U1[j];
-                l0 = (u0 * d1 - u1 * bq) * idet;
-                l1 = (u1 * d0 - u0 * bq) * idet;
-            }
-            const double ml0 = -l0, ml1 = -l1;
-            double* Tj = s_T + rbj[t];
-            auto chunk1 = [&](auto W, double* Ar, const double* W0, int j0) __attribute__((always_inline)) {
-                constexpr int CW = decltype(W)::value;
-                double a[CW], w0[CW];
-#pragma unroll
-                for (int q = 0; q < CW; ++q) {
-                    a[q] = Ar[j0 + q];
-                    w0[q] = W0[j0 + q];
+        n_act -= kstep;
+        if (n_act <= 32 && !shared) share_rows();
+        // The trailing update of the active rows j < n_act over their columns 0..j, eight at a
+        // time (the chunk past the diagonal lands in the row's padding), and of their
+        // right-hand sides; per element the FMAs run in the same order as in k_build_wide. The
+        // pivot row's eight entries are one read, spread over the lanes and broadcast by the
+        // FMAs. Every lane reads and multiplies (lanes without a row: row 0), those whose
+        // chunk lies in their row write.
+        const int na = TWO == 2 ? min(n_act, 64) : n_act;
+        const bool on = jr < na;
+        const int row = on ? rbu : 0;
+        auto update = [&](auto KS) __attribute__((always_inline)) {
+            constexpr int K = decltype(KS)::value;
+            auto factors = [&](int j, double& ml0, double& ml1) __attribute__((always_inline)) {
+                const double u0 = T(r0 + 8 * j);
+                double l0, l1 = 0.0;
+                if (K == 1) {
+                    l0 = u0 / d0;
+                } else {
+                    const double u1 = T(r1 + 8 * j);
+                    l0 = (u0 * d1 - u1 * bq) * idet;
+                    l1 = (u1 * d0 - u0 * bq) * idet;
                 }
-#pragma unroll
-                for (int q = 0; q < CW; ++q) Ar[j0 + q] = fma(ml0, w0[q], a[q]);
+                ml0 = -l0;
+                ml1 = -l1;
             };
-            auto chunk2 = [&](auto W, double* Ar, const double* W0, const double* W1, int j0)
-                              __attribute__((always_inline)) {
-                constexpr int CW = decltype(W)::value;
-                double a[CW], w0[CW], w1[CW];
+            double ml0, ml1;
+            factors(jr, ml0, ml1);
+            auto chunk = [&](int A, int W, int cc) __attribute__((always_inline)) {
+                double a[8], w1 = 0.0;
+                const double w0 = T(r0 + W);
+                if (K == 2) w1 = T(r1 + W);
 #pragma unroll
-                for (int q = 0; q < CW; ++q) {
-                    a[q] = Ar[j0 + q];
-                    w0[q] = W0[j0 + q];
-                    w1[q] = W1[j0 + q];
+                for (int q = 0; q < 8; ++q) a[q] = T(A + 8 * q);
+                fma8_row(a, w0, ml0);
+                if (K == 2) fma8_row(a, w1, ml1);
+                if (on && cc <= jr) {
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) T(A + 8 * q) = a[q];
                 }
-#pragma unroll
-                for (int q = 0; q < CW; ++q) Ar[j0 + q] = fma(ml1, w1[q], fma(ml0, w0[q], a[q]));
             };
-            using C8 = std::integral_constant<int, 8>;
-            if (kstep == 1) {
-                for (int j0 = 0; j0 < n_act; j0 += 8)
-                    if (j0 <= j) chunk1(C8{}, Tj, U0, j0);
-#pragma unroll
-                for (int c = 0; c < RC; ++c) bcol[t][c] = fma(ml0, v0[c], bcol[t][c]);
+            if (n_act <= 32) {
+                if (n_act > 0) chunk(row + cadd8, wlane + cadd8, cadd);
+                if (n_act > 16) chunk(row + cadd8 + 128, wlane + cadd8 + 128, cadd + 16);
             } else {
-                for (int j0 = 0; j0 < n_act; j0 += 8)
-                    if (j0 <= j) chunk2(C8{}, Tj, U0, U1, j0);
-#pragma unroll
-                for (int c = 0; c < RC; ++c) bcol[t][c] = fma(ml1, v1[c], fma(ml0, v0[c], bcol[t][c]));
+                for (int cc = 0; cc < na; cc += 8) chunk(row + 8 * cc, wlane + 8 * cc, cc);
             }
-        }
-        slot += kstep;
+#pragma unroll
+            for (int c = 0; c < RC; ++c) {
+                const double b = K == 1 ? fma(ml0, v0[c], bcol[c][0]) : fma(ml1, v1[c], fma(ml0, v0[c], bcol[c][0]));
+                bcol[c][0] = L < na ? b : bcol[c][0];
+            }
+            if constexpr (TWO == 2) {
+                // rows 64.. (the first steps of a system of more than 64 rows)
+                const int j = L + 64;
+                if (j < n_act) {
+                    factors(j, ml0, ml1);
+                    for (int j0 = 0; j0 <= j; j0 += 8) {
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) {
+                            const int o = 8 * (j0 + q);
+                            const double a0 = fma(ml0, T(r0 + o), T(rbj[1] + o));
+                            T(rbj[1] + o) = K == 1 ? a0 : fma(ml1, T(r1 + o), a0);
+                        }
+                    }
+#pragma unroll
+                    for (int c = 0; c < RC; ++c)
+                        bcol[c][1] = K == 1 ? fma(ml0, v0[c], bcol[c][1])
+                                             : fma(ml1, v1[c], fma(ml0, v0[c], bcol[c][1]));
+                }
+            }
+        };
+        if (kstep == 1) update(std::integral_constant<int, 1>{});
+        else update(std::integral_constant<int, 2>{});
         __syncthreads();
     }
     __syncthreads();
 
-    // ---- back substitution, last pivot (position 0) first: slot s froze into position
-    // n - 1 - s, so the rows frozen before a pivot are the positions above it
-    double x[TWO][RC], acc[TWO][RC];
+    // ---- back substitution, last pivot (position 0) first: the rows frozen before a pivot
+    // are the positions above it. A lane holds the reciprocal of its own diagonal entry and
+    // its right-hand side less what the solved positions below it contribute: its weight,
+    // once those are all solved, is the product.
+    double x[TWO][RC], acc[TWO][RC], dinv[TWO];
+    unsigned long long in_two[TWO];  // positions of 2x2 pivots (solved explicitly)
 #pragma unroll
-    for (int t = 0; t < TWO; ++t)
+    for (int t = 0; t < TWO; ++t) {
+        const int j = L + 64 * t;
+        dinv[t] = 0.0;
+        in_two[t] = twos[t] << 1 | twos[t] | (t ? twos[0] >> 63 : 0ull);
 #pragma unroll
         for (int c = 0; c < RC; ++c) {
             x[t][c] = 0.0;
             acc[t][c] = 0.0;
         }
+        if (!failed && j < n) dinv[t] = 1.0 / T(rbj[t] + 8 * j);
+    }
     if (!failed) {
-        const int nslots = slot;
-        double y[TWO][RC];
-        int bk[TWO];
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int j = L + 64 * t;
-#pragma unroll
-            for (int c = 0; c < RC; ++c) y[t][c] = j < n ? bcol[t][c] : 0.0;
-            // slot sl of the block list sits in lane sl % 64, register sl / 64
-            bk[t] = j < nslots ? (int)s_blk[j] : -1;
-        }
-        auto slot_of = [&](const int(&w)[TWO], int sl) -> int {
-            return (TWO == 2 && sl >= 64) ? rdlane(w[TWO - 1], sl & 63) : rdlane(w[0], sl & 63);
-        };
-        for (int s = nslots - 1; s >= 0; --s) {
-            const int blk = slot_of(bk, s);
-            const int bprev = s > 0 ? slot_of(bk, s - 1) : -1;
-            const bool one = blk == 1, two = (blk == 0) && (bprev == 2);
-            if (!one && !two) continue;  // first slot of a 2x2 block: solved with the second
-            // the block's pivots: pp (p0, slot s - 1 of a 2x2) and pq (p1, slot s)
-            const int pq = n - 1 - s;
+        for (int pq = 0; pq < n;) {
+            const bool two = ((TWO == 1 || pq < 64 ? twos[0] : twos[TWO - 1]) >> (pq & 63)) & 1ull;
+            // the block's pivots: pp (p0) and, for a 2x2, pq (p1) below it
             const int pp = two ? pq + 1 : pq;
+            if (!two) {
+                double arp[TWO];
+#pragma unroll
+                for (int t = 0; t < TWO; ++t) {
+                    const int j = L + 64 * t;
+                    arp[t] = (j > pp && j < n) ? T(rbj[t] + 8 * pp) : 0.0;
+                }
+#pragma unroll
+                for (int c = 0; c < RC; ++c) {
+                    if (c >= n_cols) continue;
+                    double r[TWO];
+#pragma unroll
+                    for (int t = 0; t < TWO; ++t) r[t] = (bcol[c][t] - acc[t][c]) * dinv[t];
+                    const double x0 = lane_get(r, pp);
+#pragma unroll
+                    for (int t = 0; t < TWO; ++t) {
+                        const int j = L + 64 * t;
+                        if (j > pp && j < n) acc[t][c] += arp[t] * x0;
+                    }
+                }
+                pq += 1;
+                continue;
+            }
             const int rbp = rb_of(pp), rbq = rb_of(pq);
-            const double dp = s_T[rbp + pp], dq = s_T[rbq + pq], bq = s_T[rbp + pq];
+            const double dp = T(rbp + 8 * pp), dq = T(rbq + 8 * pq), bq = T(rbp + 8 * pq);
             double arp[TWO], arq[TWO];
 #pragma unroll
             for (int t = 0; t < TWO; ++t) {
                 const int j = L + 64 * t;
                 const bool above = j > pp && j < n;
-                arp[t] = above ? s_T[rbj[t] + pp] : 0.0;
-                arq[t] = (two && above) ? s_T[rbj[t] + pq] : 0.0;
+                arp[t] = above ? T(rbj[t] + 8 * pp) : 0.0;
+                arq[t] = above ? T(rbj[t] + 8 * pq) : 0.0;
             }
-            // (one division per pivot: a 1x1 pivot needs only 1/dp, a 2x2 only 1/det)
-            double idet = 0.0, dinv = 0.0;
-            if (two) idet = 1.0 / (dp * dq - bq * bq);
-            else dinv = 1.0 / dp;
-            const int pl = pp & 63, pt = pp >> 6, ql = pq & 63, qt = pq >> 6;
-            // (the 1x1 and 2x2 solves are separate paths: a 1x1 pivot reads one right-hand
-            // side and updates with one column)
-            if (!two) {
-#pragma unroll
-                for (int c = 0; c < RC; ++c) {
-                    if (c >= n_cols) continue;
-                    const double rp0 = y[0][c] - acc[0][c];
-                    const double rp1 = TWO == 2 ? y[TWO - 1][c] - acc[TWO - 1][c] : 0.0;
-                    const double x0 = (pt ? rdlane(rp1, pl) : rdlane(rp0, pl)) * dinv;
-#pragma unroll
-                    for (int t = 0; t < TWO; ++t) {
-                        const int j = L + 64 * t;
-                        if (j == pp) x[t][c] = x0;
-                        if (j > pp && j < n) acc[t][c] += arp[t] * x0;
-                    }
-                }
-                continue;
-            }
+            const double idet = 1.0 / (dp * dq - bq * bq);
 #pragma unroll
             for (int c = 0; c < RC; ++c) {
                 if (c >= n_cols) continue;
-                const double rp0 = y[0][c] - acc[0][c];
-                const double rp1 = TWO == 2 ? y[TWO - 1][c] - acc[TWO - 1][c] : 0.0;
-                const double yp = pt ? rdlane(rp1, pl) : rdlane(rp0, pl);
-                const double yq = qt ? rdlane(rp1, ql) : rdlane(rp0, ql);
+                double r[TWO];
+#pragma unroll
+                for (int t = 0; t < TWO; ++t) r[t] = bcol[c][t] - acc[t][c];
+                const double yp = lane_get(r, pp), yq = lane_get(r, pq);
                 const double x0 = (yp * dq - yq * bq) * idet;
                 const double x1 = (yq * dp - yp * bq) * idet;
 #pragma unroll
@@ -1288,6 +1423,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
                     if (j > pp && j < n) acc[t][c] += arp[t] * x0 + arq[t] * x1;
                 }
             }
+            pq += 2;
+        }
+#pragma unroll
+        for (int t = 0; t < TWO; ++t) {
+            if ((in_two[t] >> L) & 1ull) continue;
+#pragma unroll
+            for (int c = 0; c < RC; ++c) x[t][c] = (bcol[c][t] - acc[t][c]) * dinv[t];
         }
     }
 
@@ -1366,8 +1508,10 @@ hipError_t launch_build_wide(const BuildDev& P, int dim, int rows_cap, int64_t n
     }
 }
 
-// dynamic LDS of k_build_sym: the packed triangle
-static int sym_tri(int rows_cap) { return kSymRbHost.rb[rows_cap]; }
+// dynamic LDS of k_build_sym: the packed triangle, and the entries that lanes
+// without a row may read past it in the trailing update (position 31 of row 0 at most, and
+// eight past a row's end)
+static int sym_tri(int rows_cap) { return kSymRbHost.rb[rows_cap] + 24; }
 static size_t sym_lds(int rows_cap, int n_cols)
 {
     (void)n_cols;  // (the right-hand sides live in registers)

@@ -41,6 +41,28 @@ def test_sym_build_parity_bases(RBF, O, gpu, name, kind, eps, dim, deg, k):
         _ran_sym(RBF)
 
 
+@pytest.mark.parametrize("name,kind,eps", [b for b in B.BASES if b[1] in (3, 10)])
+@pytest.mark.parametrize("dim,deg,k", [(2, 1, 4), (2, 0, 31), (2, 1, 29), (2, 1, 30), (2, 0, 33), (3, 1, 32), (3, 1, 33),
+                                       (2, 2, 58), (2, 2, 59), (2, 1, 64)])
+def test_sym_tile_edges(RBF, O, gpu, name, kind, eps, dim, deg, k):
+    """Odd and even point counts around the 32 and 64 where the assembly of point pairs and
+    the trailing update change how lanes share rows (32, 33, 64, 65 and 67 rows)."""
+    with pinned_sym(RBF):
+        B.test_build_parity_bases(RBF, O, gpu, name, kind, eps, dim, deg, k)
+        _ran_sym(RBF)
+
+
+def test_sym_more_than_64_points(RBF, O, gpu):
+    rng = np.random.default_rng(70)
+    pts = rng.random((400, 2))
+    adj = O.knn(pts, pts, 70)
+    with pinned_sym(RBF):
+        op = RBF.RadialBasisOperator(RBF.Laplacian(), pts, basis=RBF.PHS(3, poly_deg=2), adjl=[a for a in adj])
+        _ran_sym(RBF)
+    w = op.vals.cpu().numpy()
+    B.check_against_truth(O, w, pts, pts, adj, O.basis_struct(3, 2), B._op(O, 1, [(0, O.abi.OP_LAP, 0, 0, 1.0)]), 70)
+
+
 @pytest.mark.parametrize("which", ["d1", "d2", "mixed", "regrid", "grad", "hess3", "sum"])
 def test_sym_build_parity_operators(RBF, O, gpu, which):
     with pinned_sym(RBF):
