@@ -20,7 +20,7 @@
 // Bound: latency of the dependent cell-range and point loads at small sizes, VALU issue of
 // the merges beyond. Measured, whole search, before (three points per cell
 // whatever k, rings from the first, each candidate inserted as it came) and now: 900 points,
-// 2-D, k = 12: 172 -> 70 us; 100,000, 3-D, k = 20: 444 -> 216 us; 4M, 2-D, k = 20: 3.49 ->
+// 2-D, k = 12: 172 -> 70 us (a wavefront per query: 32 us); 100,000, 3-D, k = 20: 444 -> 216 us; 4M, 2-D, k = 20: 3.49 ->
 // 2.16 ms; 2M, 3-D, k = 40: 9.0 -> 5.2 ms.
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
@@ -555,6 +555,153 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
     }
 }
 
+// ---------------------------------------------------------------- few queries
+// A wavefront per query, for searches too small to fill the chip with a lane per query
+// (where one wavefront's chain of runs and merges takes 36 us whatever the count): bound by
+// the latency of its few dependent loads. The runs
+// of cells are looked up by one lane each, their candidates taken 64 at a time, and a
+// batch is merged by rank: each candidate that beats the k-th so far is broadcast, and every
+// lane counts how many come before its own. The visiting order, the distances and the
+// stopping test are k_query's, so the result is the same.
+__device__ __forceinline__ int rdlane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ double rdlane(double v, int l)
+{
+    return __hiloint2double(rdlane(__double2hiint(v), l), rdlane(__double2loint(v), l));
+}
+
+template <int DIM>
+__global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ sx, const int32_t* __restrict__ sidx,
+                                                    const int32_t* __restrict__ cell_start,
+                                                    const double* __restrict__ query, int64_t n_query,
+                                                    const Grid* __restrict__ Gd, int kmax,
+                                                    const int64_t* __restrict__ q_ptr, int32_t* __restrict__ out)
+{
+    __shared__ double s_d[4][64];
+    __shared__ int s_i[4][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int64_t qi = blockIdx.x * (int64_t)4 + w;
+    if (qi >= n_query) return;
+    const Grid G = *Gd;
+    double q[DIM];
+#pragma unroll
+    for (int d = 0; d < DIM; ++d) q[d] = query[qi * DIM + d];
+    const int c0 = cell_coord(q[0], G.lo[0], G.inv_s, G.n[0]);
+    const int c1 = DIM >= 2 ? cell_coord(q[DIM >= 2 ? 1 : 0], G.lo[1], G.inv_s, G.n[1]) : 0;
+    const int c2 = DIM == 3 ? cell_coord(q[DIM - 1], G.lo[2], G.inv_s, G.n[2]) : 0;
+    int maxn = G.n[0];
+    if (DIM >= 2) maxn = max(maxn, G.n[1]);
+    if (DIM == 3) maxn = max(maxn, G.n[2]);
+
+    // the nearest 64 so far, ascending, one per lane; the k-th of them
+    double bd = __builtin_huge_val(), kd = bd;
+    int bi = 0x7fffffff, ki = bi;
+    for (int rho = 2;; ++rho) {
+        // The block of two rings as whole rows, then a ring's rows: whole on its faces, else
+        // the two end cells (one id each).
+        const int W = 2 * rho + 1, rows = DIM == 1 ? 1 : (DIM == 2 ? W : W * W);
+        const int n_ids = rho == 2 ? rows : 2 * rows;
+        for (int id0 = 0; id0 < n_ids; id0 += 64) {
+            const int id = id0 + lane, r = rho == 2 ? id : id >> 1, part = rho == 2 ? 0 : id & 1;
+            const int dy = DIM >= 2 ? r % W - rho : 0, dz = DIM == 3 ? r / W - rho : 0;
+            const int cy = c1 + dy, cz = c2 + dz;
+            const bool face = rho == 2 || (DIM >= 2 && (dy == -rho || dy == rho)) || (DIM == 3 && (dz == -rho || dz == rho));
+            int xl = c0 - rho, xh = c0 + rho;
+            bool in = id < n_ids && cy >= 0 && cy < G.n[1] && cz >= 0 && cz < G.n[2];
+            if (face) {
+                in = in && part == 0;
+            } else if (part == 0) {
+                in = in && xl >= 0;
+                xh = xl;
+            } else {
+                in = in && xh < G.n[0];
+                xl = xh;
+            }
+            int32_t s0 = 0, cnt = 0;
+            if (in) {
+                const int64_t row = ((int64_t)cz * G.n[1] + cy) * G.n[0];
+                s0 = cell_start[row + max(xl, 0)];
+                cnt = cell_start[row + min(xh, G.n[0] - 1) + 1] - s0;
+            }
+            // candidate f of the batch lies in the first run whose inclusive count exceeds it
+            int inc = cnt;
+#pragma unroll
+            for (int s = 1; s < 64; s <<= 1) {
+                const int v = __shfl_up(inc, s, 64);
+                inc += lane >= s ? v : 0;
+            }
+            const int total = rdlane(inc, 63);
+            const int base = s0 - (inc - cnt);
+            for (int f0 = 0; f0 < total; f0 += 64) {
+                const int f = f0 + lane;
+                int run = 0;
+#pragma unroll
+                for (int s = 32; s; s >>= 1) {
+                    const int v = __shfl(inc, run + s - 1, 64);
+                    run += v <= f ? s : 0;
+                }
+                const int b = __shfl(base, run & 63, 64);
+                double cd = __builtin_huge_val();
+                int ci = 0x7fffffff;
+                if (f < total) {
+                    double x[DIM];
+#pragma unroll
+                    for (int d = 0; d < DIM; ++d) x[d] = sx[(int64_t)(b + f) * DIM + d];
+                    cd = sqdist<DIM>(x, q);
+                    ci = sidx[b + f];
+                }
+                const bool pass = f < total && lt(cd, ci, kd, ki);
+                const unsigned long long m = __ballot(pass);
+                if (!m) continue;
+                int rb = lane, rn = 0;
+                for (unsigned long long left = m; left; left &= left - 1) {
+                    const int l = __builtin_ctzll(left);
+                    const double nd = rdlane(cd, l);
+                    const int ni = rdlane(ci, l);
+                    const bool before = lt(nd, ni, bd, bi);
+                    rb += before ? 1 : 0;
+                    rn += lt(nd, ni, cd, ci) ? 1 : 0;
+                    const int ahead = 64 - __popcll(__ballot(before));
+                    rn += lane == l ? ahead : 0;
+                }
+                if (rb < 64) {
+                    s_d[w][rb] = bd;
+                    s_i[w][rb] = bi;
+                }
+                if (pass && rn < 64) {
+                    s_d[w][rn] = cd;
+                    s_i[w][rn] = ci;
+                }
+                // (a wavefront's LDS accesses complete in order)
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_wave_barrier();
+                bd = s_d[w][lane];
+                bi = s_i[w][lane];
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_wave_barrier();
+                kd = rdlane(bd, kmax - 1);
+                ki = rdlane(bi, kmax - 1);
+            }
+        }
+        // (k_query's stopping test)
+        double bound = 1e300;
+        bool covers_all = true;
+        auto side_bound = [&](int d, int cd) __attribute__((always_inline)) {
+            const double at = q[d] - G.lo[d];
+            if (cd - rho > 0) bound = fmin(bound, at - (cd - rho) * G.s);
+            if (cd + rho + 1 < G.n[d]) bound = fmin(bound, (cd + rho + 1) * G.s - at);
+            if (cd - rho > 0 || cd + rho + 1 < G.n[d]) covers_all = false;
+        };
+        side_bound(0, c0);
+        if constexpr (DIM >= 2) side_bound(1, c1);
+        if constexpr (DIM == 3) side_bound(2, c2);
+        if (covers_all || rho > maxn) break;
+        if (ki != 0x7fffffff && bound > 0.0 && kd < bound * bound * (1.0 - 1e-9)) break;
+    }
+    const int64_t base = q_ptr ? q_ptr[qi] : qi * (int64_t)kmax;
+    const int kq = q_ptr ? (int)(q_ptr[qi + 1] - q_ptr[qi]) : kmax;
+    if (lane < kq && lane < kmax) out[base + lane] = bi;
+}
+
 // ---------------------------------------------------------------- processing order
 __device__ __forceinline__ uint32_t compact_bits(uint32_t m, int dim, int d)
 {
@@ -622,12 +769,23 @@ static hipError_t scan(KnnWorkspace& ws, const int32_t* in, int32_t* out, int64_
     return hipcub::DeviceScan::ExclusiveSum(ws.scan_tmp, have, in, out, (int)n, st);
 }
 
+// A wavefront per query up to here: whole searches of 2-D points with k = 12, a wavefront
+// and a lane per query: 900 points 32 and 61 us, 8,000 66 and 86, 16,000 76 and 86, 32,000 97
+// and 89; 3-D, k = 20: 45 and 190, 83 and 170, 104 and 164, 172 and 172; 3-D, k = 40: 49 and
+// 312, 106 and 260, 142 and 330, 217 and 345.
+constexpr int64_t kWaveQueries = 24576;
+
 // the register list costs merges and VGPRs with KCAP, so KCAP follows k closely in the
 // common range
 template <int DIM>
 static hipError_t launch_query(const KnnWorkspace& ws, const double* query, const int32_t* qorder, int64_t n_query,
                                int k, const int64_t* q_ptr, int32_t* out, hipStream_t st)
 {
+    if (n_query <= kWaveQueries) {
+        hipLaunchKernelGGL(k_query_wave<DIM>, dim3((unsigned)((n_query + 3) / 4)), dim3(256), 0, st, ws.sx, ws.sidx,
+                           ws.start, query, n_query, (const Grid*)ws.grid, k, q_ptr, out);
+        return hipGetLastError();
+    }
     const dim3 gq((unsigned)((n_query + 63) / 64));
 #define RBFX_KNN_LAUNCH(KC)                                                                                  \
     if (k <= KC) {                                                                                           \

@@ -37,6 +37,28 @@ def test_knn_order_is_a_spatial_permutation(RBF, gpu, dim, n, nq):
     assert step < 8.0 * n ** (-1.0 / dim), step
 
 
+@pytest.mark.parametrize("dim,k", [(1, 5), (1, 64), (2, 1), (2, 16), (2, 20), (2, 33), (2, 64), (3, 24), (3, 48)])
+def test_knn_wavefront_and_lane_per_query_agree(RBF, gpu, dim, k):
+    """25,000 queries (a lane each) against the same queries in two parts (a wavefront each):
+    a cloud with clusters, a lattice of ties, repeated points, far queries, ragged lists."""
+    import torch
+
+    rng = np.random.default_rng(100 * dim + k)
+    x = np.concatenate([rng.random((3000, dim)), 0.5 + 1e-3 * rng.standard_normal((1500, dim)),
+                        rng.integers(0, 12, (1500, dim)) / 11.0])
+    q = np.concatenate([x, x[rng.integers(0, 6000, 18_990)] + rng.normal(0, 0.05, (18_990, dim)),
+                        rng.normal(0, 30.0, (10, dim))])
+    x, q = torch.as_tensor(x, device=gpu), torch.as_tensor(q, device=gpu)
+    whole = RBF._lib.knn(x, q, k)
+    parts = torch.cat([RBF._lib.knn(x, q[a:a + 12_500].contiguous(), k) for a in (0, 12_500)])
+    assert torch.equal(whole, parts)
+    n = torch.as_tensor(rng.integers(0, k + 1, 12_500), device=gpu)
+    ptr = torch.cat([torch.zeros(1, dtype=torch.int64, device=gpu), torch.cumsum(n, 0)])
+    ragged = RBF._lib.knn(x, q[:12_500].contiguous(), k, q_ptr=ptr)
+    mask = torch.arange(k, device=gpu)[None, :] < n[:, None]
+    assert torch.equal(ragged, whole[:12_500][mask])
+
+
 def test_operator_with_and_without_order_agree(RBF, gpu):
     """70,000 points: weights of the ordered build equal the unordered ones bit for bit."""
     import torch
