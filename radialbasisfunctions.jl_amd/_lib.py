@@ -4,6 +4,7 @@ torch is used only to own device buffers and to obtain HIP stream handles; every
 kernel is launched by the C-ABI library. There is no CPU fallback: without the
 library or without a gfx950 device the calls raise.
 """
+import contextlib
 import ctypes as C
 import pathlib
 import threading
@@ -115,10 +116,16 @@ def _check(rc):
         raise RbfxError(rc, msg)
 
 
-def torch():
-    import torch as _t
+_TORCH = None
 
-    return _t
+
+def torch():
+    global _TORCH
+    if _TORCH is None:
+        import torch as _t
+
+        _TORCH = _t
+    return _TORCH
 
 
 def device_for(device=None):
@@ -138,8 +145,22 @@ def device_for(device=None):
 
 
 def stream_ptr(dev):
+    return C.c_void_p(raw_stream(dev))
+
+
+def raw_stream(dev):
+    """The current stream of dev as an integer (no Stream object is made: 0.2 against 2 us)."""
     t = torch()
-    return C.c_void_p(t.cuda.current_stream(dev).cuda_stream)
+    return t._C._cuda_getCurrentRawStream(dev.index if dev.index is not None else t.cuda.current_device())
+
+
+_HERE = contextlib.nullcontext()
+
+
+def on_device(dev):
+    """Context that makes dev the current device (nothing to do where it already is)."""
+    t = torch()
+    return _HERE if t._C._cuda_getDevice() == dev.index else t.cuda.device(dev)
 
 
 def ptr(x):
@@ -157,7 +178,7 @@ def knn(data, query, k, q_ptr=None, order=False):
     else:
         out = t.empty(int(q_ptr[-1].item()), dtype=t.int32, device=dev)
     perm = t.empty(n_q, dtype=t.int32, device=dev) if order else None
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_knn_ordered(ptr(data), data.shape[0], ptr(query), n_q, data.shape[1], int(k), ptr(q_ptr),
                                       ptr(out), ptr(perm), stream_ptr(dev)))
     return (out, perm) if order else out
@@ -165,7 +186,7 @@ def knn(data, query, k, q_ptr=None, order=False):
 
 def build_weights(args, dev):
     t = torch()
-    with t.cuda.device(dev):
+    with on_device(dev):
         rc = lib().rbfx_build_weights(C.byref(args))
     counts = (C.c_int64 * 16)()
     lib().rbfx_last_build_counts(counts)
@@ -222,14 +243,14 @@ def tune_reset():
 
 def spmv(args, dev, asynchronous=False):
     t = torch()
-    with t.cuda.device(dev):
+    with on_device(dev):
         f = lib().rbfx_spmv_async if asynchronous else lib().rbfx_spmv
         _check(f(C.byref(args)))
 
 
 def build_weights_async(args, dev):
     t = torch()
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_build_weights_async(C.byref(args)))
 
 
@@ -255,14 +276,14 @@ def mlp_run(x, params, wbf16, workspace, batch, target=None, grads=None, loss=No
     a.workspace = workspace.data_ptr()
     a.stream = stream_ptr(dev).value
     a.row_weight = None if row_weight is None else row_weight.data_ptr()
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_mlp_run(C.byref(a)))
 
 
 def mlp_adam(params, grads, m, v, wbf16, lr, beta1, beta2, eps, step):
     t = torch()
     dev = params.device
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_mlp_adam(ptr(params), ptr(grads), ptr(m), ptr(v), ptr(wbf16), float(lr), float(beta1),
                                    float(beta2), float(eps), int(step), stream_ptr(dev)))
 
@@ -270,7 +291,7 @@ def mlp_adam(params, grads, m, v, wbf16, lr, beta1, beta2, eps, step):
 def mlp_sync_bf16(params, wbf16):
     t = torch()
     dev = params.device
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_mlp_sync_bf16(ptr(params), ptr(wbf16), stream_ptr(dev)))
 
 
@@ -288,7 +309,7 @@ def stencil_features(data, eval_points, adj, k, want_xi=True, want_x=True, want_
     x = t.empty((n, abi.MLP_IN_PAD), dtype=t.bfloat16, device=dev) if want_x else None
     h = t.empty(n, dtype=t.float64, device=dev) if want_h else None
     r1 = t.empty(n, dtype=t.float64, device=dev)
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_stencil_features(ptr(data), ptr(eval_points), n, data.shape[1], int(k), ptr(adj), ptr(xi),
                                            ptr(x), ptr(h), ptr(r1), stream_ptr(dev)))
     return xi, x, h, r1
@@ -306,7 +327,7 @@ def spatial_order(points):
     t = torch()
     dev = points.device
     out = t.empty(points.shape[0], dtype=t.int32, device=dev)
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_spatial_order(ptr(points), points.shape[0], points.shape[1], ptr(out), stream_ptr(dev)))
     return out
 
@@ -323,7 +344,7 @@ def source_tiles(n_rows, k, col, tile_rows):
     toff = t.empty(n_tiles, dtype=t.int64, device=dev)
     tcol = t.empty(int(n_rows) * int(k), dtype=t.int16, device=dev)
     n_src = C.c_int64(0)
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_source_tiles(int(n_rows), int(k), ptr(col), int(tile_rows), ptr(tn), ptr(toff), ptr(tcol),
                                        None, 0, C.byref(n_src), stream_ptr(dev)))
         tsrc = t.empty(max(1, n_src.value), dtype=t.int32, device=dev)
@@ -340,7 +361,7 @@ def permute_rows(order, k, col, vals):
     n = order.shape[0]
     col_p = t.empty_like(col)
     vals_p = t.empty_like(vals)
-    with t.cuda.device(dev):
+    with on_device(dev):
         _check(lib().rbfx_permute_rows(n, int(k), ptr(order), ptr(col), ptr(vals), vals.shape[1], vals.shape[0],
                                        ptr(col_p), ptr(vals_p), stream_ptr(dev)))
     return col_p, vals_p

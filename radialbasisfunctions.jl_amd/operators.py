@@ -398,20 +398,24 @@ def _hermite_arrays(hermite, n_data, dim, dev):
         raise DimensionMismatch(
             f"boundary_conditions ({len(bcs)}) and normals ({nrm.shape[0]}) must each have one entry per "
             f"boundary point (count(is_boundary) = {nb})")
-    bidx = np.full(n_data, -1, dtype=np.int32)
-    bidx[np.nonzero(isb)[0]] = np.arange(nb, dtype=np.int32)
+    nodes = np.flatnonzero(isb)
     al = np.array([b.alpha for b in bcs], dtype=np.float64)
     be = np.array([b.beta for b in bcs], dtype=np.float64)
+    # (the arrays over all points are filled on the device from the boundary nodes)
     t = _lib.torch()
+    at = t.as_tensor(nodes, device=dev)
+    mask = t.zeros(n_data, dtype=t.uint8, device=dev)
+    mask[at] = 1
+    bidx = t.full((n_data,), -1, dtype=t.int32, device=dev)
+    bidx[at] = t.arange(nb, dtype=t.int32, device=dev)
     arrays = dict(
-        is_boundary=t.as_tensor(isb.astype(np.uint8), device=dev),
-        bnd_index=t.as_tensor(bidx, device=dev),
+        is_boundary=mask,
+        bnd_index=bidx,
         bc_alpha=t.as_tensor(al if nb else np.zeros(1), device=dev),
         bc_beta=t.as_tensor(be if nb else np.zeros(1), device=dev),
         normals=t.as_tensor(nrm if nb else np.zeros((1, dim)), device=dev),
     )
-    host = dict(is_boundary=isb, bnd_index=bidx, bc_alpha=al, bc_beta=be)
-    return arrays, host, nb
+    return arrays, nodes[(al == 1.0) & (be == 0.0)], nb
 
 
 def _adjacency(adjl, n_eval):
@@ -555,7 +559,7 @@ class RadialBasisOperator:
         keep = []
         row_ptr = self.adj_ptr
         if self.hermite is not None:
-            arrs, host, nb = _hermite_arrays(self.hermite, self.n_data, self.dim, self.dev)
+            arrs, dirichlet, nb = _hermite_arrays(self.hermite, self.n_data, self.dim, self.dev)
             keep.append(arrs)
             a.is_boundary = _lib.ptr(arrs["is_boundary"])
             a.bnd_index = _lib.ptr(arrs["bnd_index"])
@@ -564,21 +568,13 @@ class RadialBasisOperator:
             a.normals = _lib.ptr(arrs["normals"])
             a.n_bnd = nb
             # exact row lengths (count_nonzeros, execution.jl:39-69): Dirichlet eval rows hold 1 entry
-            lens = (np.diff(self.adj_ptr.cpu().numpy()) if self.adj_ptr is not None
-                    else np.full(self.n_eval, self.k, dtype=np.int64))
-            e_idx = np.arange(self.n_eval)
-            isb = np.zeros(self.n_eval, dtype=bool)
-            m = e_idx < self.n_data
-            isb[m] = host["is_boundary"][e_idx[m]]
-            dmask = np.zeros(self.n_eval, dtype=bool)
-            if isb.any():
-                bi = host["bnd_index"][e_idx[isb]]
-                dmask[isb] = (host["bc_alpha"][bi] == 1.0) & (host["bc_beta"][bi] == 0.0)
-            if dmask.any():
-                lens = np.where(dmask, 1, lens)
-                ptr = np.zeros(self.n_eval + 1, dtype=np.int64)
-                np.cumsum(lens, out=ptr[1:])
-                row_ptr = t.as_tensor(ptr, device=self.dev)
+            dirichlet = dirichlet[dirichlet < self.n_eval]
+            if dirichlet.size:
+                lens = (self.adj_ptr[1:] - self.adj_ptr[:-1] if self.adj_ptr is not None
+                        else t.full((self.n_eval,), self.k, dtype=t.int64, device=self.dev))
+                lens[t.as_tensor(dirichlet, device=self.dev)] = 1
+                row_ptr = t.zeros(self.n_eval + 1, dtype=t.int64, device=self.dev)
+                t.cumsum(lens, 0, out=row_ptr[1:])
         nnz = int(row_ptr[-1].item()) if row_ptr is not None else self.n_eval * self.k
         # output buffers are reused across rebuilds (a captured graph keeps their addresses)
         old = getattr(self, "vals", None)
@@ -710,32 +706,20 @@ class RadialBasisOperator:
         t = _lib.torch()
         F = X.shape[1]
         Y = out if out is not None else t.empty((self.n_cols, self.n_eval, F), dtype=t.float64, device=self.dev)
-        s = abi.SpmvArgs()
-        s.n_rows = self.n_eval
-        s.n_cols = self.n_data
-        s.row_ptr = _lib.ptr(self.row_ptr)
-        s.k = self.k
-        s.col_idx = _lib.ptr(self.col)
-        s.vals = _lib.ptr(self.vals)
-        s.nnz = self.vals.shape[1]
-        s.n_valarrays = self.n_cols
-        s.n_fields = F
-        s.x = _lib.ptr(X)
-        s.x_ld_point = X.stride(0)
-        s.x_ld_field = X.stride(1)
-        s.y = _lib.ptr(Y)
-        s.y_ld_point = Y.stride(1)
-        s.y_ld_field = Y.stride(2)
-        s.y_ld_val = Y.stride(0)
-        s.alpha = float(alpha)
-        s.beta = float(beta)
-        s.stream = _lib.stream_ptr(self.dev)
+        vals, row_ptr = self.vals, self.row_ptr
+        sx, sy = X.stride(), Y.stride()
+        # (in the order of the struct's fields: one call, where an assignment a field took 7 us)
+        s = abi.SpmvArgs(self.n_eval, self.n_data, None if row_ptr is None else row_ptr.data_ptr(), self.k,
+                         self.col.data_ptr(), vals.data_ptr(), vals.shape[1], self.n_cols, F,
+                         X.data_ptr(), sx[0], sx[1], Y.data_ptr(), sy[1], sy[2], sy[0],
+                         float(alpha), float(beta), _lib.raw_stream(self.dev))
         if self._row_order is None and self.n_eval >= self.SPATIAL_ORDER_MIN:
             # rows walked along a Z-curve of the eval points: neighbouring rows gather
             # neighbouring X entries (the result does not depend on the order)
             self._row_order = _lib.spatial_order(self._d_eval)
-        s.row_order = _lib.ptr(self._row_order)
-        if self.row_ptr is not None and self._max_row is None:
+        if self._row_order is not None:
+            s.row_order = self._row_order.data_ptr()
+        if row_ptr is not None and self._max_row is None:
             self._max_row = int((self.row_ptr[1:] - self.row_ptr[:-1]).max().item()) if self.n_eval > 0 else 0
         s.max_row_len = self._max_row or 0
         s.mapping = self.SPMV_MAPPING
@@ -770,15 +754,17 @@ class RadialBasisOperator:
             self.update_weights()
         t = _lib.torch()
         is_torch = isinstance(x, t.Tensor)
-        xd = _to_device(x, self.dev, t.float64)
+        xd = x
+        if not (is_torch and x.dtype == t.float64 and x.device == self.dev and x.is_contiguous()):
+            xd = _to_device(x, self.dev, t.float64)
         if xd.shape[0] != self.n_data:
             raise DimensionMismatch(f"field has {xd.shape[0]} rows, operator has {self.n_data} data points")
         vec = xd.ndim == 1
-        X = xd[:, None] if vec else xd.reshape(xd.shape[0], -1)
+        X = xd.unsqueeze(1) if vec else xd.reshape(xd.shape[0], -1)
         Y = self._spmv(X)
         trailing = () if vec else tuple(xd.shape[1:])
         if self.rank == 0:
-            res = Y[0].reshape((self.n_eval,) + trailing)
+            res = Y.view((self.n_eval,) + trailing) if self.n_cols == 1 else Y[0].reshape((self.n_eval,) + trailing)
         elif self.rank == 1:
             res = Y.permute(1, 2, 0).reshape((self.n_eval,) + trailing + (self.n_cols,))
         else:
