@@ -14,6 +14,13 @@
 //   D. accept when max|residual| <= tol * max|L phi|: write w = w~ h^-order and the
 //      column indices; otherwise queue the stencil for the solver.
 // Four lanes (a DPP quad) share a stencil in phases A, C and D; rows i = q, q+4, ...
+//
+// Bound by VALU issue (70% of the cycles: 8,100 instructions a wavefront, the GELUs half
+// of them) and by the latency of its serial phases, so the wavefronts in flight count: the
+// FP64 tables reuse the activations' LDS (39 KB a workgroup, it was 73), the monomials are
+// evaluated where they are used and the surrogate's own basis has an instantiation of its
+// own, which holds three wavefronts per SIMD instead of two; the residual reads a point
+// once for a lane's rows. 1M stencils: 1.80 -> 1.31 ms.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -29,28 +36,25 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 constexpr int kBM = 64;           // stencils per workgroup
 constexpr int kActLd = kHid + 8;  // BF16 row stride of the activation tile (16-B aligned rows)
 
+// the value of the quad's lane (lane ^ X), X = 1 or 2, as a DPP move (a shuffle is an LDS
+// permute: the FP64 phases have 70 of these sums)
+template <int X>
+__device__ __forceinline__ double quad_xor(double v)
+{
+    constexpr int ctrl = X == 1 ? 0xB1 : 0x4E;  // quad_perm [1,0,3,2], [2,3,0,1]
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), ctrl, 0xF, 0xF, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), ctrl, 0xF, 0xF, true));
+}
 __device__ __forceinline__ double quad_sum(double v)
 {
-    v += __shfl_xor(v, 1, 64);
-    v += __shfl_xor(v, 2, 64);
+    v += quad_xor<1>(v);
+    v += quad_xor<2>(v);
     return v;
 }
 __device__ __forceinline__ double quad_max(double v)
 {
-    v = fmax(v, __shfl_xor(v, 1, 64));
-    v = fmax(v, __shfl_xor(v, 2, 64));
-    return v;
-}
-
-// monomial a (graded exponents e) at a 2-D point
-__device__ __forceinline__ double mono2(const int (&e)[3], double x, double y)
-{
-    double v = 1.0;
-#pragma unroll
-    for (int p = 0; p < kMaxPolyDeg; ++p) {
-        if (p < e[0]) v *= x;
-        if (p < e[1]) v *= y;
-    }
+    v = fmax(v, quad_xor<1>(v));
+    v = fmax(v, quad_xor<2>(v));
     return v;
 }
 
@@ -64,6 +68,8 @@ __device__ __forceinline__ void mlp_tiles(const __bf16 (*act)[kActLd], const __b
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int fr = lane & 15, fk = (lane >> 4) * 8;
+    // (unrolled further, the loads in flight spill across three wavefronts per SIMD)
+#pragma unroll 2
     for (int k0 = 0; k0 < KL; k0 += 32) {
         bf16x8 a[4], b[NT];
 #pragma unroll
@@ -98,16 +104,20 @@ __device__ __forceinline__ void hidden_layer(__bf16 (*act)[kActLd], const __bf16
     __syncthreads();
 }
 
-template <int K, int MM>
-__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(2))) void k_learned(
+// KIND: the basis, or -1 for the one P names (every basis' terms in one kernel take the
+// registers of a wavefront per SIMD)
+template <int K, int MM, int KIND>
+__global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_per_eu(KIND < 0 ? 2 : 3))) void k_learned(
     const LearnedDev P)
 {
     constexpr int R = (K + 3) / 4;  // rows per quad lane
-    __shared__ __attribute__((aligned(16))) __bf16 s_act[kBM][kActLd];
-    __shared__ double s_xi[kBM][K][2];
-    __shared__ float s_out[kBM][kOutPad + 1];
-    __shared__ double s_w[kBM][K];
-    __shared__ int s_mono[MM][3];
+    // the activations (phase B) and the FP64 tables (phases A and C) share their LDS
+    constexpr int kXi = kBM * K * 2 * 8, kW = kBM * K * 8, kOut = kBM * (kOutPad + 1) * 4, kAct = kBM * kActLd * 2;
+    __shared__ __attribute__((aligned(16))) char s_buf[kXi + kW + kOut > kAct ? kXi + kW + kOut : kAct];
+    __bf16(*s_act)[kActLd] = reinterpret_cast<__bf16(*)[kActLd]>(s_buf);
+    double(*s_xi)[K][2] = reinterpret_cast<double(*)[K][2]>(s_buf);
+    double(*s_w)[K] = reinterpret_cast<double(*)[K]>(s_buf + kXi);
+    float(*s_out)[kOutPad + 1] = reinterpret_cast<float(*)[kOutPad + 1]>(s_buf + kXi + kW);
     __shared__ TermDev s_terms[RBFX_MAX_TERMS];
 
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
@@ -118,7 +128,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     int64_t e = (P.order && wi < P.n_eval) ? (int64_t)P.order[wi] : wi;
     const bool live = wi < P.n_eval && e >= 0 && e < P.n_eval;
     if (!live) e = 0;
-    if (t < MM * 3) (&s_mono[0][0])[t] = (&P.mono_e[0][0])[t];
     if (t < RBFX_MAX_TERMS) s_terms[t] = P.terms[t];
 
     // ---- A. radius-scaled offsets and the canonical frame
@@ -128,18 +137,16 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         ye = P.eval[2 * e + 1];
     }
     double dx[R], dy[R];
-    int gi[R];
     double h2 = 0.0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int i = q + 4 * r;
         dx[r] = 0.0;
         dy[r] = 0.0;
-        gi[r] = 0;
         if (live && i < K) {
-            gi[r] = P.adj_idx[e * K + i];
-            dx[r] = P.data[2 * (int64_t)gi[r]] - xe;
-            dy[r] = P.data[2 * (int64_t)gi[r] + 1] - ye;
+            const int64_t g = P.adj_idx[e * K + i];
+            dx[r] = P.data[2 * g] - xe;
+            dy[r] = P.data[2 * g + 1] - ye;
             h2 = fmax(h2, dx[r] * dx[r] + dy[r] * dy[r]);
         }
     }
@@ -183,8 +190,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         const int i = q + 4 * r;
         dy[r] *= fl;
         if (i < K) {
-            s_xi[sl][i][0] = dx[r];
-            s_xi[sl][i][1] = dy[r];
             // BF16 high part, then the BF16 rounding of the remainder
             const __bf16 hx = (__bf16)(float)dx[r], hy = (__bf16)(float)dy[r];
             s_act[sl][2 * i] = hx;
@@ -200,9 +205,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
     hidden_layer<kInPad>(s_act, P.wbf16 + mlp_wb_off(0), P.params + mlp_b_off(0), w, lane);
     hidden_layer<kHid>(s_act, P.wbf16 + mlp_wb_off(1), P.params + mlp_b_off(1), w, lane);
     hidden_layer<kHid>(s_act, P.wbf16 + mlp_wb_off(2), P.params + mlp_b_off(2), w, lane);
+    f32x4 acc[4][1];
+    if (w < kOutPad / 16) mlp_tiles<kHid, 1>(s_act, P.wbf16 + mlp_wb_off(3), w * 16, acc, lane);
+    __syncthreads();  // the activations have been read
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int i = q + 4 * r;
+        if (i < K) {
+            s_xi[sl][i][0] = dx[r];
+            s_xi[sl][i][1] = dy[r];
+        }
+    }
     if (w < kOutPad / 16) {
-        f32x4 acc[4][1];
-        mlp_tiles<kHid, 1>(s_act, P.wbf16 + mlp_wb_off(3), w * 16, acc, lane);
         const int col = w * 16 + (lane & 15);
         const float b = P.params[mlp_b_off(3) + col];
 #pragma unroll
@@ -214,15 +228,18 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 
     // ---- C. FP64 projection, multiplier refit and collocation residual
     BasisDev B;
-    B.kind = P.basis_kind;
+    B.kind = KIND < 0 ? P.basis_kind : KIND;
     B.eps = (B.kind == RBFX_IMQ || B.kind == RBFX_GAUSSIAN) ? P.eps * h : P.eps;
     double wt[R];
     double ptw[MM], G[MM][MM];
-    double pr[R][MM];  // the monomials at this lane's rows, evaluated once
+    // the monomials at row r of this lane, evaluated at each use (three products; kept, the
+    // 30 values cost the registers of a third wavefront per SIMD)
+    auto monos = [&](int r, double (&m)[MM]) __attribute__((always_inline)) {
+        double p2[2] = {dx[r], dy[r]};
+        asm volatile("" : "+v"(p2[0]), "+v"(p2[1]));
 #pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int a = 0; a < MM; ++a) pr[r][a] = mono2(s_mono[a], dx[r], dy[r]);
+        for (int a = 0; a < MM; ++a) m[a] = mono_graded<2>(a, p2);
+    };
 #pragma unroll
     for (int a = 0; a < MM; ++a) {
         ptw[a] = 0.0;
@@ -236,11 +253,13 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
         if (i < K) {
             // the network predicts w~ r1^2 (r1: the canonical reference distance)
             wt[r] = ((double)s_out[sl][i] * P.out_std[i] + P.out_mean[i]) / (r1 * r1);
+            double pr[MM];
+            monos(r, pr);
 #pragma unroll
             for (int a = 0; a < MM; ++a) {
-                ptw[a] += pr[r][a] * wt[r];
+                ptw[a] += pr[a] * wt[r];
 #pragma unroll
-                for (int b = 0; b <= a; ++b) G[a][b] += pr[r][a] * pr[r][b];
+                for (int b = 0; b <= a; ++b) G[a][b] += pr[a] * pr[b];
             }
         }
     }
@@ -277,7 +296,8 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
             double lp = 0.0;
             for (int tt = 0; tt < P.n_terms; ++tt) {
                 const TermDev tm = s_terms[tt];
-                lp += tm.coeff * mono_op<2>(s_mono[a], tm.kind, tm.d1, tm.d2, z);
+                const int ea[3] = {graded_exp(2, a, 0), graded_exp(2, a, 1), 0};
+                lp += tm.coeff * mono_op<2>(ea, tm.kind, tm.d1, tm.d2, z);
             }
             rhs[a] = lp - ptw[a];
         }
@@ -300,49 +320,55 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int i = q + 4 * r;
-        double corr = 0.0;
+        double corr = 0.0, pr[MM];
+        monos(r, pr);
 #pragma unroll
-        for (int a = 0; a < MM; ++a) corr += pr[r][a] * rhs[a];
+        for (int a = 0; a < MM; ++a) corr += pr[a] * rhs[a];
         wt[r] += corr;
         if (i < K) s_w[sl][i] = wt[r];
     }
     __syncthreads();
-    // s_i = L phi(x_e, x_i) - sum_j phi(|xi_i - xi_j|) w~_j
+    // s_i = L phi(x_e, x_i) - sum_j phi(|xi_i - xi_j|) w~_j: a point's coordinates and
+    // weight are read once for this lane's R rows
     double sres[R], lmax = 0.0;
+    auto phi_sum = [&](auto phi) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) sres[r] = 0.0;
+#pragma unroll 1
+        for (int j = 0; j < K; ++j) {
+            const double xj = s_xi[sl][j][0], yj = s_xi[sl][j][1], wj = s_w[sl][j];
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const double ex = dx[r] - xj, ey = dy[r] - yj;
+                sres[r] += phi(ex * ex + ey * ey) * wj;
+            }
+        }
+    };
+    phi_sum([&](double q2) { return phi_r2(B, q2); });
     double pts[MM];
 #pragma unroll
     for (int a = 0; a < MM; ++a) pts[a] = 0.0;
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         const int i = q + 4 * r;
-        sres[r] = 0.0;
         if (i < K) {
             const double De[2] = {-dx[r], -dy[r]};
             const double q2 = dx[r] * dx[r] + dy[r] * dy[r];
             double lphi = 0.0;
             for (int tt = 0; tt < P.n_terms; ++tt) {
                 const TermDev tm = s_terms[tt];
-                lphi += tm.coeff * phi_term<2>(B, tm.kind, tm.d1, tm.d2, De, q2);
+                double q2t = q2;
+                asm volatile("" : "+v"(q2t));  // (or every term kind's roots move out of the loop)
+                lphi += tm.coeff * phi_term<2>(B, tm.kind, tm.d1, tm.d2, De, q2t);
             }
             lmax = fmax(lmax, fabs(lphi));
-            double acc = 0.0;
-            if (B.kind == RBFX_PHS3) {  // uniform: the surrogate's own basis, without the basis switch
-#pragma unroll 4
-                for (int j = 0; j < K; ++j) {
-                    const double ex = dx[r] - s_xi[sl][j][0], ey = dy[r] - s_xi[sl][j][1];
-                    const double q2 = ex * ex + ey * ey;
-                    acc += q2 * sqrt(q2) * s_w[sl][j];
-                }
-            } else {
-#pragma unroll 4
-                for (int j = 0; j < K; ++j) {
-                    const double ex = dx[r] - s_xi[sl][j][0], ey = dy[r] - s_xi[sl][j][1];
-                    acc += phi_r2(B, ex * ex + ey * ey) * s_w[sl][j];
-                }
-            }
-            sres[r] = lphi - acc;
+            sres[r] = lphi - sres[r];
+            double pr[MM];
+            monos(r, pr);
 #pragma unroll
-            for (int a = 0; a < MM; ++a) pts[a] += pr[r][a] * sres[r];
+            for (int a = 0; a < MM; ++a) pts[a] += pr[a] * sres[r];
+        } else {
+            sres[r] = 0.0;
         }
     }
 #pragma unroll
@@ -352,9 +378,10 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
 #pragma unroll
     for (int r = 0; r < R; ++r) {
         if (q + 4 * r < K) {
-            double v = sres[r];
+            double v = sres[r], pr[MM];
+            monos(r, pr);
 #pragma unroll
-            for (int a = 0; a < MM; ++a) v -= pr[r][a] * pts[a];
+            for (int a = 0; a < MM; ++a) v -= pr[a] * pts[a];
             rmax = fmax(rmax, fabs(v));
         }
     }
@@ -375,7 +402,7 @@ __global__ __attribute__((amdgpu_flat_work_group_size(256, 256), amdgpu_waves_pe
             const int i = q + 4 * r;
             if (i < K) {
                 P.out_val[e * K + i] = wt[r] * sc;
-                if (P.out_col) P.out_col[e * K + i] = gi[r];
+                if (P.out_col) P.out_col[e * K + i] = P.adj_idx[e * K + i];
             }
         }
         if (q == 0 && P.status) P.status[e] = RBFX_ST_LEARNED;
@@ -391,7 +418,9 @@ hipError_t launch_learned_build(const LearnedDev& P, hipStream_t s)
     if (P.k != 20 || P.n_mono != 6) return hipErrorInvalidValue;
     LearnedDev Q = P;
     Q.n_blocks = (P.n_eval + kBM - 1) / kBM;
-    hipLaunchKernelGGL((k_learned<20, 6>), dim3((unsigned)pad_to_xcds(Q.n_blocks)), dim3(256), 0, s, Q);
+    const dim3 grid((unsigned)pad_to_xcds(Q.n_blocks));
+    if (P.basis_kind == RBFX_PHS3) hipLaunchKernelGGL((k_learned<20, 6, RBFX_PHS3>), grid, dim3(256), 0, s, Q);
+    else hipLaunchKernelGGL((k_learned<20, 6, -1>), grid, dim3(256), 0, s, Q);
     return hipGetLastError();
 }
 
