@@ -279,6 +279,7 @@ static int spmv_impl(const rbfx_spmv_args* a, bool async)
     hipStream_t st = (hipStream_t)a->stream;
     rbfx::SpmvDev P;
     P.n_rows = a->n_rows;
+    P.n_src = a->n_cols > 0 ? a->n_cols : 0;
     P.row_ptr = a->row_ptr;
     P.k = a->k;
     P.col_idx = a->col_idx;

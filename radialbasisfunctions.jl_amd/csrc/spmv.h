@@ -7,6 +7,7 @@ namespace rbfx {
 
 struct SpmvDev {
     int64_t n_rows;
+    int64_t n_src;  // points of X (0: unknown)
     const int64_t* row_ptr;
     int k;
     const int32_t* col_idx;

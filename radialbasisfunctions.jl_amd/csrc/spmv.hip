@@ -326,10 +326,82 @@ __device__ __forceinline__ void fields_rows(const SpmvDev& P, int64_t r0, int64_
     }
 }
 
+// fields_rows for a staged tile whose X lies within 4 GB: the tile's columns are byte offsets
+// into X, made once per entry while staging instead of by each of a row's lanes, so a gather
+// is one 32-bit add and a load from a uniform base, and whole groups of U entries carry no
+// per-entry selects. Same products in the same order.
+// Bound by the gathers through the L1 (16 cycles of the address unit for the 1 KB of a
+// wavefront's load, 30.7 GB of them) and L2 (17 GB missed): 16 fields, 8M rows of 30:
+// 1.73 -> 1.65 ms, the same with six to thirteen workgroups on a CU, 1.89 with four.
+template <int NV, int LPR, int FPL, int U>
+__device__ __forceinline__ void fields_rows_near(const SpmvDev& P, int64_t r0, int64_t r1, int64_t b0,
+                                                 const uint32_t* off, const double* val, int vstride)
+{
+    const int f0 = (threadIdx.x % LPR) * FPL;
+    const int64_t r = r0 + threadIdx.x / LPR;
+    if (r >= r1 || f0 >= P.n_fields) return;
+    const int64_t row = P.row_order ? (int64_t)P.row_order[r] : r;
+    const int qb = (int)((P.row_ptr ? P.row_ptr[r] : r * (int64_t)P.k) - b0);
+    const int qe = (int)((P.row_ptr ? P.row_ptr[r + 1] : (r + 1) * (int64_t)P.k) - b0);
+    const char* x = reinterpret_cast<const char*>(P.x);
+    const uint32_t fo = (uint32_t)(f0 * (int)P.x_ld_field) * 8u;
+    double acc[NV][FPL];
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+#pragma unroll
+        for (int j = 0; j < FPL; ++j) acc[v][j] = 0.0;
+    auto group = [&](auto N, int q0) __attribute__((always_inline)) {
+        constexpr int n = decltype(N)::value;
+        double xv[n][FPL], w[n][NV];
+#pragma unroll
+        for (int u = 0; u < n; ++u) {
+            const uint32_t o = off[q0 + u] + fo;
+            if constexpr (FPL == 2) {
+                const f64x2 t = *reinterpret_cast<const f64x2*>(x + o);
+                xv[u][0] = t.x;
+                xv[u][1] = t.y;
+            } else {
+                xv[u][0] = *reinterpret_cast<const double*>(x + o);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < n; ++u)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) w[u][v] = val[v * vstride + q0 + u];
+#pragma unroll
+        for (int u = 0; u < n; ++u)
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+#pragma unroll
+                for (int j = 0; j < FPL; ++j) acc[v][j] += w[u][v] * xv[u][j];
+    };
+    int q0 = qb;
+    for (; q0 + U <= qe; q0 += U) group(std::integral_constant<int, U>{}, q0);
+    for (; q0 < qe; ++q0) group(std::integral_constant<int, 1>{}, q0);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+        double* yp = P.y + (int64_t)v * P.y_ld_val + row * P.y_ld_point + (int64_t)f0 * P.y_ld_field;
+#pragma unroll
+        for (int j = 0; j < FPL; ++j) acc[v][j] *= P.alpha;
+        if constexpr (FPL == 2) {
+            f64x2 out = {acc[v][0], acc[v][1]};
+            if (P.beta != 0.0) {
+                const f64x2 old = *reinterpret_cast<const f64x2*>(yp);
+                out.x += P.beta * old.x;
+                out.y += P.beta * old.y;
+            }
+            *reinterpret_cast<f64x2*>(yp) = out;
+        } else {
+            *yp = (P.beta == 0.0) ? acc[v][0] : acc[v][0] + P.beta * *yp;
+        }
+    }
+}
+
 // The workgroup's rows (256 / LPR, stored back to back) first have their index and
 // value runs copied into LDS, as in k_spmv_staged; a workgroup whose entries exceed
 // the LDS it was given (a longest-row bound that was too small) reads HBM instead.
-template <int NV, int LPR, int FPL, int U>
+// NEAR: X lies within 4 GB (fields_rows_near).
+template <int NV, int LPR, int FPL, int U, bool NEAR>
 __global__ __launch_bounds__(256) void k_spmv_fields_staged(const SpmvDev P, int64_t nb_real, int cap)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char s_raw[];
@@ -344,17 +416,21 @@ __global__ __launch_bounds__(256) void k_spmv_fields_staged(const SpmvDev P, int
         const int64_t b1 = P.row_ptr ? P.row_ptr[r1] : r1 * (int64_t)P.k;
         const int64_t n_e = b1 - b0;
         if (n_e > cap) {
-            fields_rows<NV, LPR, FPL, U>(P, r0, r1, 0, P.col_idx, P.vals, P.nnz);
+            fields_rows<NV, LPR, FPL, NEAR ? 2 : U>(P, r0, r1, 0, P.col_idx, P.vals, P.nnz);
             continue;  // LDS untouched in this tile
         }
         for (int i = threadIdx.x; i < n_e; i += 256) {
-            s_col[i] = __builtin_nontemporal_load(P.col_idx + b0 + i);
+            const int32_t c = __builtin_nontemporal_load(P.col_idx + b0 + i);
+            s_col[i] = NEAR ? (int32_t)((uint32_t)c * (uint32_t)P.x_ld_point * 8u) : c;
 #pragma unroll
             for (int v = 0; v < NV; ++v)
                 s_val[v * cap + i] = __builtin_nontemporal_load(P.vals + (int64_t)v * P.nnz + b0 + i);
         }
         __syncthreads();
-        fields_rows<NV, LPR, FPL, U>(P, r0, r1, b0, (const int32_t*)s_col, (const double*)s_val, (int64_t)cap);
+        if constexpr (NEAR)
+            fields_rows_near<NV, LPR, FPL, U>(P, r0, r1, b0, (const uint32_t*)s_col, (const double*)s_val, cap);
+        else
+            fields_rows<NV, LPR, FPL, U>(P, r0, r1, b0, (const int32_t*)s_col, (const double*)s_val, (int64_t)cap);
         __syncthreads();  // the next tile overwrites the LDS copy
     }
 }
@@ -816,6 +892,13 @@ static bool fields_pair(const SpmvDev& P)
     return (P.n_fields % 2) == 0 && P.x_ld_field == 1 && (P.x_ld_point % 2) == 0 && ((uintptr_t)P.x & 15) == 0 &&
            P.y_ld_field == 1 && (P.y_ld_point % 2) == 0 && (P.y_ld_val % 2) == 0 && ((uintptr_t)P.y & 15) == 0;
 }
+// whether every entry of X lies less than 4 GB from its start (byte offsets fit 32 bits)
+static bool fields_near(const SpmvDev& P)
+{
+    const int64_t ldp = P.x_ld_point, ldf = P.x_ld_field, lim = (int64_t(1) << 29) - 1;
+    if (P.n_src < 1 || ldp < 0 || ldf < 0 || P.n_src > lim || ldp > lim || ldf > lim / 64) return false;
+    return (__int128)(P.n_src - 1) * ldp + (P.n_fields - 1) * ldf <= lim;
+}
 static int fields_lpr(const SpmvDev& P)
 {
     const int fpl = fields_pair(P) ? 2 : 1;
@@ -892,12 +975,17 @@ static hipError_t spmv_nv(const SpmvDev& P, double avg_row, hipStream_t s)
         if (fstaged && P.mapping != 1) {
             const int64_t nbr = (P.n_rows + 256 / lpr - 1) / (256 / lpr);
             const size_t lds = (size_t)cap * (8 * NV + 4);
+            const bool near = fields_near(P);
             // 6 gathers in flight per lane: 16-field k = 30 regrid 1.78 ms, against 1.83 ms
             // for 10, 1.81 for 5, 1.86 for 4, 1.94 for 15
 #define RBFX_FSTAGED(LL, FF)                                                                                      \
     {                                                                                                             \
-        hipLaunchKernelGGL((k_spmv_fields_staged<NV, LL, FF, 6>), dim3((unsigned)pad8(nbr)), dim3(256), lds, s, P, \
-                           nbr, (int)cap);                                                                        \
+        if (near)                                                                                                 \
+            hipLaunchKernelGGL((k_spmv_fields_staged<NV, LL, FF, 6, true>), dim3((unsigned)pad8(nbr)), dim3(256), \
+                               lds, s, P, nbr, (int)cap);                                                         \
+        else                                                                                                      \
+            hipLaunchKernelGGL((k_spmv_fields_staged<NV, LL, FF, 6, false>), dim3((unsigned)pad8(nbr)), dim3(256), \
+                               lds, s, P, nbr, (int)cap);                                                         \
         return hipGetLastError();                                                                                 \
     }
             if (pair) {
