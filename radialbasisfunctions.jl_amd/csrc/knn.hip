@@ -20,8 +20,8 @@
 // Bound: latency of the dependent cell-range and point loads at small sizes, VALU issue of
 // the merges beyond. Measured, whole search, before (three points per cell
 // whatever k, rings from the first, each candidate inserted as it came) and now: 900 points,
-// 2-D, k = 12: 172 -> 70 us (a wavefront per query: 32 us); 100,000, 3-D, k = 20: 444 -> 216 us; 4M, 2-D, k = 20: 3.49 ->
-// 2.16 ms; 2M, 3-D, k = 40: 9.0 -> 5.2 ms.
+// 2-D, k = 12: 172 -> 70 us (a wavefront per query: 28 us); 100,000, 3-D, k = 20: 444 -> 216 us
+// (170 us); 4M, 2-D, k = 20: 3.49 -> 2.16 ms; 2M, 3-D, k = 40: 9.0 -> 5.2 ms (3.5 ms).
 #include <hip/hip_runtime.h>
 #include <hipcub/hipcub.hpp>
 #include <stdint.h>
@@ -328,15 +328,15 @@ __device__ __forceinline__ void run_merge(double* d, int* i, std::integer_sequen
     (comp(d[net.c[Q].a], i[net.c[Q].a], d[net.c[Q].b], i[net.c[Q].b]), ...);
 }
 
-// candidates waiting per lane (the longest lists leave registers for 8 only)
-constexpr int pend_of(int kcap) { return kcap <= 40 ? 16 : 8; }
+constexpr int kPend = 16;  // candidates waiting per lane
 
 // KCAP sorted entries (bd, bi) and the lane's n pending candidates -> the KCAP smallest
 template <int KCAP>
 __device__ __forceinline__ void merge_pending(double (&bd)[KCAP], int (&bi)[KCAP], const double (*pd)[64],
                                               const int (*pi)[64], int n)
 {
-    constexpr int P = KCAP <= 16 ? 16 : (KCAP <= 32 ? 32 : 64), kPend = pend_of(KCAP);
+    constexpr int P = KCAP <= 16 ? 16 : 32;
+    static_assert(KCAP <= 32, "longer lists are searched by wavefronts");
     const int lane = threadIdx.x & 63;
     double d[P];
     int i[P];
@@ -384,7 +384,6 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
                                               const Grid* __restrict__ Gd, int kmax,
                                               const int64_t* __restrict__ q_ptr, int32_t* __restrict__ out)
 {
-    constexpr int kPend = pend_of(KCAP);
     __shared__ double s_pd[kPend][64];
     __shared__ int s_pi[kPend][64];
     const int lane = threadIdx.x;
@@ -556,12 +555,14 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
 }
 
 // ---------------------------------------------------------------- few queries
-// A wavefront per query, for searches too small to fill the chip with a lane per query
+// A wavefront per query, for lists too long for a lane's registers and for searches too small
+// to fill the chip with a lane per query
 // (where one wavefront's chain of runs and merges takes 36 us whatever the count): bound by
 // the latency of its few dependent loads. The runs
 // of cells are looked up by one lane each, their candidates taken 64 at a time, and a
-// batch is merged by rank: each candidate that beats the k-th so far is broadcast, and every
-// lane counts how many come before its own. The visiting order, the distances and the
+// batch with many that beat the k-th so far is sorted over the lanes (DPP moves) and merged
+// with the list; a batch with few is merged by rank: each is broadcast, and every lane
+// counts how many come before its own. The visiting order, the distances and the
 // stopping test are k_query's, so the result is the same.
 __device__ __forceinline__ int rdlane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 __device__ __forceinline__ double rdlane(double v, int l)
@@ -569,18 +570,106 @@ __device__ __forceinline__ double rdlane(double v, int l)
     return __hiloint2double(rdlane(__double2hiint(v), l), rdlane(__double2loint(v), l));
 }
 
+// the value of lane ^ X: DPP moves inside a row of 16 lanes, a permute beyond
+template <int X>
+__device__ __forceinline__ int lane_xor(int v)
+{
+    if constexpr (X == 1) return __builtin_amdgcn_mov_dpp(v, 0xB1, 0xF, 0xF, true);
+    else if constexpr (X == 2) return __builtin_amdgcn_mov_dpp(v, 0x4E, 0xF, 0xF, true);
+    else if constexpr (X == 3) return __builtin_amdgcn_mov_dpp(v, 0x1B, 0xF, 0xF, true);
+    else if constexpr (X == 4) return lane_xor<3>(__builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true));
+    else if constexpr (X == 7) return __builtin_amdgcn_mov_dpp(v, 0x141, 0xF, 0xF, true);   // row_half_mirror
+    else if constexpr (X == 8) return __builtin_amdgcn_mov_dpp(v, 0x128, 0xF, 0xF, true);   // row_ror:8
+    else if constexpr (X == 15) return __builtin_amdgcn_mov_dpp(v, 0x140, 0xF, 0xF, true);  // row_mirror
+    else return __shfl_xor(v, X, 64);
+}
+template <int X>
+__device__ __forceinline__ double lane_xor(double v)
+{
+    return __hiloint2double(lane_xor<X>(__double2hiint(v)), lane_xor<X>(__double2loint(v)));
+}
+
+// lanes l and l ^ X keep the smaller and the larger of their entries, the smaller in the
+// lower lane
+template <int X>
+__device__ __forceinline__ void exchange(double& d, int& i, int lane)
+{
+    constexpr int top = X >= 32 ? 32 : (X >= 16 ? 16 : (X >= 8 ? 8 : (X >= 4 ? 4 : (X >= 2 ? 2 : 1))));
+    const double od = lane_xor<X>(d);
+    const int oi = lane_xor<X>(i);
+    const bool take = lt(od, oi, d, i) == ((lane & top) == 0);
+    d = take ? od : d;
+    i = take ? oi : i;
+}
+// ascending over the 64 lanes (bitonic, each merge begun by the mirrored exchange)
+__device__ __forceinline__ void lane_sort(double& d, int& i, int lane)
+{
+    exchange<1>(d, i, lane);
+    exchange<3>(d, i, lane);
+    exchange<1>(d, i, lane);
+    exchange<7>(d, i, lane);
+    exchange<2>(d, i, lane);
+    exchange<1>(d, i, lane);
+    exchange<15>(d, i, lane);
+    exchange<4>(d, i, lane);
+    exchange<2>(d, i, lane);
+    exchange<1>(d, i, lane);
+    exchange<31>(d, i, lane);
+    exchange<8>(d, i, lane);
+    exchange<4>(d, i, lane);
+    exchange<2>(d, i, lane);
+    exchange<1>(d, i, lane);
+    exchange<63>(d, i, lane);
+    exchange<16>(d, i, lane);
+    exchange<8>(d, i, lane);
+    exchange<4>(d, i, lane);
+    exchange<2>(d, i, lane);
+    exchange<1>(d, i, lane);
+}
+// the 64 smallest of two ascending lists, ascending
+__device__ __forceinline__ void lane_merge(double& d, int& i, double nd, int ni, int lane)
+{
+    const double rd = lane_xor<63>(nd);
+    const int ri = lane_xor<63>(ni);
+    const bool take = lt(rd, ri, d, i);
+    d = take ? rd : d;
+    i = take ? ri : i;
+    exchange<32>(d, i, lane);
+    exchange<16>(d, i, lane);
+    exchange<8>(d, i, lane);
+    exchange<4>(d, i, lane);
+    exchange<2>(d, i, lane);
+    exchange<1>(d, i, lane);
+}
+// inclusive sum over the 64 lanes
+__device__ __forceinline__ int lane_sum(int v)
+{
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, true);   // row_shr:1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, true);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // lane 15 of a row to the next one
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // lane 31 to the upper half
+    return v;
+}
+
+// candidates that a batch merges by rank (14 instructions each) rather than by sorting (280)
+constexpr int kRankMerge = 12;
+
 template <int DIM>
 __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ sx, const int32_t* __restrict__ sidx,
                                                     const int32_t* __restrict__ cell_start,
-                                                    const double* __restrict__ query, int64_t n_query,
+                                                    const double* __restrict__ query, const int32_t* __restrict__ qorder,
+                                                    int64_t n_query,
                                                     const Grid* __restrict__ Gd, int kmax,
                                                     const int64_t* __restrict__ q_ptr, int32_t* __restrict__ out)
 {
     __shared__ double s_d[4][64];
     __shared__ int s_i[4][64];
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int64_t qi = blockIdx.x * (int64_t)4 + w;
-    if (qi >= n_query) return;
+    const int64_t t = blockIdx.x * (int64_t)4 + w;
+    if (t >= n_query) return;
+    const int64_t qi = qorder ? qorder[t] : t;
     const Grid G = *Gd;
     double q[DIM];
 #pragma unroll
@@ -593,8 +682,12 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
     if (DIM == 3) maxn = max(maxn, G.n[2]);
 
     // the nearest 64 so far, ascending, one per lane; the k-th of them
-    double bd = __builtin_huge_val(), kd = bd;
-    int bi = 0x7fffffff, ki = bi;
+    // (kd read from a lane: as a constant, the compiler loads this infinity into a scalar pair
+    // with one 64-bit literal, which the hardware does not have, and gets 0)
+    double bd = __builtin_huge_val();
+    asm volatile("" : "+v"(bd));
+    double kd = rdlane(bd, 0);
+    int bi = 0x7fffffff, ki = bi, ki0 = bi;
     for (int rho = 2;; ++rho) {
         // The block of two rings as whole rows, then a ring's rows: whole on its faces, else
         // the two end cells (one id each).
@@ -623,19 +716,13 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
                 cnt = cell_start[row + min(xh, G.n[0] - 1) + 1] - s0;
             }
             // candidate f of the batch lies in the first run whose inclusive count exceeds it
-            int inc = cnt;
-#pragma unroll
-            for (int s = 1; s < 64; s <<= 1) {
-                const int v = __shfl_up(inc, s, 64);
-                inc += lane >= s ? v : 0;
-            }
+            const int inc = lane_sum(cnt), n_run = min(n_ids - id0, 64);
             const int total = rdlane(inc, 63);
             const int base = s0 - (inc - cnt);
             for (int f0 = 0; f0 < total; f0 += 64) {
                 const int f = f0 + lane;
                 int run = 0;
-#pragma unroll
-                for (int s = 32; s; s >>= 1) {
+                for (int s = n_run > 32 ? 32 : (n_run > 16 ? 16 : (n_run > 4 ? 8 : 2)); s; s >>= 1) {
                     const int v = __shfl(inc, run + s - 1, 64);
                     run += v <= f ? s : 0;
                 }
@@ -652,6 +739,21 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
                 const bool pass = f < total && lt(cd, ci, kd, ki);
                 const unsigned long long m = __ballot(pass);
                 if (!m) continue;
+                if (__popcll(m) > kRankMerge) {
+                    cd = pass ? cd : __builtin_huge_val();
+                    ci = pass ? ci : 0x7fffffff;
+                    lane_sort(cd, ci, lane);
+                    if (ki0 == 0x7fffffff) {  // nothing yet
+                        bd = cd;
+                        bi = ci;
+                    } else {
+                        lane_merge(bd, bi, cd, ci, lane);
+                    }
+                    kd = rdlane(bd, kmax - 1);
+                    ki = rdlane(bi, kmax - 1);
+                    ki0 = rdlane(bi, 0);
+                    continue;
+                }
                 int rb = lane, rn = 0;
                 for (unsigned long long left = m; left; left &= left - 1) {
                     const int l = __builtin_ctzll(left);
@@ -680,6 +782,7 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
                 __builtin_amdgcn_wave_barrier();
                 kd = rdlane(bd, kmax - 1);
                 ki = rdlane(bi, kmax - 1);
+                ki0 = rdlane(bi, 0);
             }
         }
         // (k_query's stopping test)
@@ -769,11 +872,18 @@ static hipError_t scan(KnnWorkspace& ws, const int32_t* in, int32_t* out, int64_
     return hipcub::DeviceScan::ExclusiveSum(ws.scan_tmp, have, in, out, (int)n, st);
 }
 
-// A wavefront per query up to here: whole searches of 2-D points with k = 12, a wavefront
-// and a lane per query: 900 points 32 and 61 us, 8,000 66 and 86, 16,000 76 and 86, 32,000 97
-// and 89; 3-D, k = 20: 45 and 190, 83 and 170, 104 and 164, 172 and 172; 3-D, k = 40: 49 and
-// 312, 106 and 260, 142 and 330, 217 and 345.
-constexpr int64_t kWaveQueries = 24576;
+// Searches that take a wavefront per query: all of more than 32 neighbours (a lane's list of
+// 64 no longer hides its merges: 3M points, 2-D, k = 60: 6.6 ms against 11.9 with a lane per
+// query; k = 35: 4.5 and 5.0), the others up to the count where lanes catch up. Whole
+// searches in us, a wavefront and a lane per query: 2-D, k = 13: 900 points 28 and 61, 65,000
+// 102 and 95, 300,000 294 and 169; k = 20: 900 31 and 111, 100,000 163 and 170, 150,000 220
+// and 189; 3-D, k = 20: 900 34 and 190, 100,000 170 and 208, 300,000 419 and 406 (Halton)
+// or 405 and 515 (random), 1M 1193 and 976.
+constexpr int kMaxLaneList = 32;
+static bool query_by_wavefront(int dim, int k, int64_t n_query)
+{
+    return k > kMaxLaneList || n_query <= (dim == 3 ? 262144 : 65536);
+}
 
 // the register list costs merges and VGPRs with KCAP, so KCAP follows k closely in the
 // common range
@@ -781,9 +891,10 @@ template <int DIM>
 static hipError_t launch_query(const KnnWorkspace& ws, const double* query, const int32_t* qorder, int64_t n_query,
                                int k, const int64_t* q_ptr, int32_t* out, hipStream_t st)
 {
-    if (n_query <= kWaveQueries) {
+    if (query_by_wavefront(DIM, k, n_query)) {
+        // (the spatial order pays for its load once the points outgrow the caches)
         hipLaunchKernelGGL(k_query_wave<DIM>, dim3((unsigned)((n_query + 3) / 4)), dim3(256), 0, st, ws.sx, ws.sidx,
-                           ws.start, query, n_query, (const Grid*)ws.grid, k, q_ptr, out);
+                           ws.start, query, n_query > 16384 ? qorder : nullptr, n_query, (const Grid*)ws.grid, k, q_ptr, out);
         return hipGetLastError();
     }
     const dim3 gq((unsigned)((n_query + 63) / 64));
@@ -796,10 +907,7 @@ static hipError_t launch_query(const KnnWorkspace& ws, const double* query, cons
     RBFX_KNN_LAUNCH(16)
     RBFX_KNN_LAUNCH(20)
     RBFX_KNN_LAUNCH(24)
-    RBFX_KNN_LAUNCH(32)
-    RBFX_KNN_LAUNCH(40)
-    RBFX_KNN_LAUNCH(48)
-    RBFX_KNN_LAUNCH(64)
+    RBFX_KNN_LAUNCH(kMaxLaneList)
 #undef RBFX_KNN_LAUNCH
     return hipErrorInvalidValue;
 }
