@@ -818,7 +818,7 @@ inline hipError_t launch_nse_rc(const BuildDev& P, int64_t n_work, hipStream_t s
     return hipErrorInvalidValue;
 }
 
-// Ragged launches: the two classes of one and two slots (nse_classes).
+// Ragged launches: the classes of one slot and of two (nse_classes).
 template <int KIND, int DIM, int M, int RC>
 inline hipError_t launch_nse_class_m(const BuildDev& P, int hi, int64_t n_work, hipStream_t s)
 {
@@ -827,6 +827,8 @@ inline hipError_t launch_nse_class_m(const BuildDev& P, int hi, int64_t n_work, 
         return launch_nse_one<KIND, DIM, M, 26, RC, RC <= 1 ? 2 : 1, true>(P, n_work, s);
     } else {
         if (hi <= 16 - RC) return launch_nse_one<KIND, DIM, M, 16 - RC, RC, M <= 6 ? 4 : 3, true>(P, n_work, s);
+        if constexpr (DIM == 2)
+            if (hi > 26) return launch_nse_one<KIND, DIM, M, 32 - RC, RC, 2, true>(P, n_work, s);
         return launch_nse_one<KIND, DIM, M, 26, RC, 2, true>(P, n_work, s);
     }
 }

@@ -126,7 +126,7 @@ def test_nse_repeated_builds_bit_identical(RBF, gpu):
                                                     (5, 3, (3, 3), "lap", 50)])
 def test_nse_classes_of_uneven_builds(RBF, O, gpu, kind, dim, degs, cols, kmax):
     """Ragged stencils of mixed degree: those within a class run on the elimination kernel
-    (null points from 1 to 26, a wavefront's four stencils of different k), the others on the
+    (null points from 1 to 31, a wavefront's four stencils of different k), the others on the
     rook kernels; every stencil against the extended-precision oracle at max(1e-10, kappa u),
     and a captured replay gives the eager build's bits."""
     import torch
@@ -139,7 +139,7 @@ def test_nse_classes_of_uneven_builds(RBF, O, gpu, kind, dim, degs, cols, kmax):
     deg = rng.integers(degs[0], degs[1] + 1, n).astype(np.int8)
     mono = np.array([comb(dim + d, dim) for d in deg])
     ks = np.maximum(rng.integers(mono + 1, kmax + 1), 2)
-    edges = [1, 12, 13, 14, 15, 16, 20, 21, 26, 27]
+    edges = [1, 12, 13, 14, 15, 16, 20, 21, 26, 27, 29, 30, 31, 32, 33]
     for i in range(300):  # the edges of the classes, each several times
         ks[i] = min(kmax, mono[i] + edges[i % len(edges)])
     adjl = [full[i, :ks[i]] for i in range(n)]
