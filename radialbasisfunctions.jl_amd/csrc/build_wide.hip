@@ -639,9 +639,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_wid
 //   - up to 32 active rows both halves of the wavefront share the rows;
 //   - uniform work (the search's masks and maxima, where a row starts, 2x2 flags) is scalar;
 //   - the back substitution takes the reciprocals of all diagonal entries in one division.
-// 147.5 -> 83.5 ms there; 33..64 and 65..70 rows of a disk with boundary points
-// (92,000 stencils) 18.9 -> 14.2 ms. LDS is allocated in steps of 1,280 bytes: 6,344 bytes (34 rows) hold
-// 25 wavefronts on a CU, 6,408 had held 21 (91.6 ms).
+// 147.5 -> 83.5 ms there; 290,000 stencils of 33..70 rows of a disk with boundary points
+// 18.9 -> 14.2 ms. LDS is allocated in steps of 1,280 bytes: 6,344 bytes (34 rows) hold 25
+// wavefronts on a CU, 6,408 had held 21 (91.6 ms).
 //
 // Row starts: row j holds positions 0..j padded to a multiple of eight (the update's
 // eight-column chunks stay inside the row), plus the fewest entries (0..31) that put the
