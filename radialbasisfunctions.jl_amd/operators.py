@@ -770,10 +770,12 @@ class RadialBasisOperator:
         else:
             D = self.dim
             full = t.empty((self.n_eval,) + trailing + (D, D), dtype=t.float64, device=self.dev)
-            Yp = Y.reshape((self.n_cols, self.n_eval) + trailing)
-            for c, (i, j) in enumerate(_sym_pairs(D)):
-                full[..., i, j] = Yp[c]
-                full[..., j, i] = Yp[c]
+            Yp = Y.reshape((self.n_cols, self.n_eval) + trailing).movedim(0, -1)
+            at = {p: c for c, p in enumerate(_sym_pairs(D))}
+            for i in range(D):  # row i: columns (0, i) .. (i - 1, i), then (i, i) .. (i, D - 1), in one run
+                for j in range(i):
+                    full[..., i, j] = Yp[..., at[j, i]]
+                full[..., i, i:] = Yp[..., at[i, i]:at[i, i] + D - i]
             res = full
         if self.dtype == "float32":
             res = res.to(t.float32)
