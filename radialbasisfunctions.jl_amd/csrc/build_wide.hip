@@ -638,7 +638,9 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_wid
 //     broadcast them (DPP), where eight LDS broadcasts had taken a third of the LDS cycles;
 //   - up to 32 active rows both halves of the wavefront share the rows;
 //   - uniform work (the search's masks and maxima, where a row starts, 2x2 flags) is scalar;
-//   - the back substitution takes the reciprocals of all diagonal entries in one division.
+//   - the back substitution takes the reciprocals of all diagonal entries in one division;
+//   - systems of more than 64 rows leave the two-slot loop at 64 (51,000 of 65..70 rows: 4.55
+//     -> 3.94 ms).
 // 147.5 -> 83.5 ms there; 290,000 stencils of 33..70 rows of a disk with boundary points
 // 18.9 -> 14.2 ms. LDS is allocated in steps of 1,280 bytes: 6,344 bytes (34 rows) hold 25
 // wavefronts on a CU, 6,408 had held 21 (91.6 ms).
@@ -1112,83 +1114,6 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
         om[t] = bits(n, t);
         twos[t] = 0ull;
     }
-    // Column c (uniform) of the active block to this lane's registers (v[t] = A(j, c)
-    // for its positions j < n_act: row j's entry if c <= j, else row c's entry j), and
-    // the largest |A(j, c)| over active j != c as a packed (magnitude, position) key.
-    double v[TWO];
-    auto colkey = [&](int c) -> uint32_t {
-        const int cc = __builtin_amdgcn_readfirstlane(c);
-        const int rbc = rb_of(cc);
-        uint32_t k = 0u;
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int j = L + 64 * t;
-            if (t && n_act <= 64) break;
-            unsigned long long m = bits(n_act, t);
-            if (TWO == 1 || cc >> 6 == t) m &= ~(1ull << (cc & 63));
-            // (lanes past the active rows read entry (0, cc) or of row cc, and are masked)
-            v[t] = T(j >= cc ? (j < n_act ? rbj[t] : 0) + 8 * cc : rbc + 8 * j);
-            k = max(k, lanes_in(m, row_key(v[t], j) & 0x7fffffffu));
-        }
-        return first_max_u32(k, n_act);
-    };
-    auto colval = [&](int r) -> double {
-        const int rr = __builtin_amdgcn_readfirstlane(r);
-        return (TWO == 2 && rr >= 64) ? rdlane(v[TWO - 1], rr & 63) : rdlane(v[0], rr & 63);
-    };
-    // symmetric swap of positions lo <= hi (both active): the rows and the columns, for
-    // every row of the system (frozen rows keep their entries at the active positions);
-    // each entry of the lower triangle that moves is moved by exactly one lane: lane k
-    // swaps (k, lo) with (k, hi), lane lo the diagonal entries, lane hi nothing
-    auto swap_entries = [&](int lo, int hi, int rhi) {
-        const int rlo = rb_of(lo);
-#pragma unroll
-        for (int t = 0; t < TWO; ++t) {
-            const int k = L + 64 * t;
-            if (k >= n || k == hi) continue;
-            const int k8 = 8 * k;
-            const int x0 = k >= lo ? rbj[t] + 8 * lo : rlo + k8;
-            const int x1 = k > hi ? rbj[t] + 8 * hi : rhi + (k == lo ? 8 * hi : k8);
-            const double y0 = T(x0), y1 = T(x1);
-            T(x0) = y1;
-            T(x1) = y0;
-        }
-    };
-    auto lane_put = [&](auto& w, auto v_, int p) __attribute__((always_inline)) {
-        if constexpr (TWO == 2) {
-            const auto w0 = w[0], w1 = w[1];  // (by value: a choice of elements would go to memory)
-            w[0] = p < 64 ? wrlane(w0, v_, p & 63) : w0;
-            w[1] = p < 64 ? w1 : wrlane(w1, v_, p & 63);
-        } else {
-            w[0] = wrlane(w[0], v_, p);
-        }
-    };
-    auto lane_get = [&](const auto& w, int p) __attribute__((always_inline)) {
-        const auto w0 = w[0], w1 = w[TWO - 1];
-        const auto a0 = rdlane(w0, p & 63);
-        if constexpr (TWO == 2) return p < 64 ? a0 : rdlane(w1, p & 63);
-        else return a0;
-    };
-    // The pivot of position p goes to the last active position q: its row start rq is
-    // returned, its right-hand sides in vq.
-    auto freeze = [&](int p, int q, double(&vq)[RC]) __attribute__((always_inline)) -> int {
-        const int rq = rb_of(q), o = lane_get(orig, p);
-        if (TWO == 2 && o >= 64) om[TWO - 1] &= ~(1ull << (o & 63));
-        else om[0] &= ~(1ull << (o & 63));
-#pragma unroll
-        for (int c = 0; c < RC; ++c) vq[c] = lane_get(bcol[c], p);
-        if (p != q) {
-            swap_entries(p, q, rq);
-            lane_put(orig, lane_get(orig, q), p);
-            lane_put(orig, o, q);
-#pragma unroll
-            for (int c = 0; c < RC; ++c) {
-                lane_put(bcol[c], lane_get(bcol[c], q), p);
-                lane_put(bcol[c], vq[c], q);
-            }
-        }
-        return rq;
-    };
     // The trailing update's rows: lane L updates row jr; with up to 32 active rows, both
     // halves of the wavefront share the rows, the upper half eight columns on.
     int jr = L, rbu = rbj[0];
@@ -1200,153 +1125,241 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
         shared = true;
     };
     if (n_act <= 32) share_rows();
-    while (n_act > 0) {
-        // the active row of the lowest original index starts the search
-        int c0;
-        {
-            const bool first = TWO == 1 || om[0] != 0ull;
-            const int o = first ? __builtin_ctzll(om[0]) : 64 + __builtin_ctzll(om[TWO - 1]);
-            const unsigned long long m0 = __ballot(orig[0] == o), m1 = TWO == 2 ? __ballot(orig[TWO - 1] == o) : 0ull;
-            c0 = (TWO == 1 || m0) ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
-        }
-        const uint32_t ck = colkey(c0);
-        int imax = ck ? 127 - (int)(ck & 127u) : c0;
-        const double akk = colval(c0);
-        double colmax = ck ? fabs(colval(imax)) : 0.0;
-        const double absakk = fabs(akk);
-        int kstep = 1, p = c0, kp = c0;
-        // A(p, p), A(kp, kp) and, for a 2x2 pivot, A(p, kp) as the search ends
-        double app = akk, akp = akk, apk = akk;
-        bool need_rook = absakk < alpha * colmax;
-        if (!need_rook && !(absakk > 0.0 || colmax > 0.0)) {
-            failed = true;  // zero column: singular (a search has colmax > 0)
-            break;
-        }
-        for (int it = 0; it < 2 * ROWS && need_rook; ++it) {
-            const uint32_t rk = colkey(imax);
-            const int ri = rk ? 127 - (int)(rk & 127u) : imax;
-            const double rowmax = rk ? fabs(colval(ri)) : 0.0;
-            const double aim = colval(imax);
-            const double aii = fabs(aim);
-            if (!(aii < alpha * rowmax)) {
-                kp = imax;
-                akp = aim;
-                need_rook = false;
-            } else if (p == ri || rowmax <= colmax || it == 2 * ROWS - 1) {
-                kp = imax;
-                kstep = 2;
-                akp = aim;
-                apk = colval(p);  // column imax holds A(p, imax)
-                need_rook = false;
-            } else {
-                p = imax;
-                app = aim;
-                colmax = rowmax;
-                imax = ri;
+    // S: the slots that hold active rows. Systems of more than 64 rows start with two; once
+    // 64 rows are left, the loop for one slot takes over, without the choices between them.
+    auto factorise = [&](auto SL) __attribute__((always_inline)) {
+        constexpr int S = decltype(SL)::value;
+        auto row_at = [&](int c) __attribute__((always_inline)) -> int {
+            if constexpr (S == 2) return rb_of(c);
+            else return rdlane(rbj[0], c);
+        };
+        // Column c (uniform) of the active block to this lane's registers (v[t] = A(j, c)
+        // for its positions j < n_act: row j's entry if c <= j, else row c's entry j), and
+        // the largest |A(j, c)| over active j != c as a packed (magnitude, position) key.
+        double v[S];
+        auto colkey = [&](int c) -> uint32_t {
+            const int cc = __builtin_amdgcn_readfirstlane(c);
+            const int rbc = row_at(cc);
+            uint32_t k = 0u;
+#pragma unroll
+            for (int t = 0; t < S; ++t) {
+                const int j = L + 64 * t;
+                unsigned long long m = bits(n_act, t);
+                if (S == 1 || cc >> 6 == t) m &= ~(1ull << (cc & 63));
+                // (lanes past the active rows read entry (0, cc) or of row cc, and are masked)
+                v[t] = T(j >= cc ? (j < n_act ? rbj[t] : 0) + 8 * cc : rbc + 8 * j);
+                k = max(k, lanes_in(m, row_key(v[t], j) & 0x7fffffffu));
             }
-        }
-        kstep = __builtin_amdgcn_readfirstlane(kstep);
-        const int p0 = __builtin_amdgcn_readfirstlane((kstep == 1) ? kp : p);
-        const int p1 = __builtin_amdgcn_readfirstlane(kp);  // equals p0 for a 1x1 pivot
-        // A(p0, p0), A(p1, p1), A(p0, p1)
-        const double d0 = kstep == 1 ? akp : app, d1 = akp, bq = kstep == 1 ? akp : apk;
-        double idet = 0.0;
-        if (kstep == 1) {
-            failed = d0 == 0.0;
-        } else {
-            const double det = d0 * d1 - bq * bq;
-            failed = det == 0.0;
-            idet = 1.0 / det;
-        }
-        if (failed) break;
-        // p0 to position n_act - 1, p1 (2x2) to n_act - 2
-        double v0[RC], v1[RC];
-        const int q0 = n_act - 1, r0 = freeze(p0, q0, v0);
-        int r1 = r0;
+            return first_max_u32(k, n_act);
+        };
+        auto colval = [&](int r) -> double {
+            const int rr = __builtin_amdgcn_readfirstlane(r);
+            return (S == 2 && rr >= 64) ? rdlane(v[S - 1], rr & 63) : rdlane(v[0], rr & 63);
+        };
+        // symmetric swap of positions lo <= hi (both active): the rows and the columns, for
+        // every row of the system (frozen rows keep their entries at the active positions);
+        // each entry of the lower triangle that moves is moved by exactly one lane: lane k
+        // swaps (k, lo) with (k, hi), lane lo the diagonal entries, lane hi nothing
+        auto swap_entries = [&](int lo, int hi, int rhi) {
+            const int rlo = row_at(lo);
 #pragma unroll
-        for (int c = 0; c < RC; ++c) v1[c] = 0.0;
-        if (kstep == 2) {
-            r1 = freeze(p1 == q0 ? p0 : p1, q0 - 1, v1);
-            const unsigned long long bit = 1ull << ((q0 - 1) & 63);
-            twos[0] |= TWO == 1 || q0 - 1 < 64 ? bit : 0ull;
-            if (TWO == 2) twos[TWO - 1] |= q0 - 1 < 64 ? 0ull : bit;
-        }
-        n_act -= kstep;
-        if (n_act <= 32 && !shared) share_rows();
-        // The trailing update of the active rows j < n_act over their columns 0..j, eight at a
-        // time (the chunk past the diagonal lands in the row's padding), and of their
-        // right-hand sides; per element the FMAs run in the same order as in k_build_wide. The
-        // pivot row's eight entries are one read, spread over the lanes and broadcast by the
-        // FMAs. Every lane reads and multiplies (lanes without a row: row 0), those whose
-        // chunk lies in their row write.
-        const int na = TWO == 2 ? min(n_act, 64) : n_act;
-        const bool on = jr < na;
-        const int row = on ? rbu : 0;
-        auto update = [&](auto KS) __attribute__((always_inline)) {
-            constexpr int K = decltype(KS)::value;
-            auto factors = [&](int j, double& ml0, double& ml1) __attribute__((always_inline)) {
-                const double u0 = T(r0 + 8 * j);
-                double l0, l1 = 0.0;
-                if (K == 1) {
-                    l0 = u0 / d0;
-                } else {
-                    const double u1 = T(r1 + 8 * j);
-                    l0 = (u0 * d1 - u1 * bq) * idet;
-                    l1 = (u1 * d0 - u0 * bq) * idet;
-                }
-                ml0 = -l0;
-                ml1 = -l1;
-            };
-            double ml0, ml1;
-            factors(jr, ml0, ml1);
-            auto chunk = [&](int A, int W, int cc) __attribute__((always_inline)) {
-                double a[8], w1 = 0.0;
-                const double w0 = T(r0 + W);
-                if (K == 2) w1 = T(r1 + W);
-#pragma unroll
-                for (int q = 0; q < 8; ++q) a[q] = T(A + 8 * q);
-                fma8_row(a, w0, ml0);
-                if (K == 2) fma8_row(a, w1, ml1);
-                if (on && cc <= jr) {
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) T(A + 8 * q) = a[q];
-                }
-            };
-            if (n_act <= 32) {
-                if (n_act > 0) chunk(row + cadd8, wlane + cadd8, cadd);
-                if (n_act > 16) chunk(row + cadd8 + 128, wlane + cadd8 + 128, cadd + 16);
-            } else {
-                for (int cc = 0; cc < na; cc += 8) chunk(row + 8 * cc, wlane + 8 * cc, cc);
-            }
-#pragma unroll
-            for (int c = 0; c < RC; ++c) {
-                const double b = K == 1 ? fma(ml0, v0[c], bcol[c][0]) : fma(ml1, v1[c], fma(ml0, v0[c], bcol[c][0]));
-                bcol[c][0] = L < na ? b : bcol[c][0];
-            }
-            if constexpr (TWO == 2) {
-                // rows 64.. (the first steps of a system of more than 64 rows)
-                const int j = L + 64;
-                if (j < n_act) {
-                    factors(j, ml0, ml1);
-                    for (int j0 = 0; j0 <= j; j0 += 8) {
-#pragma unroll
-                        for (int q = 0; q < 8; ++q) {
-                            const int o = 8 * (j0 + q);
-                            const double a0 = fma(ml0, T(r0 + o), T(rbj[1] + o));
-                            T(rbj[1] + o) = K == 1 ? a0 : fma(ml1, T(r1 + o), a0);
-                        }
-                    }
-#pragma unroll
-                    for (int c = 0; c < RC; ++c)
-                        bcol[c][1] = K == 1 ? fma(ml0, v0[c], bcol[c][1])
-                                             : fma(ml1, v1[c], fma(ml0, v0[c], bcol[c][1]));
-                }
+            for (int t = 0; t < TWO; ++t) {
+                const int k = L + 64 * t;
+                if (k >= n || k == hi) continue;
+                const int k8 = 8 * k;
+                const int x0 = k >= lo ? rbj[t] + 8 * lo : rlo + k8;
+                const int x1 = k > hi ? rbj[t] + 8 * hi : rhi + (k == lo ? 8 * hi : k8);
+                const double y0 = T(x0), y1 = T(x1);
+                T(x0) = y1;
+                T(x1) = y0;
             }
         };
-        if (kstep == 1) update(std::integral_constant<int, 1>{});
-        else update(std::integral_constant<int, 2>{});
-        __syncthreads();
-    }
+        auto lane_put = [&](auto& w, auto v_, int p) __attribute__((always_inline)) {
+            if constexpr (S == 2) {
+                const auto w0 = w[0], w1 = w[1];  // (by value: a choice of elements would go to memory)
+                w[0] = p < 64 ? wrlane(w0, v_, p & 63) : w0;
+                w[1] = p < 64 ? w1 : wrlane(w1, v_, p & 63);
+            } else {
+                w[0] = wrlane(w[0], v_, p);
+            }
+        };
+        auto lane_get = [&](const auto& w, int p) __attribute__((always_inline)) {
+            const auto w0 = w[0], w1 = w[S - 1];
+            const auto a0 = rdlane(w0, p & 63);
+            if constexpr (S == 2) return p < 64 ? a0 : rdlane(w1, p & 63);
+            else return a0;
+        };
+        // The pivot of position p goes to the last active position q: its row start rq is
+        // returned, its right-hand sides in vq.
+        auto freeze = [&](int p, int q, double(&vq)[RC]) __attribute__((always_inline)) -> int {
+            const int rq = row_at(q), o = lane_get(orig, p);
+            if (TWO == 2 && o >= 64) om[TWO - 1] &= ~(1ull << (o & 63));
+            else om[0] &= ~(1ull << (o & 63));
+#pragma unroll
+            for (int c = 0; c < RC; ++c) vq[c] = lane_get(bcol[c], p);
+            if (p != q) {
+                swap_entries(p, q, rq);
+                lane_put(orig, lane_get(orig, q), p);
+                lane_put(orig, o, q);
+#pragma unroll
+                for (int c = 0; c < RC; ++c) {
+                    lane_put(bcol[c], lane_get(bcol[c], q), p);
+                    lane_put(bcol[c], vq[c], q);
+                }
+            }
+            return rq;
+        };
+        while (n_act > (S == 2 ? 64 : 0)) {
+            // the active row of the lowest original index starts the search
+            int c0;
+            {
+                const bool first = TWO == 1 || om[0] != 0ull;
+                const int o = first ? __builtin_ctzll(om[0]) : 64 + __builtin_ctzll(om[TWO - 1]);
+                const unsigned long long m0 = __ballot(orig[0] == o), m1 = S == 2 ? __ballot(orig[S - 1] == o) : 0ull;
+                c0 = (S == 1 || m0) ? __builtin_ctzll(m0) : 64 + __builtin_ctzll(m1);
+            }
+            const uint32_t ck = colkey(c0);
+            int imax = ck ? 127 - (int)(ck & 127u) : c0;
+            const double akk = colval(c0);
+            double colmax = ck ? fabs(colval(imax)) : 0.0;
+            const double absakk = fabs(akk);
+            int kstep = 1, p = c0, kp = c0;
+            // A(p, p), A(kp, kp) and, for a 2x2 pivot, A(p, kp) as the search ends
+            double app = akk, akp = akk, apk = akk;
+            bool need_rook = absakk < alpha * colmax;
+            if (!need_rook && !(absakk > 0.0 || colmax > 0.0)) {
+                failed = true;  // zero column: singular (a search has colmax > 0)
+                break;
+            }
+            for (int it = 0; it < 2 * ROWS && need_rook; ++it) {
+                const uint32_t rk = colkey(imax);
+                const int ri = rk ? 127 - (int)(rk & 127u) : imax;
+                const double rowmax = rk ? fabs(colval(ri)) : 0.0;
+                const double aim = colval(imax);
+                const double aii = fabs(aim);
+                if (!(aii < alpha * rowmax)) {
+                    kp = imax;
+                    akp = aim;
+                    need_rook = false;
+                } else if (p == ri || rowmax <= colmax || it == 2 * ROWS - 1) {
+                    kp = imax;
+                    kstep = 2;
+                    akp = aim;
+                    apk = colval(p);  // column imax holds A(p, imax)
+                    need_rook = false;
+                } else {
+                    p = imax;
+                    app = aim;
+                    colmax = rowmax;
+                    imax = ri;
+                }
+            }
+            kstep = __builtin_amdgcn_readfirstlane(kstep);
+            const int p0 = __builtin_amdgcn_readfirstlane((kstep == 1) ? kp : p);
+            const int p1 = __builtin_amdgcn_readfirstlane(kp);  // equals p0 for a 1x1 pivot
+            // A(p0, p0), A(p1, p1), A(p0, p1)
+            const double d0 = kstep == 1 ? akp : app, d1 = akp, bq = kstep == 1 ? akp : apk;
+            double idet = 0.0;
+            if (kstep == 1) {
+                failed = d0 == 0.0;
+            } else {
+                const double det = d0 * d1 - bq * bq;
+                failed = det == 0.0;
+                idet = 1.0 / det;
+            }
+            if (failed) break;
+            // p0 to position n_act - 1, p1 (2x2) to n_act - 2
+            double v0[RC], v1[RC];
+            const int q0 = n_act - 1, r0 = freeze(p0, q0, v0);
+            int r1 = r0;
+#pragma unroll
+            for (int c = 0; c < RC; ++c) v1[c] = 0.0;
+            if (kstep == 2) {
+                r1 = freeze(p1 == q0 ? p0 : p1, q0 - 1, v1);
+                const unsigned long long bit = 1ull << ((q0 - 1) & 63);
+                twos[0] |= S == 1 || q0 - 1 < 64 ? bit : 0ull;
+                if (S == 2) twos[S - 1] |= q0 - 1 < 64 ? 0ull : bit;
+            }
+            n_act -= kstep;
+            if (n_act <= 32 && !shared) share_rows();
+            // The trailing update of the active rows j < n_act over their columns 0..j, eight at a
+            // time (the chunk past the diagonal lands in the row's padding), and of their
+            // right-hand sides; per element the FMAs run in the same order as in k_build_wide. The
+            // pivot row's eight entries are one read, spread over the lanes and broadcast by the
+            // FMAs. Every lane reads and multiplies (lanes without a row: row 0), those whose
+            // chunk lies in their row write.
+            const int na = S == 2 ? min(n_act, 64) : n_act;
+            const bool on = jr < na;
+            const int row = on ? rbu : 0;
+            auto update = [&](auto KS) __attribute__((always_inline)) {
+                constexpr int K = decltype(KS)::value;
+                auto factors = [&](int j, double& ml0, double& ml1) __attribute__((always_inline)) {
+                    const double u0 = T(r0 + 8 * j);
+                    double l0, l1 = 0.0;
+                    if (K == 1) {
+                        l0 = u0 / d0;
+                    } else {
+                        const double u1 = T(r1 + 8 * j);
+                        l0 = (u0 * d1 - u1 * bq) * idet;
+                        l1 = (u1 * d0 - u0 * bq) * idet;
+                    }
+                    ml0 = -l0;
+                    ml1 = -l1;
+                };
+                double ml0, ml1;
+                factors(jr, ml0, ml1);
+                auto chunk = [&](int A, int W, int cc) __attribute__((always_inline)) {
+                    double a[8], w1 = 0.0;
+                    const double w0 = T(r0 + W);
+                    if (K == 2) w1 = T(r1 + W);
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) a[q] = T(A + 8 * q);
+                    fma8_row(a, w0, ml0);
+                    if (K == 2) fma8_row(a, w1, ml1);
+                    if (on && cc <= jr) {
+#pragma unroll
+                        for (int q = 0; q < 8; ++q) T(A + 8 * q) = a[q];
+                    }
+                };
+                if (n_act <= 32) {
+                    if (n_act > 0) chunk(row + cadd8, wlane + cadd8, cadd);
+                    if (n_act > 16) chunk(row + cadd8 + 128, wlane + cadd8 + 128, cadd + 16);
+                } else {
+                    for (int cc = 0; cc < na; cc += 8) chunk(row + 8 * cc, wlane + 8 * cc, cc);
+                }
+#pragma unroll
+                for (int c = 0; c < RC; ++c) {
+                    const double b0 = fma(ml0, v0[c], bcol[c][0]);
+                    const double b = K == 1 ? b0 : fma(ml1, v1[c], b0);
+                    bcol[c][0] = L < na ? b : bcol[c][0];
+                }
+                if constexpr (S == 2) {
+                    // rows 64.. (the first steps of a system of more than 64 rows)
+                    const int j = L + 64;
+                    if (j < n_act) {
+                        factors(j, ml0, ml1);
+                        for (int j0 = 0; j0 <= j; j0 += 8) {
+#pragma unroll
+                            for (int q = 0; q < 8; ++q) {
+                                const int o = 8 * (j0 + q);
+                                const double a0 = fma(ml0, T(r0 + o), T(rbj[1] + o));
+                                T(rbj[1] + o) = K == 1 ? a0 : fma(ml1, T(r1 + o), a0);
+                            }
+                        }
+#pragma unroll
+                        for (int c = 0; c < RC; ++c)
+                            bcol[c][1] = K == 1 ? fma(ml0, v0[c], bcol[c][1])
+                                                 : fma(ml1, v1[c], fma(ml0, v0[c], bcol[c][1]));
+                    }
+                }
+            };
+            if (kstep == 1) update(std::integral_constant<int, 1>{});
+            else update(std::integral_constant<int, 2>{});
+            __syncthreads();
+        }
+    };
+    if constexpr (TWO == 2) factorise(std::integral_constant<int, 2>{});
+    if (!failed) factorise(std::integral_constant<int, 1>{});
     __syncthreads();
 
     // ---- back substitution, last pivot (position 0) first: the rows frozen before a pivot
@@ -1367,6 +1380,12 @@ __global__ __attribute__((amdgpu_flat_work_group_size(64, 64))) void k_build_sym
         }
         if (!failed && j < n) dinv[t] = 1.0 / T(rbj[t] + 8 * j);
     }
+    auto lane_get = [&](const auto& w, int p) __attribute__((always_inline)) {
+        const auto w0 = w[0], w1 = w[TWO - 1];
+        const auto a0 = rdlane(w0, p & 63);
+        if constexpr (TWO == 2) return p < 64 ? a0 : rdlane(w1, p & 63);
+        else return a0;
+    };
     if (!failed) {
         for (int pq = 0; pq < n;) {
             const bool two = ((TWO == 1 || pq < 64 ? twos[0] : twos[TWO - 1]) >> (pq & 63)) & 1ull;
