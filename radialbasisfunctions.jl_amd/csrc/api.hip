@@ -192,8 +192,9 @@ __global__ void k_set_i32(int32_t* p, int32_t v) { *p = v; }
 // Lists of an uneven build, in processing order: the size buckets n = k + m <= 32, <= 64,
 // above, and the null-space classes (a stencil of a class is in its class's list only).
 // counts: [0..2] bucket lists, [kTotals..] stencils of each size whatever their list,
-// [kClasses..] class lists. One atomic per list and workgroup (one per
-// wavefront serialises on the list's count: 254 us for 1.3M stencils, now 39), and the lists keep the order of 1,024 stencils.
+// [kClasses..] class lists. One atomic per list and workgroup (one per wavefront serialises
+// on the list's count: 254 us for 1.3M stencils, now 39); the lists keep the order of 1,024
+// stencils.
 constexpr int kSamples = 3, kTotals = 8, kClasses = 16, kCounts = 32;
 struct ClassTab {
     int n;
@@ -1105,6 +1106,7 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         P.fail_list = ds.fail_list;
         P.fail_count = ds.fail_count;
         int64_t n_solve = a->n_eval;
+        bool fp32_ran = true;  // (a kernel that factorises in FP32)
         if (a->precision == RBFX_PREC_LEARNED) {
             // surrogate + FP64 acceptance; the rejected stencils go to the solver
             if (!async) {
@@ -1174,7 +1176,13 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
             }
             g_bucket_n[b] = async ? -1 : n_solve;
             g_bucket_kernel[b] = kid;
-            if (n_solve > 0) HIPCHK(launch_kernel_id(kid, Q, sh, hb, b, true, nmax, n_solve, async, st));
+            // (a blocking build reads the null-space kernels' hand-backs with its report, and an
+            // FP64 kernel leaves nothing to re-solve: two round trips less)
+            const bool defer = !async && is_nsc(kid);
+            const HandBack hl = defer ? HandBack{ds.nsc_list, (int32_t*)(ds.hist + 17)} : hb;
+            if (n_solve > 0)
+                HIPCHK(launch_kernel_id(kid, Q, sh, hl, b, true, nmax, n_solve, async, st, defer ? &df : nullptr));
+            fp32_ran = n_solve > 0 && (kid == K_REG32 || kid == K_REG64);
         } else {
             const int rc = solve_all(a, P, sh, ds, nmax, true, mode, nullptr, st);
             if (rc != RBFX_OK) return rc;
@@ -1184,7 +1192,8 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         HIPCHK(mark(2));
         // FP64 re-solve of the stencils whose refinement did not converge
         int32_t nfail = (int32_t)a->n_eval;
-        if (!async) HIPCHK(read_count(ds.fail_count, &nfail, st));
+        if (!async && fp32_ran) HIPCHK(read_count(ds.fail_count, &nfail, st));
+        if (!fp32_ran) nfail = 0;
         rbfx::BuildDev F = P;
         F.fail_list = nullptr;
         F.fail_count = nullptr;
@@ -1221,7 +1230,12 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
         hipLaunchKernelGGL(k_set_i32, dim3(1), dim3(1), 0, st, handed, nf);
         HIPCHK(launch_kernel_id(rook_for(df.bucket, df.F.n_cols), df.F, sh, HandBack{ds.nsc_list, handed}, df.bucket,
                                 false, df.rows_cap, nf, false, st));
-        HIPCHK(mark(1));
+        if (plain) {
+            HIPCHK(mark(1));
+        } else {
+            HIPCHK(mark(2));
+            HIPCHK(mark(3));
+        }
         HIPCHK(report(handed));
     }
     ds.report_clean = true;

@@ -28,9 +28,9 @@
 // Bound by FP64 VALU issue; VGPRs (the instantiation's W waves per SIMD) and LDS
 // (NseLds) set how many wavefronts hide the LU's serial chain of pivots. Measured against
 // the kernels that served these builds before: 4M-point 2-D Laplacian (PHS3, degree 2,
-// k = 20) 12.06 -> 3.14 ms per build (null-space Cholesky, 8 lanes of three rows; 436
+// k = 20) 12.06 -> 3.09 ms per build (null-space Cholesky, 8 lanes of three rows; 386
 // VALU instructions per stencil against 897), 2M-point 3-D gradient and Laplacian (PHS5,
-// degree 3, k = 40) 149.6 -> 11.8 ms (rook LDL^T in LDS; 2,400 against 21,800).
+// degree 3, k = 40) 149.6 -> 11.8 ms (rook LDL^T in LDS; 2,320 against 21,800).
 //
 // Breakdown: an LU pivot below kNseLuTol (scaled coordinates, monomials of order one), or
 // a pivot of S below kNsePivTol of the largest one so far (the weights then carry more

@@ -278,3 +278,32 @@ def test_mlp_pass_at_tile_edges(RBF, gpu, M, shift):
         n, k = MO.n_of(l), MO.k_of(l)
         for o, c in ((MO.w_off(l), n * k), (MO.b_off(l), n)):
             assert _rel(g[o:o + c], g_ref[o:o + c]) < 2e-2, (l, c)
+
+
+def test_learned_build_hands_back_to_rook(RBF, gpu):
+    """A strip 1e-6 wide: its stencils (radius about 10/1500) have y^2 below 1e-7 of their
+    radius squared, under the elimination kernel's pivot tolerance of 1e-6. They come back
+    with the report and run on the rook kernel, with the weights of the plain build (the
+    same kernels), and the next build starts clean."""
+    import torch
+
+    rng = np.random.default_rng(8)
+    thin = rng.random((1500, 2)) * np.array([1.0, 1e-6]) + np.array([5.0, 5.0])
+    pts = np.concatenate([RBF.learned.density_cloud(4500, 12), thin])
+    model = RBF.learned.LearnedModel.initial(seed=3, device=gpu)
+    model.accept_tol = 1e-30  # every stencil to the solver
+    kw = dict(basis=RBF.PHS(3, poly_deg=2), k=20, device=gpu)
+    RBF._lib.tune_bucket(0, 8)  # (the elimination kernel for both)
+    try:
+        plain = RBF.laplacian(pts, **kw)
+        handed = RBF._lib.last_build_stats()[0]
+        assert handed > 0
+        op = RBF.laplacian(pts, precision="learned", model=model, **kw)
+        for _ in range(2):
+            assert RBF._lib.last_build_stats()[0] == handed
+            assert op.status_counts[RBF._abi.ST_FP64] == len(pts)
+            assert torch.equal(op.vals, plain.vals)
+            op.vals.zero_()
+            op.update_weights()
+    finally:
+        RBF._lib.tune_bucket(0, -1)
