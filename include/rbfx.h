@@ -77,6 +77,11 @@ enum {
     RBFX_PREC_LEARNED = 2        /* MLP surrogate, FP64 residual acceptance,
                                     FP32_REFINED fallback (needs a loaded model)    */
 };
+/* May be OR'd to a mode: the caller rounds the weights to FP32. FP64 weights of different
+ * kernels agree to some units of their last places, which is enough to move an FP32
+ * rounding here and there; such builds keep to kernels 0..7 (rbfx_tune_bucket), and those
+ * of one stencil size take the one of their shape, never one that a timing picks.    */
+enum { RBFX_WEIGHTS_F32 = 16 };
 
 /* ---- per-stencil status codes (written to args.status) ------------------ */
 enum {
@@ -149,7 +154,7 @@ typedef struct rbfx_build_args {
     double* out_val;             /* n_cols * out_nnz, column c at out_val + c*out_nnz */
     int64_t out_nnz;
     int32_t* status;             /* n_eval per-stencil status, or NULL                */
-    int32_t precision;           /* RBFX_PREC_*                                       */
+    int32_t precision;           /* RBFX_PREC_*, with RBFX_WEIGHTS_F32 or without      */
     int32_t refine_steps;        /* FP32_REFINED: refinement updates (0 -> 3)         */
     double accept_tol;           /* relative residual tolerance (0 -> default)        */
     void* stream;                /* hipStream_t, NULL = default stream                */
@@ -371,15 +376,16 @@ int rbfx_last_build_buckets(int64_t n[3], int32_t kernel[3]);
  * more wavefronts per CU); 8 null-space elimination in registers, 16 lanes per stencil
  * (interior stencils of uniform builds: PHS3, PHS5 and PHS7 definite as for 5, in 2-D up
  * to degree 4 and 3 operator columns, in 3-D up to degree 3 and 6 columns, at most 26
- * points beyond the monomials, no multipliers; the stencils whose pivots fail are re-solved
- * by kernel 0 or 7). A pinned kernel that cannot serve a build is ignored by that build. */
+ * points beyond the monomials, no multipliers, no RBFX_WEIGHTS_F32; the stencils whose
+ * pivots fail are re-solved by kernel 0 or 7). A pinned kernel that cannot serve a build is ignored by that build. */
 int rbfx_tune_bucket(int32_t bucket, int32_t kernel);
 
 /* Counters of the last rbfx_build_weights on this thread (no reference counterpart):
  * [0] stencils the null-space kernels handed to the rook kernels (breakdown, refinement
  * not settling, Hermite or out-of-shape stencils), [1] autotuner sample launches, [2]
  * the launch plan of an uneven build (1 one launch per size bucket, 2 one launch for
- * all stencils; 0 for a build of one size), the rest 0.                          */
+ * all stencils; 0 for a build of one size), [3] stencils of an uneven build solved by
+ * kernel 8 (-1: not read back), the rest 0.                                      */
 int rbfx_last_build_stats(int64_t stats[8]);
 
 /* Pin the launch plan of uneven builds (ragged k or a degree map) for later builds in

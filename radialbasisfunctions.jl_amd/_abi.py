@@ -32,6 +32,7 @@ OP_LAP = 4
 PREC_FP64 = 0
 PREC_FP32_REFINED = 1
 PREC_LEARNED = 2
+WEIGHTS_F32 = 16  # (OR'd to a mode: the caller rounds the weights to FP32)
 
 # per-stencil status
 ST_OK = 0

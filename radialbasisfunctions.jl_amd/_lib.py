@@ -214,7 +214,8 @@ def tune_bucket(bucket, kernel):
 def last_build_stats():
     """[stencils the null-space kernels handed to the rook kernels, autotuner sample
     launches, launch plan of an uneven build (1 per bucket, 2 one launch; 0 one size),
-    0, ...] of the last build on this thread."""
+    stencils of an uneven build that kernel 8 solved (-1: not read back), 0, ...] of the
+    last build on this thread."""
     st = (C.c_int64 * 8)()
     _check(lib().rbfx_last_build_stats(st))
     return list(st)

@@ -399,6 +399,8 @@ struct Shape {
     bool hermite;
     bool uniform;  // every stencil has k points and m monomials (no ragged k, no degree map)
     bool lambda;   // the caller wants the multipliers too
+    bool f32;      // the caller rounds the weights to FP32 (RBFX_WEIGHTS_F32)
+    bool no_nse() const { return lambda || f32; }  // kernel 8 and its classes keep out
 };
 
 static bool is_nsc(int kid) { return kid == K_NSC || kid == K_NSC2 || kid == K_NSE; }
@@ -425,7 +427,7 @@ static bool kernel_serves(int kid, int bucket, bool fp32, const Shape& sh, bool 
         return rbfx::nsc_fits(sh.dim, kb, sh.m, sh.n_cols, kid == K_NSC2 ? 1 : 0);
     }
     case K_NSE:
-        return sh.uniform && !sh.lambda && rbfx::nsc_sign(sh.basis_kind, sh.poly_deg) != 0 &&
+        return sh.uniform && !sh.no_nse() && rbfx::nsc_sign(sh.basis_kind, sh.poly_deg) != 0 &&
                sh.kmax + sh.m <= (bucket == 0 ? 32 : (bucket == 1 ? 64 : RBFX_MAX_N)) &&
                rbfx::nse_fits(sh.basis_kind, sh.dim, sh.kmax, sh.m, sh.n_cols);
     default: return false;
@@ -500,6 +502,23 @@ static hipError_t launch_kernel_id(int kid, const rbfx::BuildDev& P, const Shape
     return rbfx::launch_build(Q, sh.dim, (kid == K_REG32 || kid == K_REG32_F64) ? 32 : 64, f32, n_work, st);
 }
 
+// Kernel of a uniform build whose weights are rounded to FP32, by its shape: a timing that
+// falls the other way would move roundings. These are the kernels that such builds were
+// timed to before kernel 7 took half its time (100,000 stencils and more; the smaller ones
+// were timed to kernel 7 or to these): one column on the null-space Cholesky kernels except
+// in 3-D beyond four monomials; several columns up to 32 rows on the rook register kernel
+// in 2-D, and on kernel 7 in 3-D, for PHS7 and where the degree does not make the basis
+// definite. The price, Hessian, PHS5, degree 3, k = 20, 120,001 stencils: 2.29 ms; kernel 7
+// takes 1.47 and kernel 8 0.17, and 1 in 10,000 FP32 outputs then differs.
+static int f32_kernel(const Shape& sh, int bucket, bool fp32, int dflt)
+{
+    const bool definite = rbfx::nsc_sign(sh.basis_kind, sh.poly_deg) != 0;
+    const int sym = kernel_serves(K_SYM, bucket, fp32, sh, false) ? K_SYM : dflt;
+    if (sh.n_cols == 1) return is_nsc(dflt) && !(sh.dim == 3 && sh.m > 4) ? dflt : sym;
+    if (bucket == 0 && sh.dim == 2 && definite && sh.basis_kind != RBFX_PHS7) return fp32 ? K_REG32_F64 : K_REG32;
+    return sym;
+}
+
 // Kernel for a size bucket: forced (rbfx_tune_bucket), cached for this configuration,
 // or timed on a sample of the bucket's stencils (the autotuner: each kernel that serves
 // the bucket runs the sample twice, the second run timed; the fastest is kept), or the
@@ -531,8 +550,9 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
                       sh.uniform ? 1 : 0};
     // a cached or loaded choice is used only where that kernel serves this build
     // (looked up, never inserted, by a build that allocates nothing)
+    const bool by_shape = sh.f32 && sh.uniform;
     auto it = ds.tuned.find(key);
-    if (it != ds.tuned.end() && kernel_serves(it->second, bucket, fp32, sh, false)) {
+    if (!by_shape && it != ds.tuned.end() && kernel_serves(it->second, bucket, fp32, sh, false)) {
         *kid = it->second;
         return RBFX_OK;
     }
@@ -540,6 +560,10 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
     if (jt != g_tune_saved.end() && kernel_serves(jt->second, bucket, fp32, sh, false)) {
         if (mode != Mode::kNoAlloc) ds.tuned[key] = jt->second;
         *kid = jt->second;
+        return RBFX_OK;
+    }
+    if (by_shape) {
+        if (count >= kTuneMin) *kid = f32_kernel(sh, bucket, fp32, dflt);
         return RBFX_OK;
     }
     if (async || count < kTuneMin) return RBFX_OK;
@@ -692,7 +716,7 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
     ClassTab tab;
     tab.n = 0;
     const bool pinned = g_force_plan != 0 || g_force_kernel[0] >= 0 || g_force_kernel[1] >= 0 || g_force_kernel[2] >= 0;
-    if (uneven && !pinned && !sh.lambda && mode != Mode::kNoAlloc)
+    if (uneven && !pinned && !sh.no_nse() && mode != Mode::kNoAlloc)
         tab.n = rbfx::nse_classes(sh.basis_kind, dim, sh.poly_deg, sh.n_cols, tab.c);
     // (an asynchronous build uses what an earlier blocking one made room for)
     if (async && (!ds.bucket_count || ds.cap_bucket < sizeof(int32_t) * (3 + tab.n) * (size_t)a->n_eval)) tab.n = 0;
@@ -865,8 +889,12 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
     if (tab.n > 0) {
         if ((rc = run_classes()) != RBFX_OK) return rc;
         if ((rc = read_counts()) != RBFX_OK) return rc;  // (with what they handed back)
-        if (!async)
-            for (int b = 0; b < 3; ++b) g_stats[0] += cnt[b] - listed[b];
+        g_stats[3] = async ? -1 : 0;
+        for (int c = 0; !async && c < tab.n; ++c) g_stats[3] += cnt[kClasses + c];
+        for (int b = 0; !async && b < 3; ++b) {
+            g_stats[0] += cnt[b] - listed[b];
+            g_stats[3] -= cnt[b] - listed[b];
+        }
     }
     if (!timing)
         for (int b = 0; b < 3; ++b) {
@@ -904,10 +932,13 @@ static int scratch_area(int32_t** out)
     return RBFX_OK;
 }
 
-static int build_impl(const rbfx_build_args* a, Mode mode)
+static int build_impl(const rbfx_build_args* args, Mode mode)
 {
     const bool async = mode != Mode::kBlocking;
-    if (!a) return set_err(RBFX_EINVAL, "rbfx_build_weights: null args");
+    if (!args) return set_err(RBFX_EINVAL, "rbfx_build_weights: null args");
+    rbfx_build_args plain_args = *args;  // (the precision without its flag)
+    plain_args.precision &= ~RBFX_WEIGHTS_F32;
+    const rbfx_build_args* a = &plain_args;
     for (int i = 0; i < 16; ++i) g_counts[i] = 0;
     for (int i = 0; i < 4; ++i) g_stage_ms[i] = 0.0;
     for (int i = 0; i < 8; ++i) g_stats[i] = 0;
@@ -1079,6 +1110,7 @@ static int build_impl(const rbfx_build_args* a, Mode mode)
     sh.hermite = a->is_boundary != nullptr;
     sh.uniform = !a->adj_ptr && !a->poly_deg_map;
     sh.lambda = a->out_lambda != nullptr;
+    sh.f32 = (args->precision & RBFX_WEIGHTS_F32) != 0;
     // stage boundaries: ev0 | main kernel | ev1 | FP32 list solve | ev2 | FP64 fallback | ev3
     // (blocking builds only; an asynchronous build records nothing but kernels)
     auto mark = [&](int i) -> hipError_t {
@@ -1307,7 +1339,7 @@ int rbfx_tune_bucket(int32_t bucket, int32_t kernel)
     if (kernel >= 0) {
         // a kernel that can serve the bucket for some configuration (a pinned kernel that
         // cannot serve a particular build is ignored by that build)
-        Shape any{2, 20, 6, 1, RBFX_PHS3, 2, false, true, false};
+        Shape any{2, 20, 6, 1, RBFX_PHS3, 2, false, true, false, false};
         bool ok = false;
         for (int kmax : {20, 30, 40, 60})
             for (int fp32 = 0; fp32 < 2; ++fp32) {

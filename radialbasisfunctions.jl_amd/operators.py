@@ -597,7 +597,7 @@ class RadialBasisOperator:
         a.status = _lib.ptr(status)
         if self.precision not in PRECISIONS:
             raise ArgumentError(f"precision must be one of {sorted(PRECISIONS)}")
-        a.precision = PRECISIONS[self.precision]
+        a.precision = PRECISIONS[self.precision] | (abi.WEIGHTS_F32 if self.dtype == "float32" else 0)
         a.refine_steps = int(self.refine_steps)
         a.accept_tol = float(self.accept_tol)
         a.stream = _lib.stream_ptr(self.dev)
