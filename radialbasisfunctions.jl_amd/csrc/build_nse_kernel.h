@@ -33,8 +33,12 @@
 // degree 3, k = 40) 149.6 -> 11.8 ms (rook LDL^T in LDS; 2,320 against 21,800).
 //
 // Breakdown: an LU pivot below kNseLuTol (scaled coordinates, monomials of order one), or
-// a pivot of S below kNsePivTol of the largest one so far (the weights then carry more
-// than about u / kNsePivTol = 1e-7 of error), hands the stencil to the rook-pivoted kernels.
+// a pivot of S below kNsePivTol of the stencil's scale, hands the stencil to the rook-pivoted
+// kernels. The scale is the largest pivot so far and no less than the largest entry of T: the
+// entries of S are differences of products of T, so each carries an error of some u times it,
+// whatever they cancel to (a repeated point's pivot is that error alone, and a scale of the
+// pivots only would not see it in the first one). The weights accepted carry up to some
+// u / kNsePivTol = 1e-7 of error from the elimination.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -640,6 +644,21 @@ k_nse(const BuildDev P)
         });
     }
 
+    // the largest |T| of the null points (its leading bits; infinity, which no pivot passes, for a NaN)
+    double tscale;
+    {
+        uint32_t hi = 0;
+#pragma unroll
+        for (int t = 0; t < SLN; ++t)
+#pragma unroll
+            for (int a = 0; a < M; ++a) {
+                const uint32_t h = (uint32_t)((unsigned long long)__double_as_longlong(T[t][a]) >> 32) & 0x7fffffffu;
+                hi = max(hi, t == SLN - 1 && isg ? 0u : h);
+            }
+        hi = min(group_max_u32<16>(hi), 0x7ff00000u);
+        tscale = __longlong_as_double((long long)((unsigned long long)hi << 32));
+    }
+
     // ---- S = Phi_NN + T (-C)^T + (-C) T^T, and the same for the operator columns
     nse_for<NN>([&](auto j) RBFX_INL {
         RBFX_NSE_POINT(o, xn[j.value / 16], j.value % 16)
@@ -686,7 +705,7 @@ k_nse(const BuildDev P)
     for (int t = 0; t < SLN; ++t) dinv[t] = 0.0;
     {
         constexpr double sg = KIND == RBFX_PHS5 ? -1.0 : 1.0;  // (nsc_sign)
-        double dmax = 0.0;
+        double dmax = tscale;
         nse_for<NN>([&](auto jc) RBFX_INL {
             constexpr int j = jc.value, jt = j / 16, jl = j % 16, rest = NN - 1 - j;
             if (j < nnw) {

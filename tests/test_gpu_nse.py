@@ -172,3 +172,30 @@ def test_nse_classes_of_uneven_builds(RBF, O, gpu, kind, dim, degs, cols, kmax):
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(op.vals, eager)
+
+
+@pytest.mark.parametrize("where", ["front", "back", "apart"])
+@pytest.mark.parametrize("kind,dim,deg,nn,cols", [(3, 2, 1, 1, "grad"), (3, 2, 2, 1, "lap"), (3, 2, 2, 2, "lap"),
+                                                 (3, 2, 2, 3, "lap"), (3, 2, 2, 6, "hess"), (5, 2, 3, 1, "lap"),
+                                                 (5, 2, 3, 2, "grad"), (7, 2, 4, 1, "lap"), (3, 3, 2, 1, "lap"),
+                                                 (3, 3, 2, 2, "grad"), (5, 3, 3, 1, "lap"), (5, 3, 3, 2, "gradlap")])
+def test_nse_never_accepts_a_repeated_point(RBF, O, gpu, kind, dim, deg, nn, cols, where):
+    """Stencils of m + nn points, two of them the same point: singular systems, of which
+    rounding leaves pivots of either sign. Every one goes back to the rook kernel, which solves
+    or reports it, wherever the pair stands in the stencil and however few points there are."""
+    k = comb(dim + deg, dim) + nn
+    n = 901
+    pts = np.random.default_rng(13 * kind + deg + nn).random((n, dim))
+    near = O.knn(pts, pts, k - 1)
+    q = {"front": 0, "back": k - 2, "apart": (k - 1) // 2}[where]
+    twin = near[:, q:q + 1] + n
+    adj = np.concatenate([near[:, :1], twin, near[:, 1:]] if where == "front" else [near, twin], axis=1)
+    L, n_cols, terms = _operator(RBF, O, dim, cols)
+    with pinned(RBF, K_NSE):
+        try:
+            RBF.RadialBasisOperator(L, np.concatenate([pts, pts]), eval_points=pts, basis=RBF.PHS(kind, poly_deg=deg),
+                                    adjl=list(adj))
+        except RBF.SingularException:
+            pass
+    assert K_NSE in RBF._lib.last_build_buckets()[1]
+    assert RBF._lib.last_build_stats()[0] == n
