@@ -115,3 +115,30 @@ def test_weights_as_exact_as_the_replaced_kernels(RBF, O, gpu):
         print((kind, dim, deg, k, cols), "%.3f" % (e8 / eo))
         ratios.append(e8 / eo)
     assert np.exp(np.mean(np.log(ratios))) <= 1.0, ratios
+
+
+ALL = [(3, 2, 1, 12, "lap", 6), (3, 2, 2, 7, "lap", 6), (3, 2, 2, 12, "grad", 0), (3, 2, 2, 20, "lap", 6),
+       (3, 2, 2, 25, "lap", 5), (3, 2, 2, 32, "dx", 5), (5, 2, 2, 20, "lap", 6), (3, 3, 1, 12, "lap", 6),
+       (3, 3, 2, 20, "grad", 7)] + HIGH
+
+
+def test_polynomial_conditions_as_exact_as_the_replaced_kernels(RBF, O, gpu):
+    """Residual of P^T w = L P relative to the stencil's largest weight (what an applied operator
+    shows on a smooth field), root mean square over the stencils of a shape, kernel 8 over
+    the replaced kernel: at most 1 in the geometric mean over the shapes."""
+    ratios = []
+    for kind, dim, deg, k, cols, other in ALL:
+        pts, ev, adj, x, s = _stencils(O, dim, k, 7 * kind + k + len(cols))
+        P = _block(x.astype(np.longdouble), _monomials(dim, deg))
+        res = []
+        for kern in (K_NSE, other):
+            w = _weights(RBF, pts, ev, adj, kind, deg, _operator(RBF, dim, cols), kern).astype(np.longdouble)
+            r = []
+            for c, t in enumerate(_columns(dim, cols)):
+                wc = np.ldexp(w[c], s * (2 if t == "lap" else 1))
+                g = [2.0 * (sorted(e) == [0] * (dim - 1) + [2]) if t == "lap" else float(e == t) for e in _monomials(dim, deg)]
+                r.append(((P * wc[:, :, None]).sum(1) - g) / np.abs(wc).max(1)[:, None])
+            res.append(float(np.sqrt((np.array(r) ** 2).mean())))
+        print((kind, dim, deg, k, cols), "%.3f" % (res[0] / res[1]))
+        ratios.append(res[0] / res[1])
+    assert np.exp(np.mean(np.log(ratios))) <= 1.0, ratios
