@@ -401,7 +401,8 @@ int rbfx_tune_plan(int32_t plan);
 
 /* Save / load the autotuner's choices (no reference counterpart; the checkpoint of
  * the tuning map): one text line per configuration (dimension, operator columns,
- * precision, size bucket, largest k, monomials, basis kind, boundary data, kernel).
+ * precision, size bucket, largest k, monomials, basis kind, boundary data, one shape,
+ * kernel; then a 1 for builds that keep out kernel 8, which would serve their shape).
  * A loaded choice is used instead of timing samples, on every device, for the
  * configurations it names.                                                       */
 int rbfx_tune_save(const char* path);

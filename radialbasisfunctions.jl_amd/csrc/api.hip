@@ -51,9 +51,10 @@ int set_err(int code, const char* fmt, ...)
 
 // Autotuner configuration key: dimension, operator columns, precision mode, size
 // bucket, largest stencil (k points, m monomials), basis kind, whether the build has
-// boundary data and whether every stencil has the same shape (no ragged k, no degree
-// map: the null-space kernels serve only such builds).
-typedef std::tuple<int, int, int, int, int, int, int, int, int> TuneKey;
+// boundary data, whether every stencil has the same shape (no ragged k, no degree
+// map: the null-space kernels serve only such builds), and whether the build keeps out
+// kernel 8, which would serve it (nse_kept_out).
+typedef std::tuple<int, int, int, int, int, int, int, int, int, int> TuneKey;
 
 // What a blocking build reports to the host, written by the device into pinned memory:
 // stencils per status, and how many the null-space kernel handed back.
@@ -434,6 +435,40 @@ static bool kernel_serves(int kid, int bucket, bool fp32, const Shape& sh, bool 
     }
 }
 
+// Whether kernel 8 (a bucket of a uniform build) or its classes (a plan) would serve this
+// build, did it not keep them out: its choices are then entries of their own, or a build
+// with multipliers would decide the kernel of the plain builds of its shape.
+static bool nse_kept_out(const Shape& sh, int bucket)
+{
+    if (!sh.no_nse()) return false;
+    rbfx::NseClass c[rbfx::kNseClasses];
+    if (bucket == kPlanKey) return rbfx::nse_classes(sh.basis_kind, sh.dim, sh.poly_deg, sh.n_cols, c) > 0;
+    Shape plain = sh;
+    plain.lambda = plain.f32 = false;
+    return kernel_serves(K_NSE, bucket, false, plain, false);
+}
+
+static TuneKey tune_key(const rbfx_build_args* a, const Shape& sh, int bucket, bool kept_out)
+{
+    return TuneKey{sh.dim,        sh.n_cols,          a->precision,       bucket,         sh.kmax, sh.m,
+                   sh.basis_kind, sh.hermite ? 1 : 0, sh.uniform ? 1 : 0, kept_out ? 1 : 0};
+}
+
+// The kernel kept for a bucket, or -1: timed in this process, else from a loaded map. A build
+// that keeps kernel 8 out goes by its own entries, then by the plain ones whose kernel serves it.
+static int kept_kernel(const rbfx_build_args* a, const Shape& sh, const DeviceState& ds, int bucket, bool fp32)
+{
+    const bool out = nse_kept_out(sh, bucket);
+    const std::map<TuneKey, int>* const maps[2] = {&ds.tuned, &g_tune_saved};
+    for (const auto* m : maps)
+        for (int o = out ? 1 : 0; o >= 0; --o) {
+            if (sh.f32 && sh.uniform && m == &ds.tuned) continue;  // (its shape's kernel, or a loaded map's)
+            const auto it = m->find(tune_key(a, sh, bucket, o != 0));
+            if (it != m->end() && kernel_serves(it->second, bucket, fp32, sh, false)) return it->second;
+        }
+    return -1;
+}
+
 // The rook kernel that re-solves what a null-space launch handed back (FP64).
 static int rook_for(int bucket, int n_cols)
 {
@@ -546,23 +581,14 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
         *kid = forced;
         return RBFX_OK;
     }
-    const TuneKey key{a->dim,         sh.n_cols, a->precision, bucket, sh.kmax, sh.m, sh.basis_kind, sh.hermite ? 1 : 0,
-                      sh.uniform ? 1 : 0};
     // a cached or loaded choice is used only where that kernel serves this build
-    // (looked up, never inserted, by a build that allocates nothing)
-    const bool by_shape = sh.f32 && sh.uniform;
-    auto it = ds.tuned.find(key);
-    if (!by_shape && it != ds.tuned.end() && kernel_serves(it->second, bucket, fp32, sh, false)) {
-        *kid = it->second;
+    const TuneKey key = tune_key(a, sh, bucket, nse_kept_out(sh, bucket));
+    const int kept = kept_kernel(a, sh, ds, bucket, fp32);
+    if (kept >= 0) {
+        *kid = kept;
         return RBFX_OK;
     }
-    auto jt = g_tune_saved.find(key);  // a map loaded with rbfx_tune_load
-    if (jt != g_tune_saved.end() && kernel_serves(jt->second, bucket, fp32, sh, false)) {
-        if (mode != Mode::kNoAlloc) ds.tuned[key] = jt->second;
-        *kid = jt->second;
-        return RBFX_OK;
-    }
-    if (by_shape) {
+    if (sh.f32 && sh.uniform) {
         if (count >= kTuneMin) *kid = f32_kernel(sh, bucket, fp32, dflt);
         return RBFX_OK;
     }
@@ -624,12 +650,7 @@ static bool would_time(const rbfx_build_args* a, const Shape& sh, const DeviceSt
 {
     if (count < kTuneMin || (g_force_kernel[bucket] >= 0 && kernel_serves(g_force_kernel[bucket], bucket, fp32, sh, true)))
         return false;
-    const TuneKey key{a->dim,         sh.n_cols, a->precision, bucket, sh.kmax, sh.m, sh.basis_kind, sh.hermite ? 1 : 0,
-                      sh.uniform ? 1 : 0};
-    auto it = ds.tuned.find(key);
-    if (it != ds.tuned.end() && kernel_serves(it->second, bucket, fp32, sh, false)) return false;
-    auto jt = g_tune_saved.find(key);
-    return !(jt != g_tune_saved.end() && kernel_serves(jt->second, bucket, fp32, sh, false));
+    return kept_kernel(a, sh, ds, bucket, fp32) < 0;
 }
 
 // Device time of one launch of kernel kid on a sample (a warm-up run, then a timed one).
@@ -749,12 +770,14 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
     // the launch plan: pinned, or the tuned choice for this configuration, or decided below
     const int cap_single = std::min(nmax, RBFX_MAX_N);
     const bool single_ok = rbfx::sym_fits(cap_single, sh.n_cols);
-    const TuneKey pkey{a->dim,        sh.n_cols, a->precision, kPlanKey, sh.kmax, sh.m, sh.basis_kind,
-                       sh.hermite ? 1 : 0, sh.uniform ? 1 : 0};
+    const bool kept_out = nse_kept_out(sh, kPlanKey);
+    const TuneKey pkey = tune_key(a, sh, kPlanKey, kept_out);
     int plan = g_force_plan;
     if (plan == 0) {
         auto it = ds.tuned.find(pkey);
         auto jt = g_tune_saved.find(pkey);
+        // (a plan timed here without the entry's flag was timed with the classes, or without)
+        if (jt == g_tune_saved.end() && kept_out) jt = g_tune_saved.find(tune_key(a, sh, kPlanKey, false));
         if (it != ds.tuned.end()) plan = it->second;
         else if (jt != g_tune_saved.end()) plan = jt->second;
     }
@@ -1379,7 +1402,8 @@ int rbfx_tune_plan(int32_t plan)
 }
 
 // Text format, one configuration per line:
-//   dim n_cols precision bucket kmax m basis_kind hermite uniform kernel
+//   dim n_cols precision bucket kmax m basis_kind hermite uniform kernel [1]
+// (1: builds that keep out kernel 8, which would serve their shape)
 int rbfx_tune_save(const char* path)
 {
     if (!path) return set_err(RBFX_EINVAL, "rbfx_tune_save: null path");
@@ -1392,12 +1416,13 @@ int rbfx_tune_save(const char* path)
     }
     FILE* f = std::fopen(path, "w");
     if (!f) return set_err(RBFX_EINVAL, "rbfx_tune_save: cannot open %s for writing", path);
-    std::fprintf(f, "# rbfx autotuner choices: dim n_cols precision bucket kmax m basis hermite uniform kernel\n");
+    std::fprintf(f, "# rbfx autotuner choices: dim n_cols precision bucket kmax m basis hermite uniform kernel "
+                    "[1: builds without kernel 8]\n");
     for (const auto& kv : all) {
         const TuneKey& k = kv.first;
-        std::fprintf(f, "%d %d %d %d %d %d %d %d %d %d\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
+        std::fprintf(f, "%d %d %d %d %d %d %d %d %d %d%s\n", std::get<0>(k), std::get<1>(k), std::get<2>(k),
                      std::get<3>(k), std::get<4>(k), std::get<5>(k), std::get<6>(k), std::get<7>(k), std::get<8>(k),
-                     kv.second);
+                     kv.second, std::get<9>(k) ? " 1" : "");
     }
     const bool ok = std::fclose(f) == 0;
     if (!ok) return set_err(RBFX_EDEVICE, "rbfx_tune_save: write to %s failed", path);
@@ -1425,15 +1450,16 @@ int rbfx_tune_load(const char* path)
     while (std::fgets(line, sizeof(line), f)) {
         ++lineno;
         if (line[0] == '#' || line[0] == '\n') continue;
-        int v[10];
-        if (std::sscanf(line, "%d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6], &v[7],
-                        &v[8], &v[9]) != 10 ||
+        int v[11];
+        v[10] = 0;
+        if (std::sscanf(line, "%d %d %d %d %d %d %d %d %d %d %d", &v[0], &v[1], &v[2], &v[3], &v[4], &v[5], &v[6],
+                        &v[7], &v[8], &v[9], &v[10]) < 10 ||
             v[3] < 0 || v[3] > kPlanKey || v[9] < 0 || v[9] >= kNumKernels ||
             (v[3] == kPlanKey && v[9] != kPlanBucketed && v[9] != kPlanSingle)) {
             std::fclose(f);
             return set_err(RBFX_EINVAL, "rbfx_tune_load: %s line %d is not a tuning entry", path, lineno);
         }
-        got[TuneKey{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8]}] = v[9];
+        got[TuneKey{v[0], v[1], v[2], v[3], v[4], v[5], v[6], v[7], v[8], v[10] == 1 ? 1 : 0}] = v[9];
     }
     std::fclose(f);
     std::lock_guard<std::mutex> lk(g_mu);
