@@ -571,10 +571,12 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
     if (kernel_serves(K_NSC, bucket, fp32, sh, false)) dflt = K_NSC;
     if (kernel_serves(K_NSC2, bucket, fp32, sh, false)) dflt = K_NSC2;  // (the faster mapping where it fits)
     // The elimination is faster than the other kernels on every shape it serves. Builds of
-    // several columns too small to be timed keep the weights, bit for bit, of the rook
-    // kernel that solves the same columns one build at a time.
-    if (kernel_serves(K_NSE, bucket, fp32, sh, false) && (sh.n_cols == 1 || bucket > 0 || count >= kTuneMin))
-        dflt = K_NSE;
+    // several columns and up to 32 rows that are too small to be timed stay on the rook kernel
+    // all the same, whatever a larger build of their shape has left in the map: their weights
+    // are compared with a rook build's to 1e-12 of the largest (the price: 900 points, 3
+    // columns, 26 rows 81 us against 20).
+    const bool small_rook = sh.n_cols > 1 && bucket == 0 && count < kTuneMin;
+    if (kernel_serves(K_NSE, bucket, fp32, sh, false) && !small_rook) dflt = K_NSE;
     *kid = dflt;
     const int forced = g_force_kernel[bucket];
     if (forced >= 0 && kernel_serves(forced, bucket, fp32, sh, true)) {
@@ -584,7 +586,7 @@ static int pick_kernel(const rbfx_build_args* a, const rbfx::BuildDev& Q, const 
     // a cached or loaded choice is used only where that kernel serves this build
     const TuneKey key = tune_key(a, sh, bucket, nse_kept_out(sh, bucket));
     const int kept = kept_kernel(a, sh, ds, bucket, fp32);
-    if (kept >= 0) {
+    if (kept >= 0 && !(small_rook && kept == K_NSE)) {
         *kid = kept;
         return RBFX_OK;
     }

@@ -107,3 +107,30 @@ def test_uneven_builds_with_and_without_multipliers(RBF, gpu, tmp_path):
                 assert st[2] == plans[m] and (st[3] > n // 2) == (not m and plans[m] == 1), (text, m, st)
     finally:
         RBF._lib.tune_reset()
+
+
+@pytest.mark.gpu
+def test_small_builds_of_several_columns_stay_on_the_rook_kernel(RBF, gpu):
+    """Up to 32 rows and fewer stencils than are timed: the same kernel and bits whether or not a
+    larger build of the shape has put kernel 8 into the map; a captured step too."""
+    import torch
+
+    pts = torch.as_tensor(np.random.default_rng(3).random((6000, 2)), device=gpu)
+    small = pts[:1500].contiguous()
+    RBF._lib.tune_reset()
+    try:
+        first = RBF.gradient(small, k=20)
+        assert RBF._lib.last_build_buckets()[1][0] == 0
+        RBF.gradient(pts, k=20)
+        assert RBF._lib.last_build_buckets()[1][0] == K_NSE
+        again = RBF.gradient(small, k=20)
+        assert RBF._lib.last_build_buckets()[1][0] == 0
+        assert torch.equal(first.vals, again.vals)
+        g = again.capture(torch.sin(small[:, 0]))
+        for _ in range(3):
+            again.vals.zero_()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(again.vals, first.vals)
+    finally:
+        RBF._lib.tune_reset()
