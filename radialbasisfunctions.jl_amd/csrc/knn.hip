@@ -447,9 +447,15 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
     // Within a run, four candidates per step as long as any lane has some; a merge when any
     // lane might run out of room, and at the end of the block and of each ring. (The loop
     // holds the only copy of the merge.)
+    // A wavefront most of whose lanes find eight times the mean in their first row, between an
+    // eighth and half of it in their own cell, stands in a wide cluster, where the two rings
+    // hold far more than the k nearest: it goes ring by ring from its own cells (300,000
+    // points, a cluster of up to 400 times the mean density, k = 20: 3.38 -> 2.61 ms in 2-D;
+    // where a single cell holds the row, the other order is the faster one: 11.2 against 14 ms).
     constexpr int R0 = 2, NROW = DIM == 1 ? 1 : (DIM == 2 ? 5 : 25), STEP = 4;
     int np = 0;  // pending candidates
     int rho = R0, j = 0, dy = 0, dz = 0, part = 0;
+    bool block = true;
     bool open = live;
     struct Run {
         int32_t s0, s1;
@@ -460,7 +466,7 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
         Run r;
         int cy, cz, xl = c0 - rho, xh = c0 + rho;
         bool in = open;
-        if (rho == R0) {
+        if (block) {
             cy = c1 + (DIM == 3 ? kRowY[j] : (DIM == 2 ? kRowY2[j] : 0));
             cz = c2 + (DIM == 3 ? kRowZ[j] : 0);
             r.last = ++j == NROW;
@@ -495,6 +501,15 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
         return r;
     };
     Run cur = next();
+    if (DIM >= 2 && __popcll(__ballot(cur.s1 - cur.s0 > 4 * kmax)) > 32) {
+        const int64_t own = row_id(c1, c2) + c0;
+        const int32_t n_own = cell_start[own + 1] - cell_start[own], n_row = cur.s1 - cur.s0;
+        if (__popcll(__ballot(n_row > 4 * kmax && 2 * n_own < n_row && n_row < 8 * n_own)) > 32) {
+            block = false;
+            rho = 0;
+            cur = next();
+        }
+    }
     for (;;) {
         Run nxt;
         if (!cur.last) nxt = next();
@@ -535,6 +550,7 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
         if (cur.last) {
             open = open && !settled(rho);
             if (!__ballot(open)) break;
+            block = false;
             ++rho;
             dy = DIM >= 2 ? -rho : 0;
             dz = DIM == 3 ? -rho : 0;
@@ -562,8 +578,8 @@ __global__ __launch_bounds__(64) void k_query(const double* __restrict__ sx, con
 // of cells are looked up by one lane each, their candidates taken 64 at a time, and a
 // batch with many that beat the k-th so far is sorted over the lanes (DPP moves) and merged
 // with the list; a batch with few is merged by rank: each is broadcast, and every lane
-// counts how many come before its own. The visiting order, the distances and the
-// stopping test are k_query's, so the result is the same.
+// counts how many come before its own. The distances, their order and the stopping test
+// are k_query's, so the result is the same.
 __device__ __forceinline__ int rdlane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
 __device__ __forceinline__ double rdlane(double v, int l)
 {
@@ -653,6 +669,11 @@ __device__ __forceinline__ int lane_sum(int v)
     return v;
 }
 
+// candidates of the block of two rings that are read at once (eight batches; a uniform cloud's
+// hold 50 to 330): 300,000 points, k = 40, most in a cluster of up to 400 times the mean density:
+// 2-D 12.2 ms with blocks of any size, 2.0 with this limit (6.9 before there were wavefront
+// searches); 3-D 107 and 8.5
+constexpr int kBlockMost = 512;
 // candidates that a batch merges by rank (14 instructions each) rather than by sorting (280)
 constexpr int kRankMerge = 12;
 
@@ -688,104 +709,119 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
     asm volatile("" : "+v"(bd));
     double kd = rdlane(bd, 0);
     int bi = 0x7fffffff, ki = bi, ki0 = bi;
-    for (int rho = 2;; ++rho) {
-        // The block of two rings as whole rows, then a ring's rows: whole on its faces, else
-        // the two end cells (one id each).
-        const int W = 2 * rho + 1, rows = DIM == 1 ? 1 : (DIM == 2 ? W : W * W);
-        const int n_ids = rho == 2 ? rows : 2 * rows;
-        for (int id0 = 0; id0 < n_ids; id0 += 64) {
-            const int id = id0 + lane, r = rho == 2 ? id : id >> 1, part = rho == 2 ? 0 : id & 1;
-            const int dy = DIM >= 2 ? r % W - rho : 0, dz = DIM == 3 ? r / W - rho : 0;
-            const int cy = c1 + dy, cz = c2 + dz;
-            const bool face = rho == 2 || (DIM >= 2 && (dy == -rho || dy == rho)) || (DIM == 3 && (dz == -rho || dz == rho));
-            int xl = c0 - rho, xh = c0 + rho;
-            bool in = id < n_ids && cy >= 0 && cy < G.n[1] && cz >= 0 && cz < G.n[2];
-            if (face) {
-                in = in && part == 0;
-            } else if (part == 0) {
-                in = in && xl >= 0;
-                xh = xl;
-            } else {
-                in = in && xh < G.n[0];
-                xl = xh;
+    auto side = [&](int d, int lo_cell, int hi_cell) __attribute__((always_inline)) {
+        const double at = q[d] - G.lo[d];
+        const double g = fmax(lo_cell * G.s - at, at - (hi_cell + 1) * G.s);
+        return g > 0.0 ? g * g : 0.0;
+    };
+    // The candidates of up to 64 runs of cells: rows of the block of two rings, or of ring rho
+    // (whole on its faces, else the two end cells, one id each; only those closer than the
+    // k-th so far). False, with nothing read, for a block of more than kBlockMost.
+    auto scan = [&](auto blk, const int rho, const int id0, const int n_ids) __attribute__((always_inline)) {
+        constexpr bool BLOCK = decltype(blk)::value;
+        const int W = 2 * rho + 1;
+        const int id = id0 + lane, r = BLOCK ? id : id >> 1, part = BLOCK ? 0 : id & 1;
+        const int dy = DIM >= 2 ? r % W - rho : 0, dz = DIM == 3 ? r / W - rho : 0;
+        const int cy = c1 + dy, cz = c2 + dz;
+        const bool face = BLOCK || rho == 0 || (DIM >= 2 && (dy == -rho || dy == rho)) ||
+                          (DIM == 3 && (dz == -rho || dz == rho));
+        int xl = c0 - rho, xh = c0 + rho;
+        bool in = id < n_ids && cy >= 0 && cy < G.n[1] && cz >= 0 && cz < G.n[2];
+        if (face) {
+            in = in && part == 0;
+        } else if (part == 0) {
+            in = in && xl >= 0;
+            xh = xl;
+        } else {
+            in = in && xh < G.n[0];
+            xl = xh;
+        }
+        if (!BLOCK && ki != 0x7fffffff) {
+            double g2 = side(0, xl, xh);
+            if constexpr (DIM >= 2) g2 += side(1, cy, cy);
+            if constexpr (DIM == 3) g2 += side(2, cz, cz);
+            in = in && g2 * (1.0 - 1e-9) < kd;
+        }
+        int32_t s0 = 0, cnt = 0;
+        if (in) {
+            const int64_t row = ((int64_t)cz * G.n[1] + cy) * G.n[0];
+            s0 = cell_start[row + max(xl, 0)];
+            cnt = cell_start[row + min(xh, G.n[0] - 1) + 1] - s0;
+        }
+        // candidate f of the batch lies in the first run whose inclusive count exceeds it
+        const int inc = lane_sum(cnt), n_run = min(n_ids - id0, 64);
+        const int total = rdlane(inc, 63);
+        if (BLOCK && total > kBlockMost) return false;
+        const int base = s0 - (inc - cnt);
+        for (int f0 = 0; f0 < total; f0 += 64) {
+            const int f = f0 + lane;
+            int run = 0;
+            for (int s = n_run > 32 ? 32 : (n_run > 16 ? 16 : (n_run > 4 ? 8 : 2)); s; s >>= 1) {
+                const int v = __shfl(inc, run + s - 1, 64);
+                run += v <= f ? s : 0;
             }
-            int32_t s0 = 0, cnt = 0;
-            if (in) {
-                const int64_t row = ((int64_t)cz * G.n[1] + cy) * G.n[0];
-                s0 = cell_start[row + max(xl, 0)];
-                cnt = cell_start[row + min(xh, G.n[0] - 1) + 1] - s0;
-            }
-            // candidate f of the batch lies in the first run whose inclusive count exceeds it
-            const int inc = lane_sum(cnt), n_run = min(n_ids - id0, 64);
-            const int total = rdlane(inc, 63);
-            const int base = s0 - (inc - cnt);
-            for (int f0 = 0; f0 < total; f0 += 64) {
-                const int f = f0 + lane;
-                int run = 0;
-                for (int s = n_run > 32 ? 32 : (n_run > 16 ? 16 : (n_run > 4 ? 8 : 2)); s; s >>= 1) {
-                    const int v = __shfl(inc, run + s - 1, 64);
-                    run += v <= f ? s : 0;
-                }
-                const int b = __shfl(base, run & 63, 64);
-                double cd = __builtin_huge_val();
-                int ci = 0x7fffffff;
-                if (f < total) {
-                    double x[DIM];
+            const int b = __shfl(base, run & 63, 64);
+            double cd = __builtin_huge_val();
+            int ci = 0x7fffffff;
+            if (f < total) {
+                double x[DIM];
 #pragma unroll
-                    for (int d = 0; d < DIM; ++d) x[d] = sx[(int64_t)(b + f) * DIM + d];
-                    cd = sqdist<DIM>(x, q);
-                    ci = sidx[b + f];
+                for (int d = 0; d < DIM; ++d) x[d] = sx[(int64_t)(b + f) * DIM + d];
+                cd = sqdist<DIM>(x, q);
+                ci = sidx[b + f];
+            }
+            const bool pass = f < total && lt(cd, ci, kd, ki);
+            const unsigned long long m = __ballot(pass);
+            if (!m) continue;
+            if (__popcll(m) > kRankMerge) {
+                cd = pass ? cd : __builtin_huge_val();
+                ci = pass ? ci : 0x7fffffff;
+                lane_sort(cd, ci, lane);
+                if (ki0 == 0x7fffffff) {  // nothing yet
+                    bd = cd;
+                    bi = ci;
+                } else {
+                    lane_merge(bd, bi, cd, ci, lane);
                 }
-                const bool pass = f < total && lt(cd, ci, kd, ki);
-                const unsigned long long m = __ballot(pass);
-                if (!m) continue;
-                if (__popcll(m) > kRankMerge) {
-                    cd = pass ? cd : __builtin_huge_val();
-                    ci = pass ? ci : 0x7fffffff;
-                    lane_sort(cd, ci, lane);
-                    if (ki0 == 0x7fffffff) {  // nothing yet
-                        bd = cd;
-                        bi = ci;
-                    } else {
-                        lane_merge(bd, bi, cd, ci, lane);
-                    }
-                    kd = rdlane(bd, kmax - 1);
-                    ki = rdlane(bi, kmax - 1);
-                    ki0 = rdlane(bi, 0);
-                    continue;
-                }
-                int rb = lane, rn = 0;
-                for (unsigned long long left = m; left; left &= left - 1) {
-                    const int l = __builtin_ctzll(left);
-                    const double nd = rdlane(cd, l);
-                    const int ni = rdlane(ci, l);
-                    const bool before = lt(nd, ni, bd, bi);
-                    rb += before ? 1 : 0;
-                    rn += lt(nd, ni, cd, ci) ? 1 : 0;
-                    const int ahead = 64 - __popcll(__ballot(before));
-                    rn += lane == l ? ahead : 0;
-                }
-                if (rb < 64) {
-                    s_d[w][rb] = bd;
-                    s_i[w][rb] = bi;
-                }
-                if (pass && rn < 64) {
-                    s_d[w][rn] = cd;
-                    s_i[w][rn] = ci;
-                }
-                // (a wavefront's LDS accesses complete in order)
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_wave_barrier();
-                bd = s_d[w][lane];
-                bi = s_i[w][lane];
-                asm volatile("" ::: "memory");
-                __builtin_amdgcn_wave_barrier();
                 kd = rdlane(bd, kmax - 1);
                 ki = rdlane(bi, kmax - 1);
                 ki0 = rdlane(bi, 0);
+                continue;
             }
+            int rb = lane, rn = 0;
+            for (unsigned long long left = m; left; left &= left - 1) {
+                const int l = __builtin_ctzll(left);
+                const double nd = rdlane(cd, l);
+                const int ni = rdlane(ci, l);
+                const bool before = lt(nd, ni, bd, bi);
+                rb += before ? 1 : 0;
+                rn += lt(nd, ni, cd, ci) ? 1 : 0;
+                const int ahead = 64 - __popcll(__ballot(before));
+                rn += lane == l ? ahead : 0;
+            }
+            if (rb < 64) {
+                s_d[w][rb] = bd;
+                s_i[w][rb] = bi;
+            }
+            if (pass && rn < 64) {
+                s_d[w][rn] = cd;
+                s_i[w][rn] = ci;
+            }
+            // (a wavefront's LDS accesses complete in order)
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            bd = s_d[w][lane];
+            bi = s_i[w][lane];
+            asm volatile("" ::: "memory");
+            __builtin_amdgcn_wave_barrier();
+            kd = rdlane(bd, kmax - 1);
+            ki = rdlane(bi, kmax - 1);
+            ki0 = rdlane(bi, 0);
         }
-        // (k_query's stopping test)
+        return true;
+    };
+    // (k_query's stopping test)
+    auto settled = [&](const int rho) {
         double bound = 1e300;
         bool covers_all = true;
         auto side_bound = [&](int d, int cd) __attribute__((always_inline)) {
@@ -797,9 +833,17 @@ __global__ __launch_bounds__(256) void k_query_wave(const double* __restrict__ s
         side_bound(0, c0);
         if constexpr (DIM >= 2) side_bound(1, c1);
         if constexpr (DIM == 3) side_bound(2, c2);
-        if (covers_all || rho > maxn) break;
-        if (ki != 0x7fffffff && bound > 0.0 && kd < bound * bound * (1.0 - 1e-9)) break;
-    }
+        return covers_all || rho > maxn || (ki != 0x7fffffff && bound > 0.0 && kd < bound * bound * (1.0 - 1e-9));
+    };
+    // The block of two rings, then ring by ring; in a cluster, where the block holds far more
+    // than the k nearest, ring by ring from the query's own cell.
+    const bool whole = scan(std::true_type{}, 2, 0, DIM == 1 ? 1 : (DIM == 2 ? 5 : 25));
+    if (!whole || !settled(2))
+        for (int rho = whole ? 3 : 0;; ++rho) {
+            const int W = 2 * rho + 1, n_ids = rho == 0 ? 1 : 2 * (DIM == 1 ? 1 : (DIM == 2 ? W : W * W));
+            for (int id0 = 0; id0 < n_ids; id0 += 64) scan(std::false_type{}, rho, id0, n_ids);
+            if (settled(rho)) break;
+        }
     const int64_t base = q_ptr ? q_ptr[qi] : qi * (int64_t)kmax;
     const int kq = q_ptr ? (int)(q_ptr[qi + 1] - q_ptr[qi]) : kmax;
     if (lane < kq && lane < kmax) out[base + lane] = bi;

@@ -74,3 +74,24 @@ def test_operator_with_and_without_order_agree(RBF, gpu):
     op._row_order, op.SPATIAL_ORDER_MIN = None, 10 ** 12
     op.update_weights()
     assert torch.equal(op.vals, w)
+
+
+@pytest.mark.parametrize("dim,k", [(1, 9), (2, 12), (2, 40), (3, 20), (3, 33)])
+def test_knn_inside_dense_clusters(RBF, O, gpu, dim, k):
+    """Clusters of a hundred to ten thousand times the mean density, where the block of two rings
+    holds thousands of points and both searches go ring by ring from the query's own cell:
+    against brute force, in the clusters, at their rims and between them."""
+    import torch
+
+    rng = np.random.default_rng(10 * dim + k)
+    x = np.concatenate([0.5 + 0.02 * rng.standard_normal((9000, dim)), 0.2 + 2e-4 * rng.standard_normal((6000, dim)),
+                        rng.random((1000, dim))])
+    x = x[rng.permutation(len(x))]
+    some = np.concatenate([x[:1500], 0.5 + 0.06 * rng.standard_normal((500, dim)), 0.2 + 6e-4 * rng.standard_normal((500, dim))])
+    want = O.knn(x, some, k)
+    assert np.array_equal(RBF.find_neighbors(x, some, k=k), want)
+    if k <= 32:  # the same queries among enough others that a lane takes each
+        n = 263_000 if dim == 3 else 66_000
+        q = torch.as_tensor(np.concatenate([some, x[rng.integers(0, len(x), n)]]), device=gpu)
+        got = RBF._lib.knn(torch.as_tensor(x, device=gpu), q, k)
+        assert np.array_equal(got[:len(some)].cpu().numpy(), want)
