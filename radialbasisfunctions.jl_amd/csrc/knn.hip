@@ -987,7 +987,12 @@ static hipError_t knn_dim(KnnWorkspace& ws, const double* data, int64_t n_data, 
     hipError_t err;
     if ((err = ws.reserve_points(n_data, n_query, DIM, self, st)) != hipSuccess) return err;
     Grid G;
-    if (n_data <= kSmallPoints && !out_order) {
+    // One workgroup's binning leaves queries that are not the points in their own order. With a
+    // lane per query that costs coherence, in 3-D more than binning them costs: 4,000 points,
+    // k = 20: 1M queries 1.37 ms against 0.88 binned, 4M 4.94 and 2.93 (900 points: 1.47 and
+    // 1.12; 300: 1.67 and 1.48, but k = 16 1.12 and 1.20; 2-D, 4,000: 0.59 and 0.61).
+    const bool binned_queries = DIM == 3 && !self && n_data > 512 && !query_by_wavefront(DIM, k, n_query);
+    if (n_data <= kSmallPoints && !out_order && !binned_queries) {
         if ((err = ws.reserve_cells(kSmallCells, true)) != hipSuccess) return err;
         hipLaunchKernelGGL(k_bin_small<DIM>, dim3(1), dim3(kSmallThreads), 0, st, data, (int)n_data, target, (Grid*)ws.grid,
                            ws.start, ws.sidx, ws.sx);

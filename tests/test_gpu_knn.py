@@ -95,3 +95,18 @@ def test_knn_inside_dense_clusters(RBF, O, gpu, dim, k):
         q = torch.as_tensor(np.concatenate([some, x[rng.integers(0, len(x), n)]]), device=gpu)
         got = RBF._lib.knn(torch.as_tensor(x, device=gpu), q, k)
         assert np.array_equal(got[:len(some)].cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("dim,n", [(2, 4000), (3, 512), (3, 513), (3, 4000)])
+def test_knn_many_queries_of_a_small_cloud(RBF, O, gpu, dim, n):
+    """More queries than wavefronts take, not the points themselves, of clouds small enough for
+    one workgroup's binning: in 3-D beyond 512 points the queries are binned too."""
+    import torch
+
+    rng = np.random.default_rng(n)
+    x, some = rng.random((n, dim)), rng.random((1000, dim)) * 1.4 - 0.2
+    q = torch.as_tensor(np.concatenate([some, rng.random((265_000, dim))]), device=gpu)
+    got = RBF._lib.knn(torch.as_tensor(x, device=gpu), q, 20)
+    assert np.array_equal(got[:1000].cpu().numpy(), O.knn(x, some, 20))
+    part = RBF._lib.knn(torch.as_tensor(x, device=gpu), q[-50_000:].contiguous(), 20)  # (a wavefront each)
+    assert torch.equal(got[-50_000:], part)
