@@ -455,9 +455,12 @@ class RadialBasisOperator:
     scipy.sparse matrices (a tuple for rank >= 1)."""
 
     SPATIAL_ORDER_MIN = 65536  # below this the X vector sits in L2 anyway
-    # up to here the processing order is the neighbour search's curve over its cells, which
-    # costs 20 us and serves builds and applies as well as a Morton sort (150 us) while X fits
-    # one XCD's L2 (4 MB); beyond, the sort's finer order (1M points, 2-D: apply 62 against 68 us)
+    # up to this many evaluation points the processing order is the neighbour search's curve
+    # over its cells, which costs 20 us and more with the cells, a Morton sort 150 to 400;
+    # beyond, the sort's finer order pays for itself (1M points, 2-D: apply 62 against 68 us).
+    # The data may be more: 3-D regrid to 400,000 points, construction with the curve and with
+    # the sort, and an apply with either: from 600,000 points 3.3 and 3.7 ms, 50 and 49 us, from
+    # 8M 4.9 and 5.2 ms, 127 and 127 us; to 70,000 points from 8M 2.13 and 2.08 ms
     CELL_ORDER_MAX = 524288
     SPMV_MAPPING = 0  # rbfx_spmv_args.mapping: 0 automatic, 1 lanes per row, 2 staged through LDS, 3 vector loads,
     # 4 source tiles
