@@ -852,20 +852,28 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
     if (rc == RBFX_OK) rc = read_counts();
     if (rc != RBFX_OK) return rc;
     // The first time a configuration is seen, its buckets' kernels are timed on samples of
-    // all their stencils (also those of a class), and the plan is decided when every
-    // nonempty bucket was just timed: the single launch's kernel on each bucket's sample
-    // against the bucket's own pick, weighted by the stencils that kernel would get, and the
-    // classes' launches.
+    // what the classes leave them, or of all their stencils where that is too little, and the
+    // plan is decided when every nonempty bucket was just timed: the single launch's kernel on
+    // each bucket's sample against the bucket's own pick, weighted by the stencils that
+    // kernel would get, and the classes' launches.
     bool timing = false;
     if (!async)
         for (int b = 0; b < 3; ++b) timing = timing || would_time(a, sh, ds, b, fp32, cnt[kTotals + b]);
     int kid[3];
     if (timing) {
         int32_t rest[3] = {cnt[0], cnt[1], cnt[2]};
-        float class_ms = 0.f;
+        float class_ms = 0.f, per_stencil[3] = {-1.f, -1.f, -1.f};
+        bool picked[3] = {false, false, false};
         ClassTab none;
         none.n = 0;
         if (tab.n > 0) {
+            for (int b = 0; b < 3; ++b) {
+                if (rest[b] < kTuneMin) continue;
+                rc = pick_kernel(a, bucket_of(b), sh, ds, hb, b, fp32, rows_cap[b], rest[b],
+                                 ds.bucket_count + kSamples + b, mode, st, &kid[b], &per_stencil[b]);
+                if (rc != RBFX_OK) return rc;
+                picked[b] = true;
+            }
             for (int i = 0; i < 2; ++i)
                 if (!ds.tev[i]) HIPCHK(hipEventCreate(&ds.tev[i]));
             HIPCHK(hipEventRecord(ds.tev[0], st));
@@ -876,12 +884,13 @@ static int solve_all(const rbfx_build_args* a, const rbfx::BuildDev& P, const Sh
             if ((rc = classify(none)) != RBFX_OK) return rc;
             if ((rc = read_counts()) != RBFX_OK) return rc;
         }
-        float per_stencil[3];
         bool all_timed = true;
         for (int b = 0; b < 3; ++b) {
-            rc = pick_kernel(a, bucket_of(b), sh, ds, hb, b, fp32, rows_cap[b], cnt[b],
-                             ds.bucket_count + kSamples + b, mode, st, &kid[b], &per_stencil[b]);
-            if (rc != RBFX_OK) return rc;
+            if (!picked[b]) {
+                rc = pick_kernel(a, bucket_of(b), sh, ds, hb, b, fp32, rows_cap[b], cnt[b],
+                                 ds.bucket_count + kSamples + b, mode, st, &kid[b], &per_stencil[b]);
+                if (rc != RBFX_OK) return rc;
+            }
             if (cnt[b] > 0 && per_stencil[b] < 0.f) all_timed = false;
         }
         if (plan == 0 && single_ok && all_timed) {
