@@ -16,10 +16,11 @@ hipError_t launch_nse_3d_phs7(const BuildDev& P, int64_t n_work, hipStream_t s);
 hipError_t launch_nse_rag_2d(const BuildDev& P, int m, int hi, int64_t n_work, hipStream_t s);
 hipError_t launch_nse_rag_3d(const BuildDev& P, int m, int hi, int64_t n_work, hipStream_t s);
 
-// The null points (k - m) and the operator columns share the lanes of one or two slots
-// of 16, so at most 26 null points; the monomial tables of degree 1 to 4 (2-D) and 1 to 3
-// (3-D) that the basis is definite with. Other shapes (1-D, other bases, wider
-// stencils, more columns) stay with the other kernels.
+// Shapes of uniform builds. The null points (k - m) and the operator columns share the lanes of
+// one or two slots of 16: at most 26 null points with the most columns, and none beyond that
+// here (the classes of uneven builds below go to 32 less the columns in 2-D). The monomial
+// tables of degree 1 to 4 (2-D) and 1 to 3 (3-D) that the basis is definite with. Other
+// shapes (1-D, other bases, wider stencils, more columns) stay with the other kernels.
 bool nse_fits(int kind, int dim, int k, int m, int n_cols)
 {
     const int nn = k - m;

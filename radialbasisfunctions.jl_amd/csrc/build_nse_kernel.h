@@ -22,15 +22,17 @@
 // (v_fmac_f64 with row_newbcast), which runs at the FMA's own rate (5.1 against 4.7
 // cycles measured, four waves per SIMD): no LDS read and no move per broadcast operand.
 // S is eliminated by Gauss-Jordan steps, so no triangular solve follows and the columns of
-// the right-hand sides are updated by the same instructions. LDS carries only the pivot
-// rows of the LU and the two changes of layout.
+// the right-hand sides are updated by the same instructions. Last, w_B is corrected once by the
+// residual of the polynomial conditions (Gauss-Jordan on P_B^T, in the lanes as well). LDS
+// carries the pivot rows of the LU, the two changes of layout, and what the correction reads
+// again.
 //
 // Bound by FP64 VALU issue; VGPRs (the instantiation's W waves per SIMD) and LDS
 // (NseLds) set how many wavefronts hide the LU's serial chain of pivots. Measured against
 // the kernels that served these builds before: 4M-point 2-D Laplacian (PHS3, degree 2,
-// k = 20) 12.06 -> 3.09 ms per build (null-space Cholesky, 8 lanes of three rows; 386
+// k = 20) 12.03 -> 3.51 ms per build (null-space Cholesky, 8 lanes of three rows; 448
 // VALU instructions per stencil against 897), 2M-point 3-D gradient and Laplacian (PHS5,
-// degree 3, k = 40) 149.6 -> 11.8 ms (rook LDL^T in LDS; 2,320 against 21,800).
+// degree 3, k = 40) 149.1 -> 13.9 ms (rook LDL^T in LDS; 2,850 against 21,800).
 //
 // Breakdown: an LU pivot below kNseLuTol (scaled coordinates, monomials of order one), or
 // a pivot of S below kNsePivTol of the stencil's scale, hands the stencil to the rook-pivoted
